@@ -20,6 +20,7 @@
 #include <vector>
 
 #include "../../include/doug.h"
+#include "doug_front_kernels.hpp"
 #include "doug_kernels.hpp"
 #include "doug_setup.hpp"
 
@@ -55,6 +56,12 @@ struct StreamOverride {
 
 }  // namespace
 
+// The subdomains' unknowns on the device, each subdomain in its factor's
+// order, and each node's positions in them (ascending): [ptr[i], ptr[i + 1]).
+struct LocalLists {
+  int32_t *inds = nullptr, *occ_ptr = nullptr, *occ_pos = nullptr;
+};
+
 struct doug_ctx {
   int device = 0;
   StreamRef stream;  // the main stream (or this thread's override)
@@ -65,6 +72,7 @@ struct doug_ctx {
   std::vector<hipEvent_t> cevents;  // coarse factorisation step ends, then the inverse's end
   // temporaries of the device coarse build, kept between set-ups
   std::vector<std::pair<void*, size_t>> scratch_slots;
+  std::pair<void*, size_t> front_scratch{nullptr, 0};  // update matrices of the frontal factorisation
   std::thread reaper;  // frees the buffers of the previous set-up
   std::string err;
   Params p;
@@ -143,11 +151,24 @@ struct doug_ctx {
   int trsm_cg = 1;                  // column layout of that solve (1..3, DOUG_OPT_BATCH_COLUMN_GROUPS)
   int local_order = 1;              // 1: reverse Cuthill-McKee inside each subdomain
   BlockDesc* d_sub_trsv = nullptr;  // descriptors in dispatch order
+  // frontal factors (nested dissection), the form used unless the caller asks
+  // for the index-set order or a subdomain exceeds the format
+  bool fronts = false;
+  FrontSub *d_fsub = nullptr, *d_fsub_solve = nullptr;  // as partitioned; in dispatch order
+  std::vector<FrontSub> h_fsub;
+  int maxwork = 0;  // largest work vector of a subdomain
+  int64_t factor_elems = 0;
+  // the batched solve's envelope factors and lists (the ones above where the
+  // single-vector solve uses envelopes too)
+  LocalLists batch_lists;
+  double* d_btiles = nullptr;
+  float* d_btiles32 = nullptr;
+  int front_nw = 8;  // wavefronts per subdomain in the single-vector solve
   doug_tuning tuning{};
   double* d_tiles = nullptr;   // FP64 factors
   float* d_tiles32 = nullptr;  // FP32 factors (DOUG_PREC_FP32_FACTORS)
   int precision = DOUG_PREC_FP64;
-  int32_t *d_inds = nullptr, *d_occ_ptr = nullptr, *d_occ_pos = nullptr;
+  LocalLists lists;
   double* d_subsol = nullptr;
   // fine_method 2: symmetric Gauss-Seidel on each subdomain's matrix
   SgsDesc* d_sgs = nullptr;
@@ -272,16 +293,18 @@ static void join_reaper(doug_ctx* ctx) {
   if (ctx->reaper.joinable()) ctx->reaper.join();
 }
 
-// The coarse build's device temporaries (kept between set-ups unless
+// The set-up's device temporaries (kept between set-ups unless
 // DOUG_OPT_KEEP_SETUP_TEMPS is 0).
 static void free_scratch_slots(doug_ctx* ctx) {
   for (auto& q : ctx->scratch_slots)
     if (q.first) (void)hipFree(q.first);
   ctx->scratch_slots.clear();
+  if (ctx->front_scratch.first) (void)hipFree(ctx->front_scratch.first);
+  ctx->front_scratch = {nullptr, 0};
 }
 
 static int64_t scratch_slot_bytes(const doug_ctx* ctx) {
-  int64_t b = 0;
+  int64_t b = (int64_t)ctx->front_scratch.second;
   for (const auto& q : ctx->scratch_slots) b += (int64_t)q.second;
   return b;
 }
@@ -894,10 +917,11 @@ static bool has_duplicate_entries(const Csr& A) {
 
 // build_blocks for the subdomain factors (envelope storage, one-block solve
 // limit) with the envelope and the entries taken on the device from the
-// uploaded matrix, unknown lists (ctx->d_inds) and occurrence lists, so the
-// host builds no scatter map.  A must have no duplicate (i, j) pair.
+// uploaded matrix, unknown lists and occurrence lists, so the host builds no
+// scatter map.  A must have no duplicate (i, j) pair.
 template <typename T>
-static int build_blocks_device(doug_ctx* ctx, const std::vector<int>& starts, std::vector<BlockDesc>& desc,
+static int build_blocks_device(doug_ctx* ctx, const std::vector<int>& starts, const LocalLists& lists,
+                               std::vector<BlockDesc>& desc,
                                BlockDesc** d_desc, T** d_tiles, int64_t* total_elems,
                                std::vector<int>& offcount, double* chol_flops) {
   const int nb = (int)starts.size() - 1;
@@ -921,7 +945,7 @@ static int build_blocks_device(doug_ctx* ctx, const std::vector<int>& starts, st
   int32_t *d_st, *d_r0, *d_fc;
   if ((rc = upload(ctx, &d_st, st32)) || (rc = upload(ctx, &d_r0, row0)) || (rc = upload(ctx, &d_fc, fc)))
     return rc;
-  launch_block_envelope(d_st, d_r0, nb, ctx->d_inds, ctx->d_occ_ptr, ctx->d_occ_pos, ctx->d_ptr,
+  launch_block_envelope(d_st, d_r0, nb, lists.inds, lists.occ_ptr, lists.occ_pos, ctx->d_ptr,
                         ctx->d_col, d_fc, ctx->stream);
   HIPCHK(hipGetLastError());
   HIPCHK(hipMemcpyAsync(fc.data(), d_fc, fc.size() * sizeof(int32_t), hipMemcpyDeviceToHost, ctx->stream));
@@ -971,7 +995,7 @@ static int build_blocks_device(doug_ctx* ctx, const std::vector<int>& starts, st
   int maxpad = 0;
   for (auto& d : desc) maxpad = std::max(maxpad, d.nt * kTile - d.s);
   launch_pad_identity(*d_tiles, *d_desc, nb, maxpad, ctx->stream);
-  launch_scatter_blocks(*d_tiles, *d_desc, nb, ctx->d_inds, ctx->d_occ_ptr, ctx->d_occ_pos, ctx->d_ptr,
+  launch_scatter_blocks(*d_tiles, *d_desc, nb, lists.inds, lists.occ_ptr, lists.occ_pos, ctx->d_ptr,
                         ctx->d_col, ctx->d_val, ctx->stream);
   // the host tables above must stay alive until the stream consumed them
   HIPCHK(hipStreamSynchronize(ctx->stream));
@@ -990,6 +1014,182 @@ static int enqueue_factor(doug_ctx* ctx, T* tiles, const BlockDesc* d_desc,
     launch_chol_offdiag(tiles, d_desc, (int)desc.size(), j, offcount[j], ctx->stream);
   }
   HIPCHK(hipGetLastError());
+  return DOUG_OK;
+}
+
+// Frontal factors of the subdomains, enqueued: the patterns' arrays (shared
+// by subdomains of one structure) on the device, the matrix entries in the
+// zeroed panels and the factorisation height by height.  With `host_map` the
+// entries come through a host-built map that sums repeated (i, j) pairs in
+// stored order.
+template <typename T>
+static int build_fronts(doug_ctx* ctx, const Csr& M, const std::vector<int>& starts, const std::vector<int>& dinds,
+                        const std::vector<FrontPattern>& pats, const std::vector<int>& pat, bool host_map,
+                        T** d_tiles, int64_t* total_elems, double* chol_flops, hipEvent_t ev0, int* flag) {
+  const int nb = (int)starts.size() - 1;
+  hipStream_t st = ctx->stream;
+  int rc;
+  // every pattern's arrays in one allocation each
+  struct Off {
+    size_t fr, rec, col, hp, hl, uf, ub, lf, lb;
+  };
+  std::vector<Off> off;
+  std::vector<Front> fr;
+  std::vector<uint16_t> rpos, col, hl;
+  std::vector<uint32_t> src;
+  std::vector<FrontUnit> uf, ub;
+  std::vector<int32_t> hp, lf, lb;
+  std::vector<double> flops;
+  for (const FrontPattern& P : pats) {
+    off.push_back(Off{fr.size(), rpos.size(), col.size(), hp.size(), hl.size(), uf.size(), ub.size(), lf.size(),
+                      lb.size()});
+    fr.insert(fr.end(), P.fronts.begin(), P.fronts.end());
+    rpos.insert(rpos.end(), P.rpos.begin(), P.rpos.end());
+    src.insert(src.end(), P.src.begin(), P.src.end());
+    col.insert(col.end(), P.colfront.begin(), P.colfront.end());
+    hp.insert(hp.end(), P.hptr.begin(), P.hptr.end());
+    hl.insert(hl.end(), P.hlist.begin(), P.hlist.end());
+    uf.insert(uf.end(), P.units_f.begin(), P.units_f.end());
+    ub.insert(ub.end(), P.units_b.begin(), P.units_b.end());
+    lf.insert(lf.end(), P.list_f.begin(), P.list_f.end());
+    lb.insert(lb.end(), P.list_b.begin(), P.list_b.end());
+    double f = 0.0;
+    for (const Front& q : P.fronts)
+      f += (double)q.k * q.k * q.k * 2.0 / 3.0 + 4.0 * q.k * q.k * q.m + 1.0 * q.k * q.m * q.m;
+    flops.push_back(f);
+  }
+  Front* d_fr;
+  uint16_t *d_rpos, *d_col, *d_hl;
+  uint32_t* d_src;
+  FrontUnit *d_uf, *d_ub;
+  int32_t *d_hp, *d_lf, *d_lb;
+  if ((rc = upload(ctx, &d_fr, fr)) || (rc = upload(ctx, &d_rpos, rpos)) || (rc = upload(ctx, &d_src, src)) ||
+      (rc = upload(ctx, &d_col, col)) || (rc = upload(ctx, &d_hp, hp)) || (rc = upload(ctx, &d_hl, hl)) ||
+      (rc = upload(ctx, &d_uf, uf)) || (rc = upload(ctx, &d_ub, ub)) || (rc = upload(ctx, &d_lf, lf)) ||
+      (rc = upload(ctx, &d_lb, lb)))
+    return rc;
+  std::vector<FrontSub>& subs = ctx->h_fsub;
+  subs.assign((size_t)nb, FrontSub{});
+  int64_t base = 0, sch = 0;
+  int heights = 0;
+  std::vector<int> maxcount;
+  std::vector<char> wide;
+  double f = 0.0;
+  ctx->maxwork = 0;
+  for (int b = 0; b < nb; b++) {
+    const FrontPattern& P = pats[pat[b]];
+    const Off& o = off[pat[b]];
+    const int nh = (int)P.hptr.size() - 1;
+    subs[b] = FrontSub{base, (int64_t)starts[b], sch, d_fr + o.fr, d_rpos + o.rec, d_src + o.rec,
+                       d_col + o.col, d_hp + o.hp, d_hl + o.hl, d_uf + o.uf, d_ub + o.ub, d_lf + o.lf,
+                       d_lb + o.lb, P.n, P.top0, P.work(), nh};
+    base += P.elems;
+    sch += (P.schur + 15) / 16 * 16;
+    f += flops[pat[b]];
+    heights = std::max(heights, nh);
+    maxcount.resize((size_t)heights, 0);
+    wide.resize((size_t)heights, 0);
+    for (int h = 0; h < nh; h++) {
+      maxcount[h] = std::max(maxcount[h], P.hptr[h + 1] - P.hptr[h]);
+      for (int i = P.hptr[h]; i < P.hptr[h + 1]; i++) wide[h] |= P.fronts[P.hlist[i]].k > 32;
+    }
+    ctx->maxwork = std::max(ctx->maxwork, P.work());
+  }
+  *total_elems = base;
+  if (chol_flops) *chol_flops = f;
+  if ((rc = upload(ctx, &ctx->d_fsub, subs))) return rc;
+  if ((rc = dalloc(ctx, d_tiles, (size_t)base))) return rc;
+  const size_t sch_bytes = (size_t)std::max<int64_t>(sch, 1) * sizeof(T);
+  if (ctx->front_scratch.second < sch_bytes) {
+    if (ctx->front_scratch.first) (void)hipFree(ctx->front_scratch.first);
+    ctx->front_scratch = {nullptr, 0};
+    void* q = nullptr;
+    const hipError_t e = device_malloc(ctx, &q, sch_bytes);
+    if (e != hipSuccess) {
+      (void)hipGetLastError();
+      return fail(ctx, DOUG_E_NOMEM, "hipMalloc of " + std::to_string(sch_bytes) + " bytes failed: " +
+                                         hipGetErrorString(e));
+    }
+    ctx->front_scratch = {q, sch_bytes};
+  }
+  T* d_schur = (T*)ctx->front_scratch.first;
+  HIPCHK(hipMemsetAsync(*d_tiles, 0, (size_t)base * sizeof(T), st));
+  if (!host_map) {
+    launch_front_scatter(*d_tiles, ctx->d_fsub, nb, ctx->lists.inds, ctx->lists.occ_ptr, ctx->lists.occ_pos, ctx->d_ptr,
+                         ctx->d_col, ctx->d_val, st);
+    HIPCHK(hipStreamSynchronize(st));  // the host arrays above go out of scope
+  } else {
+    // (element, entry) pairs block by block; a repeated element's entries
+    // become a group that the summing pass adds in stored order
+    std::vector<int64_t> dst, gdst, gseg(1, 0);
+    std::vector<int32_t> ent, gsrc;
+    std::vector<int> floc((size_t)M.nrows, -1);
+    std::vector<std::pair<int64_t, int32_t>> row;
+    for (int b = 0; b < nb; b++) {
+      const int s0 = starts[b], s = starts[b + 1] - s0;
+      for (int p = 0; p < s; p++) floc[dinds[s0 + p]] = p;
+      for (int p = 0; p < s; p++) {
+        const int g = dinds[s0 + p];
+        row.clear();
+        for (int e = M.ptr[g]; e < M.ptr[g + 1]; e++) {
+          const int q = floc[M.col[e]];
+          if (q >= 0 && q <= p)
+            row.push_back({subs[b].base + front_entry(pats[pat[b]], q, p, sizeof(T) == 8), (int32_t)e});
+        }
+        std::sort(row.begin(), row.end());
+        for (size_t i = 0, j; i < row.size(); i = j) {
+          for (j = i + 1; j < row.size() && row[j].first == row[i].first;) j++;
+          dst.push_back(row[i].first);
+          ent.push_back(row[i].second);
+          if (j - i > 1) {
+            gdst.push_back(row[i].first);
+            for (size_t q = i; q < j; q++) gsrc.push_back(row[q].second);
+            gseg.push_back((int64_t)gsrc.size());
+          }
+        }
+      }
+      for (int p = 0; p < s; p++) floc[dinds[s0 + p]] = -1;
+    }
+    int64_t* d_dst;
+    int32_t* d_ent;
+    if ((rc = upload(ctx, &d_dst, dst)) || (rc = upload(ctx, &d_ent, ent))) return rc;
+    launch_scatter_entries(*d_tiles, d_dst, d_ent, ctx->d_val, (int64_t)dst.size(), st);
+    if (!gdst.empty()) {
+      int64_t *d_gdst, *d_gseg;
+      int32_t* d_gsrc;
+      if ((rc = upload(ctx, &d_gdst, gdst)) || (rc = upload(ctx, &d_gseg, gseg)) || (rc = upload(ctx, &d_gsrc, gsrc)))
+        return rc;
+      launch_scatter_sums(*d_tiles, d_gdst, d_gseg, d_gsrc, ctx->d_val, (int64_t)gdst.size(), st);
+    }
+    HIPCHK(hipStreamSynchronize(st));  // the host arrays go out of scope
+  }
+  HIPCHK(hipEventRecord(ev0, st));
+  for (int h = 0; h < heights; h++)
+    launch_front_factor(*d_tiles, d_schur, ctx->d_fsub, nb, h, maxcount[h], wide[h] != 0, flag, st);
+  HIPCHK(hipGetLastError());
+  return DOUG_OK;
+}
+
+// Envelope factors of the subdomains, enqueued; `ev` (optional) is recorded
+// where their factorisation begins.
+template <typename T>
+static int envelope_factors(doug_ctx* ctx, const std::vector<int>& dinds, const LocalLists& L, bool host_map, T** tiles,
+                            int64_t* elems, double* flops, hipEvent_t ev, int* flag) {
+  std::vector<int> offcount;
+  int rc = host_map ? build_blocks(ctx, ctx->A, ctx->d_val, ctx->sstarts, dinds, true, true, ctx->h_sub, &ctx->d_sub,
+                                   tiles, elems, offcount, flops)
+                    : build_blocks_device(ctx, ctx->sstarts, L, ctx->h_sub, &ctx->d_sub, tiles, elems, offcount,
+                                          flops);
+  if (rc) return rc;
+  if (ev) HIPCHK(hipEventRecord(ev, ctx->stream));
+  if ((rc = enqueue_factor(ctx, *tiles, ctx->d_sub, ctx->h_sub, offcount, flag))) return rc;
+  ctx->maxnt = 0;
+  ctx->work_rows = 0;
+  for (auto& d : ctx->h_sub) {
+    ctx->maxnt = std::max(ctx->maxnt, d.nt);
+    ctx->work_rows += (int64_t)d.nt * kTile;
+  }
+  prepare_trsv<T>(ctx->maxnt);
   return DOUG_OK;
 }
 
@@ -1012,7 +1212,7 @@ static void phase_values(doug_ctx* ctx, std::vector<double>& scaled, std::vector
 }
 
 // virtual_ranks for the context's decomposition and aggregation parameters
-static void run_virtual_ranks(doug_ctx* ctx, RankSetup& out, const Csr* rcm, bool keep_local) {
+static void run_virtual_ranks(doug_ctx* ctx, RankSetup& out, bool keep_local) {
   const Params& p = ctx->p;
   const double strong_conn1 = p.strong1 != 0.0 ? p.strong1 : 0.67;
   const int radius1 = p.radius1 > 0 ? p.radius1 : 2;
@@ -1020,12 +1220,12 @@ static void run_virtual_ranks(doug_ctx* ctx, RankSetup& out, const Csr* rcm, boo
   const int max_asize1 = p.maxasize1 > 0 ? p.maxasize1 : (2 * radius1 + 1) * (2 * radius1 + 1);
   if (rows_sorted_by_column(ctx->A)) {
     virtual_ranks(ctx->A, ctx->A_input_val, ctx->eptn, ctx->nranks, ctx->ol_dist, ctx->ol,
-                  ctx->num_subdomains, radius1, min_asize1, max_asize1, strong_conn1, out, rcm,
+                  ctx->num_subdomains, radius1, min_asize1, max_asize1, strong_conn1, out,
                   &ctx->rank_ws, keep_local);
   } else {
     Csr As = sort_rows_by_column(ctx->A, ctx->A_input_val);
     virtual_ranks(As, As.val, ctx->eptn, ctx->nranks, ctx->ol_dist, ctx->ol, ctx->num_subdomains,
-                  radius1, min_asize1, max_asize1, strong_conn1, out, rcm, &ctx->rank_ws, keep_local,
+                  radius1, min_asize1, max_asize1, strong_conn1, out, &ctx->rank_ws, keep_local,
                   &As.src);
   }
 }
@@ -1064,24 +1264,13 @@ static void phase_aggregate(doug_ctx* ctx, const std::vector<double>& scaled,
     form(nf, full, ctx->ffull);
   } else if (ctx->nranks > 0) {
     // each rank aggregates its own rows of the values as read
-    // with at least one rank per worker thread the ranks also put their
-    // subdomains in the factor order of the device copy (reverse
-    // Cuthill-McKee over A's pattern); with fewer ranks the threaded
-    // block_rcm of the subdomain preparation keeps every thread busy.
-    // When the subdomain work is prepared beside the coarse build (doug_setup)
-    // that order is left to it too: only the aggregates are needed before
-    // the coarse space can start.
     const bool beside = p.fine_method == 1 && ctx->ol_dist == 1 && ctx->smoothers == 1 &&
                         ctx->use_device_coarse && ctx->inj_nagr == 0 && ctx->has_coarse;
-    const Csr* rcm = (p.fine_method == 1 && ctx->local_order == 1 && ctx->device >= 0 &&
-                      ctx->nranks >= setup_threads() && !beside)
-                         ? &ctx->A
-                         : nullptr;
     // the device coarse build forms the several-process coarse space from
     // the whole matrix: the ranks' local matrices (and their ghost rows) are
     // then not kept; the host build, should it be needed, forms them again
     ctx->ranks_kept_local = !beside || ctx->device < 0;
-    run_virtual_ranks(ctx, ctx->rsetup, rcm, ctx->ranks_kept_local);
+    run_virtual_ranks(ctx, ctx->rsetup, ctx->ranks_kept_local);
     ctx->fin = std::move(ctx->rsetup.inner);
     ctx->ffull = std::move(ctx->rsetup.full);
   } else {
@@ -1624,6 +1813,20 @@ static int setup_host(doug_ctx* ctx) {
 static int set_trsv_order(doug_ctx* ctx, int order) {
   ctx->trsv_order = order;
   ctx->d_sub_trsv = ctx->d_sub;
+  ctx->d_fsub_solve = ctx->d_fsub;
+  if (order == 1 && ctx->fronts) {
+    std::vector<int64_t> size(ctx->h_fsub.size());
+    std::vector<int> by((size_t)ctx->h_fsub.size());
+    std::iota(by.begin(), by.end(), 0);
+    for (size_t b = 0; b < size.size(); b++)
+      size[b] = (b + 1 < size.size() ? ctx->h_fsub[b + 1].base : ctx->factor_elems) - ctx->h_fsub[b].base;
+    std::stable_sort(by.begin(), by.end(), [&](int a, int b) { return size[a] > size[b]; });
+    std::vector<FrontSub> sorted;
+    for (int b : by) sorted.push_back(ctx->h_fsub[b]);
+    int rc = upload(ctx, &ctx->d_fsub_solve, sorted);
+    if (rc) return rc;
+    HIPCHK(hipStreamSynchronize(ctx->stream));  // `sorted` goes out of scope
+  }
   if (order == 0 || ctx->h_sub.empty()) return DOUG_OK;
   std::vector<BlockDesc> sorted(ctx->h_sub);
   std::stable_sort(sorted.begin(), sorted.end(),
@@ -1850,6 +2053,35 @@ static int host_values_now(doug_ctx* ctx) {
   return DOUG_OK;
 }
 
+// Unknown lists and occurrence lists (for the deterministic overlap sum: a
+// node's occurrences in ascending subdomain order), the latter formed on the
+// device: counts per node, their prefix sum, and the positions stably sorted
+// on their node.  Enqueued: `dinds` has to outlive the stream's work.
+static int make_lists(doug_ctx* ctx, const std::vector<int>& dinds, LocalLists& L) {
+  const int n = ctx->A.nrows;
+  const int64_t total = (int64_t)dinds.size();
+  hipStream_t st = ctx->stream;
+  int32_t *cnt, *keys_out, *iota;
+  int rc;
+  if ((rc = upload(ctx, &L.inds, dinds)) || (rc = dalloc(ctx, &L.occ_ptr, (size_t)n + 1)) ||
+      (rc = dalloc(ctx, &cnt, (size_t)n + 1)) || (rc = dalloc(ctx, &L.occ_pos, (size_t)total)) ||
+      (rc = dalloc(ctx, &keys_out, (size_t)total)) || (rc = dalloc(ctx, &iota, (size_t)total)))
+    return rc;
+  HIPCHK(hipMemsetAsync(cnt, 0, ((size_t)n + 1) * sizeof(int32_t), st));
+  launch_key_histogram(total, L.inds, cnt, st);
+  launch_iota(total, iota, st);
+  int end_bit = 1;
+  while (end_bit < 31 && (1 << end_bit) <= n) end_bit++;
+  size_t scan_bytes = 0, sort_bytes = 0;
+  HIPCHK(exclusive_scan(nullptr, scan_bytes, cnt, L.occ_ptr, n + 1, st));
+  HIPCHK(stable_sort_pairs(nullptr, sort_bytes, L.inds, keys_out, iota, L.occ_pos, (int)total, end_bit, st));
+  char* tmp;
+  if ((rc = dalloc(ctx, &tmp, std::max(scan_bytes, sort_bytes)))) return rc;
+  HIPCHK(exclusive_scan(tmp, scan_bytes, cnt, L.occ_ptr, n + 1, st));
+  HIPCHK(stable_sort_pairs(tmp, sort_bytes, L.inds, keys_out, iota, L.occ_pos, (int)total, end_bit, st));
+  return DOUG_OK;
+}
+
 static int device_fine(doug_ctx* ctx, hipEvent_t ev0, hipEvent_t ev1) {
   const Params& p = ctx->p;
   doug_info& info = ctx->info;
@@ -1861,47 +2093,43 @@ static int device_fine(doug_ctx* ctx, hipEvent_t ev0, hipEvent_t ev1) {
   // the reference's order): reverse Cuthill-McKee narrows the factor's
   // tile envelope
   std::vector<int> dinds;
+  std::vector<FrontPattern> pats;
+  std::vector<int> pat;
+  ctx->fronts = false;
+  ctx->h_sub.clear();
+  ctx->h_fsub.clear();
   if (p.fine_method == 1 && ctx->local_order == 1) {
-    if (ctx->nranks > 0 && ctx->rsetup.dinds.size() == ctx->sinds.size())
-      dinds = std::move(ctx->rsetup.dinds);  // ordered by the ranks' workers
-    else
-      block_rcm(A, ctx->sstarts, ctx->sinds, dinds, &ctx->rank_ws);
+    // frontal factors: 2.7 times fewer entries than the envelopes on cubes of
+    // 18^3 unknowns, 3.7 times on squares of 66^2; as long as the solve's work
+    // vector fits a workgroup's LDS
+    const int64_t max_work = 160 * 1024 / (ctx->precision == DOUG_PREC_FP32_FACTORS ? 4 : 8) - 64;
+    const bool f32 = ctx->precision == DOUG_PREC_FP32_FACTORS;
+    // eight wavefronts where two workgroups share a CU (512 subdomains, FP64:
+    // 806 us, 852 us with sixteen), sixteen where there is a CU for each (9
+    // subdomains: 113 us, 122 us with eight)
+    ctx->front_nw = ctx->nsub > 256 ? 8 : 16;
+    // (the envelope solve's size limit holds for either: the batched solve uses it)
+    bool sizes = true;
+    for (size_t b = 0; b + 1 < ctx->sstarts.size(); b++)
+      sizes = sizes && ctx->sstarts[b + 1] - ctx->sstarts[b] <= kMaxTrsvTiles * kTile;
+    ctx->fronts = sizes && build_front_patterns(A, ctx->sstarts, ctx->sinds, max_work, ctx->front_nw, f32 ? 8 : 4,
+                                                pats, pat, dinds);
+    if (!ctx->fronts) block_rcm(A, ctx->sstarts, ctx->sinds, dinds, &ctx->rank_ws);
   } else {
     dinds = ctx->sinds;
     if (p.fine_method == 2)  // Gauss-Seidel sweeps the rows in ascending order
       for (size_t b = 0; b + 1 < ctx->sstarts.size(); b++)
         std::sort(dinds.begin() + ctx->sstarts[b], dinds.begin() + ctx->sstarts[b + 1]);
   }
-  // occurrence lists for the deterministic overlap sum (a node's
-  // occurrences in ascending subdomain order), formed on the device: counts
-  // per node, their prefix sum, and the positions stably sorted on their node
-  if ((rc = upload(ctx, &ctx->d_inds, dinds))) return rc;
-  const int64_t total = (int64_t)dinds.size();
-  if ((rc = dalloc(ctx, &ctx->d_occ_ptr, (size_t)n + 1))) return rc;
   hipStream_t st = ctx->stream;
   if (p.fine_method >= 1) {
-    int32_t *cnt, *keys_out, *iota;
-    if ((rc = dalloc(ctx, &cnt, (size_t)n + 1)) || (rc = dalloc(ctx, &ctx->d_occ_pos, (size_t)total)) ||
-        (rc = dalloc(ctx, &keys_out, (size_t)total)) || (rc = dalloc(ctx, &iota, (size_t)total)))
-      return rc;
-    HIPCHK(hipMemsetAsync(cnt, 0, ((size_t)n + 1) * sizeof(int32_t), st));
-    launch_key_histogram(total, ctx->d_inds, cnt, st);
-    launch_iota(total, iota, st);
-    int end_bit = 1;
-    while (end_bit < 31 && (1 << end_bit) <= n) end_bit++;
-    size_t scan_bytes = 0, sort_bytes = 0;
-    HIPCHK(exclusive_scan(nullptr, scan_bytes, cnt, ctx->d_occ_ptr, n + 1, st));
-    HIPCHK(stable_sort_pairs(nullptr, sort_bytes, ctx->d_inds, keys_out, iota, ctx->d_occ_pos, (int)total,
-                             end_bit, st));
-    char* tmp;
-    if ((rc = dalloc(ctx, &tmp, std::max(scan_bytes, sort_bytes)))) return rc;
-    HIPCHK(exclusive_scan(tmp, scan_bytes, cnt, ctx->d_occ_ptr, n + 1, st));
-    HIPCHK(stable_sort_pairs(tmp, sort_bytes, ctx->d_inds, keys_out, iota, ctx->d_occ_pos, (int)total,
-                             end_bit, st));
+    if ((rc = make_lists(ctx, dinds, ctx->lists))) return rc;
   } else {  // no fine solves: z starts as r (FinePreconditioner_Apply, type NONE)
-    if ((rc = dalloc(ctx, &ctx->d_occ_pos, (size_t)n))) return rc;
-    launch_iota((int64_t)n + 1, ctx->d_occ_ptr, st);
-    launch_iota(n, ctx->d_occ_pos, st);
+    if ((rc = upload(ctx, &ctx->lists.inds, dinds)) || (rc = dalloc(ctx, &ctx->lists.occ_ptr, (size_t)n + 1)) ||
+        (rc = dalloc(ctx, &ctx->lists.occ_pos, (size_t)n)))
+      return rc;
+    launch_iota((int64_t)n + 1, ctx->lists.occ_ptr, st);
+    launch_iota(n, ctx->lists.occ_pos, st);
   }
   if ((rc = dalloc(ctx, &ctx->d_subsol, ctx->sinds.size()))) return rc;
   for (double** v : {&ctx->d_x, &ctx->d_r, &ctx->d_z, &ctx->d_p, &ctx->d_q, &ctx->d_b, &ctx->d_tmp})
@@ -1918,49 +2146,40 @@ static int device_fine(doug_ctx* ctx, hipEvent_t ev0, hipEvent_t ev1) {
   // ---- Factorise_subdomains (subsolvers.F90:78-163) ----
   int64_t elems = 0;
   size_t esize = ctx->precision == DOUG_PREC_FP32_FACTORS ? sizeof(float) : sizeof(double);
-  std::vector<int> offcount;
   if (p.fine_method == 1) {
     // duplicate (i, j) pairs would race in the device scatter: the host
     // scatter map finds whether one falls inside a subdomain (and is the
     // one DOUG_OPT_DEVICE_BLOCKS 0 asks for)
     if (ctx->dup_state < 0) ctx->dup_state = has_duplicate_entries(A) ? 1 : 0;
     const bool dup = ctx->dup_state == 1 || !ctx->use_device_blocks;
-    if (ctx->precision == DOUG_PREC_FP32_FACTORS) {
-      if ((rc = dup ? build_blocks(ctx, A, ctx->d_val, ctx->sstarts, dinds, true, true, ctx->h_sub,
-                                   &ctx->d_sub, &ctx->d_tiles32, &elems, offcount, &info.factor_flops)
-                    : build_blocks_device(ctx, ctx->sstarts, ctx->h_sub, &ctx->d_sub, &ctx->d_tiles32,
-                                          &elems, offcount, &info.factor_flops)))
-        return rc;
-      HIPCHK(hipEventRecord(ev0, ctx->stream));
-      if ((rc = enqueue_factor(ctx, ctx->d_tiles32, ctx->d_sub, ctx->h_sub, offcount, ctx->d_flag)))
-        return rc;
+    if (ctx->fronts) {
+      rc = ctx->precision == DOUG_PREC_FP32_FACTORS
+               ? build_fronts(ctx, A, ctx->sstarts, dinds, pats, pat, dup, &ctx->d_tiles32, &elems,
+                              &info.factor_flops, ev0, ctx->d_flag)
+               : build_fronts(ctx, A, ctx->sstarts, dinds, pats, pat, dup, &ctx->d_tiles, &elems,
+                              &info.factor_flops, ev0, ctx->d_flag);
     } else {
-      if ((rc = dup ? build_blocks(ctx, A, ctx->d_val, ctx->sstarts, dinds, true, true, ctx->h_sub,
-                                   &ctx->d_sub, &ctx->d_tiles, &elems, offcount, &info.factor_flops)
-                    : build_blocks_device(ctx, ctx->sstarts, ctx->h_sub, &ctx->d_sub, &ctx->d_tiles,
-                                          &elems, offcount, &info.factor_flops)))
-        return rc;
-      HIPCHK(hipEventRecord(ev0, ctx->stream));
-      if ((rc = enqueue_factor(ctx, ctx->d_tiles, ctx->d_sub, ctx->h_sub, offcount, ctx->d_flag)))
-        return rc;
+      rc = ctx->precision == DOUG_PREC_FP32_FACTORS
+               ? envelope_factors(ctx, dinds, ctx->lists, dup, &ctx->d_tiles32, &elems, &info.factor_flops, ev0,
+                                  ctx->d_flag)
+               : envelope_factors(ctx, dinds, ctx->lists, dup, &ctx->d_tiles, &elems, &info.factor_flops, ev0,
+                                  ctx->d_flag);
     }
+    if (rc) return rc;
   } else {
     HIPCHK(hipEventRecord(ev0, ctx->stream));
   }
   HIPCHK(hipEventRecord(ev1, ctx->stream));
   info.factor_bytes = elems * (int64_t)esize;
-  info.factor_tiles = elems / kTileElems;
+  info.factor_tiles = (elems + kTileElems - 1) / kTileElems;
+  ctx->factor_elems = elems;
   if ((rc = set_trsv_order(ctx, ctx->trsv_order))) return rc;
-  ctx->maxnt = 0;
-  ctx->work_rows = 0;
-  for (auto& d : ctx->h_sub) {
-    ctx->maxnt = std::max(ctx->maxnt, d.nt);
-    ctx->work_rows += (int64_t)d.nt * kTile;
+  if (ctx->fronts) {
+    if (ctx->precision == DOUG_PREC_FP32_FACTORS)
+      prepare_front_solve<float>(ctx->maxwork);
+    else
+      prepare_front_solve<double>(ctx->maxwork);
   }
-  if (ctx->precision == DOUG_PREC_FP32_FACTORS)
-    prepare_trsv<float>(ctx->maxnt);
-  else
-    prepare_trsv<double>(ctx->maxnt);
   return DOUG_OK;
 }
 
@@ -2143,7 +2362,7 @@ int doug_setup(doug_ctx* ctx, int32_t precision) {
         // the same decomposition again, now keeping each rank's local
         // matrix (the aggregation is deterministic: the same results)
         RankSetup again;
-        run_virtual_ranks(ctx, again, nullptr, true);
+        run_virtual_ranks(ctx, again, true);
         ctx->rsetup.ranks = std::move(again.ranks);
         ctx->ranks_kept_local = true;
       }
@@ -2347,17 +2566,26 @@ static PrecWork ctx_work(doug_ctx* ctx) {
 static void enqueue_subdomain_solves(doug_ctx* ctx, const double* r, double* subsol,
                                      const double* skip = nullptr) {
   if (ctx->p.fine_method == 2) {  // FinePreconditioner_sgs_Apply
-    launch_gather_positions((int64_t)ctx->sinds.size(), ctx->d_inds, r, subsol, ctx->stream);
+    launch_gather_positions((int64_t)ctx->sinds.size(), ctx->lists.inds, r, subsol, ctx->stream);
     launch_sgs(ctx->d_sgs, ctx->nsub, ctx->sgs_mmax, ctx->d_sgs_levptr, ctx->d_sgs_lrows,
                ctx->d_sgs_rbeg, ctx->d_sgs_rlen, ctx->d_sgs_col, ctx->d_sgs_val, ctx->d_sgs_diag,
                subsol, ctx->sgs_iters, ctx->stream);
     return;
   }
+  if (ctx->fronts) {
+    if (ctx->precision == DOUG_PREC_FP32_FACTORS)
+      launch_front_solve(ctx->d_tiles32, ctx->d_fsub_solve, ctx->nsub, ctx->front_nw, ctx->maxwork, ctx->lists.inds, r, subsol,
+                         ctx->stream, skip);
+    else
+      launch_front_solve(ctx->d_tiles, ctx->d_fsub_solve, ctx->nsub, ctx->front_nw, ctx->maxwork, ctx->lists.inds, r, subsol,
+                         ctx->stream, skip);
+    return;
+  }
   if (ctx->precision == DOUG_PREC_FP32_FACTORS)
-    launch_trsv(ctx->d_tiles32, ctx->d_sub_trsv, ctx->nsub, ctx->maxnt, ctx->d_inds, r, subsol,
+    launch_trsv(ctx->d_tiles32, ctx->d_sub_trsv, ctx->nsub, ctx->maxnt, ctx->lists.inds, r, subsol,
                 ctx->stream, skip);
   else
-    launch_trsv(ctx->d_tiles, ctx->d_sub_trsv, ctx->nsub, ctx->maxnt, ctx->d_inds, r, subsol,
+    launch_trsv(ctx->d_tiles, ctx->d_sub_trsv, ctx->nsub, ctx->maxnt, ctx->lists.inds, r, subsol,
                 ctx->stream, skip);
 }
 
@@ -2397,11 +2625,11 @@ static void enqueue_prec(doug_ctx* ctx, const double* r, double* z, const PrecWo
     fine_src = w.subsol;
   }
   if (dot)
-    launch_overlap_sum_dot(ctx->n, fine ? ctx->d_occ_ptr : nullptr, ctx->d_occ_pos, fine_src,
+    launch_overlap_sum_dot(ctx->n, fine ? ctx->lists.occ_ptr : nullptr, ctx->lists.occ_pos, fine_src,
                            coarse ? ctx->d_Rtptr : nullptr, ctx->d_Rtcol, ctx->d_Rtval, w.csol, z, r,
                            ctx->d_partial, ctx->d_scal, ctx->stream);
   else
-    launch_overlap_sum(ctx->n, fine ? ctx->d_occ_ptr : nullptr, ctx->d_occ_pos, fine_src,
+    launch_overlap_sum(ctx->n, fine ? ctx->lists.occ_ptr : nullptr, ctx->lists.occ_pos, fine_src,
                        coarse ? ctx->d_Rtptr : nullptr, ctx->d_Rtcol, ctx->d_Rtval, w.csol, z,
                        ctx->stream);
 }
@@ -2748,6 +2976,34 @@ static int next_pow2(int v) {
   return p;
 }
 
+// The envelope factors of the batched solve: the single-vector solve's own
+// where it uses envelopes, else built here.  For 32 columns the envelope's
+// 64 x 64 tiles keep the matrix cores busier than fronts of 4 to 64 columns
+// do, which makes up for 2.7 times as many entries: on 512 subdomains of 5440
+// unknowns an application took 2.83 ms with either in FP32, and 4.6 ms against
+// 5.1 ms with fronts in FP64.
+static int batch_factors(doug_ctx* ctx) {
+  ctx->batch_lists = ctx->lists;
+  ctx->d_btiles = ctx->d_tiles;
+  ctx->d_btiles32 = ctx->d_tiles32;
+  if (!ctx->fronts) return DOUG_OK;
+  std::vector<int> dinds;
+  block_rcm(ctx->A, ctx->sstarts, ctx->sinds, dinds, &ctx->rank_ws);
+  int *d_flag, flag = 0, rc;
+  if ((rc = make_lists(ctx, dinds, ctx->batch_lists)) || (rc = dalloc(ctx, &d_flag, 1))) return rc;
+  HIPCHK(hipMemsetAsync(d_flag, 0, sizeof(int), ctx->stream));
+  const bool host_map = ctx->dup_state == 1 || !ctx->use_device_blocks;
+  int64_t elems;
+  rc = ctx->precision == DOUG_PREC_FP32_FACTORS
+           ? envelope_factors(ctx, dinds, ctx->batch_lists, host_map, &ctx->d_btiles32, &elems, nullptr, nullptr, d_flag)
+           : envelope_factors(ctx, dinds, ctx->batch_lists, host_map, &ctx->d_btiles, &elems, nullptr, nullptr, d_flag);
+  if (rc || (rc = set_trsv_order(ctx, ctx->trsv_order))) return rc;
+  HIPCHK(hipMemcpyAsync(&flag, d_flag, sizeof(int), hipMemcpyDeviceToHost, ctx->stream));
+  HIPCHK(hipStreamSynchronize(ctx->stream));
+  if (flag) return fail(ctx, DOUG_E_NUMERIC, "subdomain " + std::to_string(flag - 1) + " is not positive definite");
+  return DOUG_OK;
+}
+
 int doug_prepare_batch(doug_ctx* ctx) {
   if (!ctx) return DOUG_E_ARG;
   if (!ctx->ready) return fail(ctx, DOUG_E_STATE, "doug_prepare_batch before doug_setup");
@@ -2760,8 +3016,8 @@ int doug_prepare_batch(doug_ctx* ctx) {
   hipStream_t st = ctx->stream;
   int rc;
   if (ctx->p.fine_method == 1) {
-    // panels of the envelope solves; the factors themselves are shared with
-    // the single right-hand-side path
+    if ((rc = batch_factors(ctx))) return rc;
+    // panels of the envelope solves
     if (ctx->precision == DOUG_PREC_FP32_FACTORS) {
       float* u;
       if ((rc = dalloc(ctx, &u, (size_t)ctx->work_rows * NR))) return rc;
@@ -2821,19 +3077,19 @@ static void enqueue_prec_multi(doug_ctx* ctx, int nrp, const double* r, double* 
   const double* fine_src = r;
   if (p.fine_method == 1) {
     if (ctx->precision == DOUG_PREC_FP32_FACTORS)
-      launch_trsm_multi(ctx->d_tiles32, ctx->d_sub_trsv, ctx->nsub, ctx->d_inds, r, nrp,
+      launch_trsm_multi(ctx->d_btiles32, ctx->d_sub_trsv, ctx->nsub, ctx->batch_lists.inds, r, nrp,
                         (float*)ctx->d_U, ctx->d_subsolm, nrp, nrp, NR, ctx->trsm_kb, ctx->trsm_cg, st);
     else
-      launch_trsm_multi(ctx->d_tiles, ctx->d_sub_trsv, ctx->nsub, ctx->d_inds, r, nrp,
+      launch_trsm_multi(ctx->d_btiles, ctx->d_sub_trsv, ctx->nsub, ctx->batch_lists.inds, r, nrp,
                         (double*)ctx->d_U, ctx->d_subsolm, nrp, nrp, NR, ctx->trsm_kb, ctx->trsm_cg, st);
     fine_src = ctx->d_subsolm;
   }
   if (rz_dot)
-    launch_overlap_sum_dot_multi2(n, nrp, ctx->d_occ_ptr, ctx->d_occ_pos, fine_src,
+    launch_overlap_sum_dot_multi2(n, nrp, ctx->batch_lists.occ_ptr, ctx->batch_lists.occ_pos, fine_src,
                                   coarse ? ctx->d_Rtptr : nullptr, ctx->d_Rtcol, ctx->d_Rtval, ctx->d_cS, NR,
                                   z, r, ctx->d_partialm, ctx->d_counterm, ctx->d_scalm, st);
   else
-    launch_overlap_sum_multi(n, nrp, ctx->d_occ_ptr, ctx->d_occ_pos, fine_src, coarse ? ctx->d_Rtptr : nullptr,
+    launch_overlap_sum_multi(n, nrp, ctx->batch_lists.occ_ptr, ctx->batch_lists.occ_pos, fine_src, coarse ? ctx->d_Rtptr : nullptr,
                              ctx->d_Rtcol, ctx->d_Rtval, ctx->d_cS, NR, z, st);
 }
 
@@ -3167,7 +3423,9 @@ int doug_autotune(doug_ctx* ctx, int32_t reps, doug_tuning* out) {
         (rc = time_launches(ctx, rt, [&]() { enqueue_subdomain_solves(ctx, ctx->d_r); }, &tu.trsv_ms[0])))
       return rc;
     bool sorted = true;
-    for (int i = 1; i < ctx->nsub; i++) sorted = sorted && ctx->h_sub[i - 1].nt >= ctx->h_sub[i].nt;
+    for (int i = 1; i < ctx->nsub; i++)
+      sorted = sorted && (ctx->fronts ? ctx->h_fsub[i - 1].n >= ctx->h_fsub[i].n
+                                      : ctx->h_sub[i - 1].nt >= ctx->h_sub[i].nt);
     if (!sorted) {
       if ((rc = set_trsv_order(ctx, 1)) ||
           (rc = time_launches(ctx, rt, [&]() { enqueue_subdomain_solves(ctx, ctx->d_r); }, &tu.trsv_ms[1])))

@@ -1,0 +1,823 @@
+// gfx950 kernels of the frontal subdomain factors (doug_fronts.hpp): scatter
+// of the matrix entries, the factorisation height by height, and the solves
+// for one and for several right-hand sides.
+#include "doug_tile.hpp"
+#include "doug_front_kernels.hpp"
+
+namespace doug {
+
+namespace {
+
+// Pointers out of a descriptor are generic: as global ones their loads do not
+// count as LDS accesses.
+template <typename U>
+using Global = const U __attribute__((address_space(1))) *;
+template <typename U>
+__device__ __forceinline__ Global<U> global(const U* p) {
+  return reinterpret_cast<Global<U>>(reinterpret_cast<uint64_t>(p));
+}
+
+// A value that is the same in every lane, in a scalar register.
+__device__ __forceinline__ int uniform(int v) { return __builtin_amdgcn_readfirstlane(v); }
+
+// element (row, col) of a panel of H rows (host: front_elem)
+template <typename T>
+__device__ __forceinline__ int panel_elem(int H, int row, int col) {
+  const int g = col >> 2, j = col & 3, base = 4 * (g * H - 2 * g * (g - 1));
+  if (sizeof(T) == 4) return base + 4 * (row - 4 * g) + j;
+  return base + (j >> 1) * 2 * (H - 4 * g) + 2 * (row - 4 * g) + (j & 1);
+}
+
+// The four entries of column group g in one row: the panel is streamed once
+// per pass, so its loads are non-temporal.
+template <typename T>
+struct Quad;
+template <>
+struct Quad<float> {
+  typedef float v4 __attribute__((ext_vector_type(4)));
+  v4 a;
+  __device__ __forceinline__ void load(const float* pan, int H, int g, int row) {
+    // 32-bit offsets from a uniform base keep the addresses in one register
+    const uint32_t o = 16u * (uint32_t)(row + g * (H - 2 * g - 2));
+    a = __builtin_nontemporal_load(reinterpret_cast<const v4*>(reinterpret_cast<const char*>(pan) + o));
+  }
+  __device__ __forceinline__ float get(int j) const { return a[j]; }
+  __device__ __forceinline__ void zero() { a = v4{0, 0, 0, 0}; }
+};
+template <>
+struct Quad<double> {
+  typedef double v2 __attribute__((ext_vector_type(2)));
+  v2 a, b;
+  __device__ __forceinline__ void load(const double* pan, int H, int g, int row) {
+    const uint32_t o = 16u * (uint32_t)(2 * g * H - 4 * g * (g - 1) + row - 4 * g);
+    a = __builtin_nontemporal_load(reinterpret_cast<const v2*>(reinterpret_cast<const char*>(pan) + o));
+    b = __builtin_nontemporal_load(
+        reinterpret_cast<const v2*>(reinterpret_cast<const char*>(pan) + (o + 16u * (uint32_t)(H - 4 * g))));
+  }
+  __device__ __forceinline__ double get(int j) const { return j < 2 ? a[j & 1] : b[j & 1]; }
+  __device__ __forceinline__ void zero() { a = v2{0, 0}; b = v2{0, 0}; }
+};
+
+__device__ __forceinline__ float lane_value(float v, int l) {
+  return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), l));
+}
+__device__ __forceinline__ double lane_value(double v, int l) {
+  const int lo = __builtin_amdgcn_readlane(__double2loint(v), l);
+  const int hi = __builtin_amdgcn_readlane(__double2hiint(v), l);
+  return __hiloint2double(hi, lo);
+}
+
+// ------------------------------------------------------------------------
+// set-up
+// ------------------------------------------------------------------------
+
+// The lower entries of each subdomain's matrix into its zeroed panels; A must
+// hold no (i, j) pair twice.
+template <typename T>
+__global__ __launch_bounds__(256) void k_front_scatter(T* __restrict__ tiles, const FrontSub* __restrict__ subs,
+                                                       const int32_t* __restrict__ inds,
+                                                       const int32_t* __restrict__ occ_ptr,
+                                                       const int32_t* __restrict__ occ_pos,
+                                                       const int32_t* __restrict__ a_ptr,
+                                                       const int32_t* __restrict__ a_col,
+                                                       const double* __restrict__ a_val) {
+  const FrontSub s = subs[blockIdx.x];
+  const int s0 = (int)s.vec;
+  for (int p = blockIdx.y * 256 + threadIdx.x; p < s.n; p += 256 * gridDim.y) {
+    const int g = inds[s0 + p];
+    for (int e = a_ptr[g]; e < a_ptr[g + 1]; e++) {
+      const int q = local_col(occ_ptr, occ_pos, a_col[e], s0, s.n);
+      if (q < 0 || q > p) continue;
+      const Front f = s.fronts[s.colfront[q]];
+      int row = p - f.c0;
+      if (row >= f.k) {  // a boundary row: its place in the ascending list
+        const uint16_t* rp = s.rpos + f.row0;
+        int lo = f.k, hi = f.k + f.m;
+        while (hi - lo > 1) {
+          const int mid = (lo + hi) >> 1;
+          if (rp[mid] <= p) lo = mid;
+          else hi = mid;
+        }
+        row = lo;
+      }
+      tiles[s.base + f.pan + panel_elem<T>(f.k + f.m, row, q - f.c0)] = (T)a_val[e];
+    }
+  }
+}
+
+// Cholesky factor of a k x k block (k <= 32) at As (row stride LDX, lower
+// part) and D = L^-1 at Bs, zeros right of the diagonal, by one wavefront in
+// registers: lane r holds row r, a column step broadcasts the pivot column's
+// entries through scalar registers (v_readlane), so that a step waits on no
+// LDS access or cross-lane permute.  D by rows, x L = e_r, last column first.
+// As ends with L.  A non-positive pivot is replaced by 1 and reported as `id`.
+template <typename T, int LDX>
+__device__ __forceinline__ void wave_factor_invert(T* As, T* Bs, int k, int lane, int id, int* flag) {
+  constexpr int KB = 32;
+  T v[KB];
+  const int r = lane & 31;
+#pragma unroll
+  for (int c = 0; c < KB; c++) v[c] = As[r * LDX + c];
+  T rinv = (T)0;  // lane r: 1 / L_rr
+#pragma unroll
+  for (int c = 0; c < KB; c++)
+    if (c < k) {
+      T piv = lane_value(v[c], c);
+      if (!(piv > (T)0)) {
+        if (lane == 0) atomicCAS(flag, 0, id);
+        piv = (T)1;
+      }
+      const T sc = rsqrt(piv);
+      rinv = lane == c ? sc : rinv;
+      v[c] = lane == c ? piv * sc : v[c] * sc;
+#pragma unroll
+      for (int q0 = c + 1 - (c + 1) % 8; q0 < KB; q0 += 8)
+        if (q0 < k) {
+#pragma unroll
+          for (int q = q0; q < q0 + 8; q++)
+            if (q > c) v[q] = v[q] - v[c] * lane_value(v[c], q);
+        }
+    }
+  if (lane < k) {
+#pragma unroll
+    for (int c = 0; c < KB; c++)
+      if (c < k) As[lane * LDX + c] = c <= lane ? v[c] : (T)0;
+  }
+  if (sizeof(T) == 8) wave_lds_sync();
+  T x[KB];
+#pragma unroll
+  for (int c = 0; c < KB; c++) x[c] = lane == c ? (T)1 : (T)0;
+#pragma unroll
+  for (int c = KB - 1; c >= 0; c--)
+    if (c < k) {
+      x[c] = x[c] * lane_value(rinv, c);
+      // L's row c: from its lane (FP32), or from LDS where two sets of rows
+      // would take too many registers
+#pragma unroll
+      for (int j = 0; j < c; j++) x[j] = x[j] - x[c] * (sizeof(T) == 4 ? lane_value(v[j], c) : As[c * LDX + j]);
+    }
+  if (lane < k) {
+#pragma unroll
+    for (int c = 0; c < KB; c++)
+      if (c < k) Bs[lane * LDX + c] = c <= lane ? x[c] : (T)0;
+  }
+}
+
+// A child's update matrix as the parent reads it.
+template <typename T>
+struct Child {
+  const T* s;
+  int m, u;  // rows, work index of its first update entry
+  // row of the child that record x (half c) names, -1 if none
+  __device__ __forceinline__ int row(uint32_t x, int c, int none) const {
+    const int i = c == 0 ? (int)(x & 0xffffu) : (int)(x >> 16);
+    return i != none ? i - u : -1;
+  }
+  // entry (i, j), or entry 0 where either is missing; see kept()
+  __device__ __forceinline__ T read(int i, int j) const { return s[(uint32_t)(i >= 0 && j >= 0 ? i * m + j : 0)]; }
+};
+template <typename T>
+__device__ __forceinline__ T kept(T x, int i, int j) {
+  return i >= 0 && j >= 0 ? x : (T)0;
+}
+
+// One front of height h per workgroup of NW wavefronts (its children's update
+// matrices are complete), fronts of at most 16 NB columns, or with NB = 4
+// those of more than 32.  The pivot block and its inverse D in LDS; then each
+// wavefront takes 16 boundary rows at a time, L_RS = F_RS D^T, kept in the
+// panel; then 32x32 tiles of the update matrix F_RR - L_RS L_RS^T, their
+// operands read from the panel (through L2) straight into the matrix cores'
+// registers; and last C = L_RS D over L_RS.  Only three workgroup barriers
+// follow the pivot block, and LDS holds nothing but that block, so that many
+// fronts are in flight per CU: the work is bound by the latency of short
+// dependent steps, not by arithmetic or bandwidth.  Whole factorisation, 512
+// subdomains of 5440 unknowns: 11.7 ms in FP64 and 8.7 ms in FP32 (11.9 and
+// 7.4 ms for the envelope factor with its 2.7 times as many entries); 64 of
+// 3900 in two dimensions: 1.5 ms (4.7 ms).
+template <typename T, int NB, int NW>
+__global__ __launch_bounds__(64 * NW) void k_front_factor(T* tiles, T* schur, const FrontSub* __restrict__ subs,
+                                                          int h, int* __restrict__ flag) {
+  constexpr int KB = 16 * NB, LDX = KB + 1, NG = 4 * NB;
+  __shared__ T As[KB * LDX];
+  __shared__ T Bs[KB * LDX];
+  __shared__ int mc[2][KB];  // rows of the children for the pivot columns
+  typedef typename Mma<T>::v4 V;
+  const FrontSub s = subs[blockIdx.x];
+  if (h >= s.nheights) return;
+  const int fi = s.hptr[h] + blockIdx.y;
+  if (fi >= s.hptr[h + 1]) return;
+  const Front f = s.fronts[s.hlist[fi]];
+  const int k = uniform(f.k), m = uniform(f.m), H = k + m, ng = (k + 3) >> 2, n = s.n;
+  if (NB == 4 ? k <= 32 : k > KB) return;
+  const int t = threadIdx.x, lane = t & 63, w = __builtin_amdgcn_readfirstlane(t >> 6);
+  const int li = lane & 15, lk = lane >> 4;
+  T* pan = tiles + s.base + uniform(f.pan);
+  T* S = schur + s.sch + uniform(f.sch);
+  const Global<uint32_t> src = global(s.src) + uniform(f.row0);
+  Child<T> kid[2];
+#pragma unroll
+  for (int c = 0; c < 2; c++) {
+    const int i = uniform(f.child[c]);
+    const Front q = s.fronts[max(i, 0)];
+    kid[c] = Child<T>{schur + s.sch + uniform(q.sch), i >= 0 ? uniform(q.m) : 0, uniform(q.u)};
+  }
+  const bool grown = kid[0].m > 0 || kid[1].m > 0;
+  if (t < KB) {
+    const uint32_t x = t < k ? src[t] : 0u;
+#pragma unroll
+    for (int c = 0; c < 2; c++) mc[c][t] = t < k && kid[c].m > 0 ? kid[c].row(x, c, n) : -1;
+  }
+  if (k > 0) {
+    // pivot block: the lower entries of the matrix, the children's, ones on
+    // the diagonal past the last column.  Every thread's loads are issued
+    // before the first is used.
+    constexpr int PER = KB * KB / (64 * NW) > 0 ? KB * KB / (64 * NW) : 1;
+    if (grown) __syncthreads();
+    T v[PER], u[2][PER];
+#pragma unroll
+    for (int q = 0; q < PER; q++) {
+      const int e = t + 64 * NW * q, r = e / KB, c = e % KB;
+      v[q] = pan[(uint32_t)(r < k && c <= r ? panel_elem<T>(H, r, c) : 0)];
+    }
+#pragma unroll
+    for (int x = 0; x < 2; x++) {
+      if (kid[x].m > 0) {
+#pragma unroll
+        for (int q = 0; q < PER; q++) {
+          const int e = t + 64 * NW * q, r = e / KB, c = e % KB;
+          u[x][q] = kid[x].read(c <= r ? mc[x][min(r, KB - 1)] : -1, mc[x][c]);
+        }
+#pragma unroll
+        for (int q = 0; q < PER; q++) {
+          const int e = t + 64 * NW * q, r = e / KB, c = e % KB;
+          u[x][q] = kept(u[x][q], c <= r ? mc[x][min(r, KB - 1)] : -1, mc[x][c]);
+        }
+      } else {
+#pragma unroll
+        for (int q = 0; q < PER; q++) u[x][q] = (T)0;
+      }
+    }
+#pragma unroll
+    for (int q = 0; q < PER; q++) {
+      const int e = t + 64 * NW * q, r = e / KB, c = e % KB;
+      const T x = r < k && c <= r ? v[q] : r == c ? (T)1 : (T)0;
+      if (r < KB) {
+        As[r * LDX + c] = x + (u[0][q] + u[1][q]);
+        Bs[r * LDX + c] = (T)0;
+      }
+    }
+    __syncthreads();
+    // halves of 32 columns; in between, the second half's block minus
+    // L_21 L_21^T with L_21 = A_21 D_1^T, and last D_21 = -D_2 (L_21 D_1), one
+    // 16x16 block of them per wavefront
+    const int I = (w >> 1) & 1, J = w & 1;
+    auto block = [&](const T* X, const T* Y, bool yt) {  // 16x16 block (I, J) of a 32x32 product
+      V a = V{0, 0, 0, 0};
+#pragma unroll
+      for (int q = 0; q < 8; q++)
+        a = Mma<T>::op(X[(16 * I + li) * LDX + 4 * q + lk],
+                       yt ? Y[(16 * J + li) * LDX + 4 * q + lk] : Y[(4 * q + lk) * LDX + 16 * J + li], a);
+      return a;
+    };
+#pragma unroll 1
+    for (int b = 0; b < (NB == 4 ? 2 : 1); b++) {
+      const int o = 32 * b;
+      if (w == 0)
+        wave_factor_invert<T, LDX>(As + o * LDX + o, Bs + o * LDX + o, min(k - o, 32), lane, (int)blockIdx.x + 1,
+                                   flag);
+      if (NB == 2 || b == 1) break;
+      __syncthreads();
+      T* A21 = As + 32 * LDX;
+      V a = block(A21, Bs, true);
+      __syncthreads();
+      if (w < 4)
+#pragma unroll
+        for (int q = 0; q < 4; q++) A21[(16 * I + Mma<T>::row(lane, q)) * LDX + 16 * J + li] = a[q];
+      __syncthreads();
+      a = block(A21, A21, true);
+      if (w < 4)
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+          T* e = A21 + 32 + (16 * I + Mma<T>::row(lane, q)) * LDX + 16 * J + li;
+          *e = *e - a[q];
+        }
+      __syncthreads();
+    }
+    __syncthreads();
+    if (NB == 4) {
+      V a = block(As + 32 * LDX, Bs, false);  // L_21 D_1
+      __syncthreads();
+      if (w < 4)
+#pragma unroll
+        for (int q = 0; q < 4; q++) As[(32 + 16 * I + Mma<T>::row(lane, q)) * LDX + 16 * J + li] = a[q];
+      __syncthreads();
+      a = block(Bs + 32 * LDX + 32, As + 32 * LDX, false);
+      if (w < 4)
+#pragma unroll
+        for (int q = 0; q < 4; q++) Bs[(32 + 16 * I + Mma<T>::row(lane, q)) * LDX + 16 * J + li] = -a[q];
+      __syncthreads();
+    }
+    // D over the pivot block
+    for (int e = t; e < k * 4 * ng; e += 64 * NW) {
+      const int r = (e >> 2) % k, c = 4 * ((e >> 2) / k) + (e & 3);
+      if (c < 4 * ((r >> 2) + 1)) pan[panel_elem<T>(H, r, c)] = c <= r ? Bs[r * LDX + c] : (T)0;
+    }
+  }
+  if (m == 0) return;
+  if (k == 0) __syncthreads();
+  // L_RS, 16 rows per wavefront at a time (columns past the last one meet
+  // zeros of D)
+  if (k > 0)
+    for (int r0 = 16 * w; r0 < m; r0 += 16 * NW) {
+      const int row = min(k + r0 + li, H - 1);
+      const uint32_t x = src[(uint32_t)row];
+      V acc[NB];
+#pragma unroll
+      for (int q = 0; q < NB; q++) acc[q] = V{0, 0, 0, 0};
+#pragma unroll
+      for (int q0 = 0; q0 < NG; q0 += 8)
+        if (q0 < ng) {
+          T a[8], b[2][8];
+#pragma unroll
+          for (int q = 0; q < 8; q++) a[q] = pan[(uint32_t)panel_elem<T>(H, row, 4 * min(q0 + q, ng - 1) + lk)];
+#pragma unroll
+          for (int c = 0; c < 2; c++)
+            if (kid[c].m > 0) {
+              const int i = kid[c].row(x, c, n);
+              int j[8];
+#pragma unroll
+              for (int q = 0; q < 8; q++) j[q] = mc[c][4 * (q0 + q) + lk];
+#pragma unroll
+              for (int q = 0; q < 8; q++) b[c][q] = kid[c].read(i, j[q]);
+#pragma unroll
+              for (int q = 0; q < 8; q++) b[c][q] = kept(b[c][q], i, j[q]);
+            } else {
+#pragma unroll
+              for (int q = 0; q < 8; q++) b[c][q] = (T)0;
+            }
+#pragma unroll
+          for (int q = 0; q < 8; q++) {
+            const T e = a[q] + (b[0][q] + b[1][q]);
+#pragma unroll
+            for (int c = 0; c < NB; c++)
+              if (4 * (q0 + q) < 16 * (c + 1))  // D is lower triangular
+                acc[c] = Mma<T>::op(e, Bs[(16 * c + li) * LDX + 4 * (q0 + q) + lk], acc[c]);
+          }
+        }
+#pragma unroll
+      for (int c = 0; c < NB; c++)
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+          const int ro = k + r0 + Mma<T>::row(lane, q), co = 16 * c + li;
+          if (ro < H && co < 4 * ng) pan[(uint32_t)panel_elem<T>(H, ro, co)] = acc[c][q];
+        }
+    }
+  __syncthreads();
+  // update matrix, 32x32 tiles of its lower part
+  const int nt = (m + 31) >> 5;
+  for (int e = w; e < nt * (nt + 1) / 2; e += NW) {
+    int I = (int)((sqrtf(8.0f * e + 1.0f) - 1.0f) * 0.5f);
+    while ((I + 1) * (I + 2) / 2 <= e) I++;
+    while (I * (I + 1) / 2 > e) I--;
+    const int J = e - I * (I + 1) / 2;
+    V acc[2][2];
+    zero_acc(acc);
+    uint32_t xc[2], xr[2][4];
+#pragma unroll
+    for (int y = 0; y < 2; y++) xc[y] = src[(uint32_t)min(k + 32 * J + 16 * y + li, H - 1)];
+#pragma unroll
+    for (int x = 0; x < 2; x++)
+#pragma unroll
+      for (int q = 0; q < 4; q++) xr[x][q] = src[(uint32_t)min(k + 32 * I + 16 * x + Mma<T>::row(lane, q), H - 1)];
+#pragma unroll
+    for (int q0 = 0; q0 < NG; q0 += 8)
+      if (q0 < ng) {
+        T a[2][8], b[2][8];
+#pragma unroll
+        for (int x = 0; x < 2; x++) {
+          const int ra = min(k + 32 * I + 16 * x + li, H - 1), rb = min(k + 32 * J + 16 * x + li, H - 1);
+#pragma unroll
+          for (int q = 0; q < 8; q++) {
+            const int c = 4 * min(q0 + q, ng - 1) + lk;
+            a[x][q] = pan[(uint32_t)panel_elem<T>(H, ra, c)];
+            b[x][q] = pan[(uint32_t)panel_elem<T>(H, rb, c)];
+          }
+        }
+#pragma unroll
+        for (int q = 0; q < 8; q++) {
+          const T a0 = q0 + q < ng ? a[0][q] : (T)0, a1 = q0 + q < ng ? a[1][q] : (T)0;
+          acc[0][0] = Mma<T>::op(a0, b[0][q], acc[0][0]);
+          acc[0][1] = Mma<T>::op(a0, b[1][q], acc[0][1]);
+          acc[1][0] = Mma<T>::op(a1, b[0][q], acc[1][0]);
+          acc[1][1] = Mma<T>::op(a1, b[1][q], acc[1][1]);
+        }
+      }
+#pragma unroll
+    for (int x = 0; x < 2; x++) {
+      T v[2][2][4];
+#pragma unroll
+      for (int c = 0; c < 2; c++)
+        if (kid[c].m > 0) {
+          int i[4], j[2];
+#pragma unroll
+          for (int q = 0; q < 4; q++) i[q] = kid[c].row(xr[x][q], c, n);
+#pragma unroll
+          for (int y = 0; y < 2; y++) j[y] = kid[c].row(xc[y], c, n);
+#pragma unroll
+          for (int y = 0; y < 2; y++)
+#pragma unroll
+            for (int q = 0; q < 4; q++) v[c][y][q] = kid[c].read(j[y] <= i[q] ? i[q] : -1, j[y]);
+#pragma unroll
+          for (int y = 0; y < 2; y++)
+#pragma unroll
+            for (int q = 0; q < 4; q++) v[c][y][q] = kept(v[c][y][q], i[q], j[y]);
+        } else {
+#pragma unroll
+          for (int y = 0; y < 2; y++)
+#pragma unroll
+            for (int q = 0; q < 4; q++) v[c][y][q] = (T)0;
+        }
+#pragma unroll
+      for (int y = 0; y < 2; y++)
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+          const int row = 32 * I + 16 * x + Mma<T>::row(lane, q), col = 32 * J + 16 * y + li;
+          if (row < m && col <= row) S[(uint32_t)(row * m + col)] = (v[0][y][q] + v[1][y][q]) - acc[x][y][q];
+        }
+    }
+  }
+  if (k == 0) return;
+  __syncthreads();
+  // C = L_RS D over L_RS
+  for (int r0 = 16 * w; r0 < m; r0 += 16 * NW) {
+    const int row = min(k + r0 + li, H - 1);
+    T a[NG];
+#pragma unroll
+    for (int q = 0; q < NG; q++) a[q] = pan[(uint32_t)panel_elem<T>(H, row, 4 * min(q, ng - 1) + lk)];
+    V acc[NB];
+#pragma unroll
+    for (int c = 0; c < NB; c++) acc[c] = V{0, 0, 0, 0};
+#pragma unroll
+    for (int q = 0; q < NG; q++)
+#pragma unroll
+      for (int c = 0; c < NB; c++)
+        if (4 * q + 3 >= 16 * c) acc[c] = Mma<T>::op(a[q], Bs[(4 * q + lk) * LDX + 16 * c + li], acc[c]);
+#pragma unroll
+    for (int c = 0; c < NB; c++)
+#pragma unroll
+      for (int q = 0; q < 4; q++) {
+        const int ro = k + r0 + Mma<T>::row(lane, q), co = 16 * c + li;
+        if (ro < H && co < 4 * ng) pan[(uint32_t)panel_elem<T>(H, ro, co)] = acc[c][q];
+      }
+  }
+}
+
+// ------------------------------------------------------------------------
+// solve, one right-hand side
+// ------------------------------------------------------------------------
+
+__device__ __forceinline__ float fused(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
+__device__ __forceinline__ double fused(double a, double b, double c) { return __builtin_fma(a, b, c); }
+
+// A lane's 32-bit value as another lane of its row of 16 sees it (DPP).
+template <int CTRL>
+__device__ __forceinline__ float lane_swap(float v) {
+  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xf, 0xf, true));
+}
+template <int CTRL>
+__device__ __forceinline__ double lane_swap(double v) {
+  const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), CTRL, 0xf, 0xf, true);
+  const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), CTRL, 0xf, 0xf, true);
+  return __hiloint2double(hi, lo);
+}
+constexpr int kDppXor1 = 0xB1, kDppXor2 = 0x4E;        // quad_perm
+constexpr int kDppXor8 = 0x128, kDppXor7 = 0x141;      // row_ror:8, row_half_mirror
+
+// a + b after half the lanes have exchanged them: lanes of the lower half
+// (of each 64, or of each 32) return a's sum over the two halves, the others b's.
+__device__ __forceinline__ float fold32(float a, float b) {
+  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+  return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+}
+__device__ __forceinline__ float fold16(float a, float b) {
+  const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+  return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+}
+__device__ __forceinline__ double fold32(double a, double b) {
+  const auto l = __builtin_amdgcn_permlane32_swap(__double2loint(a), __double2loint(b), false, false);
+  const auto h = __builtin_amdgcn_permlane32_swap(__double2hiint(a), __double2hiint(b), false, false);
+  return __hiloint2double(h[0], l[0]) + __hiloint2double(h[1], l[1]);
+}
+__device__ __forceinline__ double fold16(double a, double b) {
+  const auto l = __builtin_amdgcn_permlane16_swap(__double2loint(a), __double2loint(b), false, false);
+  const auto h = __builtin_amdgcn_permlane16_swap(__double2hiint(a), __double2hiint(b), false, false);
+  return __hiloint2double(h[0], l[0]) + __hiloint2double(h[1], l[1]);
+}
+template <int CTRL, typename T>
+__device__ __forceinline__ T fold_row(T a, T b, bool hi) {
+  const T keep = hi ? b : a, send = hi ? a : b;
+  return keep + lane_swap<CTRL>(send);
+}
+
+// v[0..N-1] (N = 16 or 32) summed over the 64 lanes: lane l returns the sum
+// of entry l / (64 / N).  Each halving hands one half of the entries to the
+// other half of the lanes; all exchanges are register-to-register.
+template <typename T, int N>
+__device__ __forceinline__ T reduce_scatter(T (&v)[N], int lane) {
+#pragma unroll
+  for (int q = 0; q < N / 2; q++) v[q] = fold32(v[q], v[q + N / 2]);
+#pragma unroll
+  for (int q = 0; q < N / 4; q++) v[q] = fold16(v[q], v[q + N / 4]);
+#pragma unroll
+  for (int q = 0; q < N / 8; q++) v[q] = fold_row<kDppXor8>(v[q], v[q + N / 8], lane & 8);
+#pragma unroll
+  for (int q = 0; q < N / 16; q++) v[q] = fold_row<kDppXor7>(v[q], v[q + N / 16], lane & 4);
+  if (N == 32)
+    v[0] = fold_row<kDppXor2>(v[0], v[1 % N], lane & 2);
+  else
+    v[0] = v[0] + lane_swap<kDppXor2>(v[0]);
+  return v[0] + lane_swap<kDppXor1>(v[0]);
+}
+
+// Workgroup barrier that orders LDS alone: loads of panels already issued for
+// the units behind it stay in flight.
+__device__ __forceinline__ void lds_barrier() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
+// The work lists are read through the constant address space: the barriers'
+// fences would otherwise send these uniform loads down the vector path.
+typedef const FrontUnit __attribute__((address_space(4))) * UnitPtr;
+__device__ __forceinline__ UnitPtr unit_list(const FrontUnit* p) {
+  return reinterpret_cast<UnitPtr>(reinterpret_cast<uint64_t>(p));
+}
+__device__ __forceinline__ int list_at(const int32_t* p, int i) {
+  typedef const int32_t __attribute__((address_space(4))) * P;
+  return __builtin_amdgcn_readfirstlane(reinterpret_cast<P>(reinterpret_cast<uint64_t>(p))[i]);
+}
+__device__ __forceinline__ FrontUnit unit_at(UnitPtr p) {
+  typedef uint32_t v4 __attribute__((ext_vector_type(4)));
+  typedef const v4 __attribute__((address_space(4))) * P4;
+  const P4 q = (P4)p;
+  const v4 a = q[0], b = q[1];
+  FrontUnit u;
+  u.pan = (int32_t)a[0];
+  u.row0 = (int32_t)a[1];
+  u.h = (uint16_t)a[2];
+  u.k = (uint16_t)(a[2] >> 16);
+  u.c0 = (uint16_t)a[3];
+  u.u = (uint16_t)(a[3] >> 16);
+  u.g0 = (uint8_t)b[0];
+  u.g1 = (uint8_t)(b[0] >> 8);
+  u.chunk = (uint8_t)(b[0] >> 16);
+  u.flags = (uint8_t)(b[0] >> 24);
+  u.nbar = (uint16_t)b[1];
+  return u;
+}
+
+// column groups per unit: 64 rows of them are 8 KB in either precision
+template <typename T>
+constexpr int kUnitGroups = sizeof(T) == 4 ? 8 : 4;
+
+// The loads of one unit: its panel rows, the row records of its rows (lane =
+// row) and, forward, those of the front's columns (lane = column).  Always
+// the same number of loads (a group or row past the end repeats the last
+// one), so that the next unit's stay in flight while this one is used.
+template <typename T>
+struct UnitLoad {
+  Quad<T> v[kUnitGroups<T>];
+  uint32_t r, c;
+};
+template <typename T>
+__device__ __forceinline__ void load_panel(UnitLoad<T>& b, const T* pan, const FrontUnit& d, int rc) {
+#pragma unroll
+  for (int q = 0; q < kUnitGroups<T>; q++) {
+    const int g = min(d.g0 + q, d.g1 - 1);
+    b.v[q].load(pan, d.h, g, max(rc, 4 * g));
+  }
+}
+
+// Forward and backward substitution for one subdomain per workgroup, in the
+// factor's precision T; the right-hand side is gathered from (and the solution
+// written to) FP64 vectors.  The work vector (positions, then update vectors
+// or the top fronts' solution) lives in LDS.  Nothing when *skip is set.
+// Forward: one front's panel times its right-hand side, a lane per row, the
+// columns' values broadcast from the lanes that gathered them.  Backward: the
+// panel's transpose times [y; -x], a lane per row, the columns' sums reduced
+// over the lanes at the end.
+// Each pass streams the panels once.  With hundreds of subdomains that is what
+// bounds it (512 of 5440 unknowns, FP64: 4.5 GB in 806 us, 5.6 TB/s; the
+// envelope factor's 12 GB took 1735 us); with few, the chain of fronts from a
+// leaf to the root does (9 of 2100 unknowns: 113 us, 310 us with envelopes).
+// Hence the unit lists: a wavefront's next panel rows are always on their way,
+// across barriers too, and the leaves' subtrees run side by side without any.
+template <typename T, int NW>
+__global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(4))) void k_front_solve(
+    const T* __restrict__ tiles, const FrontSub* __restrict__ subs, const int32_t* __restrict__ inds,
+    const double* __restrict__ rhs, double* __restrict__ sol, const double* skip) {
+  if (skip && *skip != 0.0) return;
+  constexpr int UG = kUnitGroups<T>;
+  extern __shared__ __align__(16) unsigned char front_dyn[];
+  T* L = reinterpret_cast<T*>(front_dyn);
+  const FrontSub s = subs[blockIdx.x];
+  const int t = threadIdx.x, lane = t & 63, w = __builtin_amdgcn_readfirstlane(t >> 6);
+  const T* base = tiles + s.base;
+  const int n = s.n, top0 = s.top0;
+  if (n == 0) return;
+  const Global<uint32_t> src = global(s.src);
+  const Global<uint16_t> rpos = global(s.rpos);
+  for (int p = t; p < n; p += 64 * NW) L[p] = (T)rhs[inds[s.vec + p]];
+  if (t == 0) L[n] = (T)0;
+  lds_barrier();
+  {
+    const UnitPtr units = unit_list(s.units_f);
+    int u0 = list_at(s.list_f, w);
+    const int last = list_at(s.list_f, w + 1) - 1;
+    T fv = (T)0, a[4] = {(T)0, (T)0, (T)0, (T)0};
+    // y of a front that several wavefronts share: its right-hand side is
+    // still read by the others, so it is written behind the next barrier
+    T pend = (T)0;
+    int pend_at = -1;
+    auto load = [&](UnitLoad<T>& b, const FrontUnit& d) {
+      const int rc = min(64 * d.chunk + lane, d.h - 1);
+      b.c = src[(uint32_t)(d.row0 + min(lane, d.h - 1))];
+      b.r = src[(uint32_t)(d.row0 + rc)];
+      load_panel(b, base + d.pan, d, rc);
+    };
+    auto work = [&](const UnitLoad<T>& b, const FrontUnit& d) {
+      {
+        const int row = 64 * d.chunk + lane, k = d.k;
+        if (d.flags & FU_FIRST) {
+          fv = (T)0;
+          if (lane < k) fv = L[d.c0 + lane] + (L[b.c & 0xffffu] + L[b.c >> 16]);
+        }
+        if (d.flags & FU_BEGIN) a[0] = a[1] = a[2] = a[3] = (T)0;
+#pragma unroll
+        for (int q = 0; q < UG; q++) {
+          const bool in = row >= 4 * (d.g0 + q);  // right of the diagonal there is nothing
+#pragma unroll
+          for (int j = 0; j < 4; j++)
+            a[j] = fused(in ? b.v[q].get(j) : (T)0, lane_value(fv, 4 * (d.g0 + q) + j), a[j]);
+        }
+        if (d.flags & FU_END) {
+          const T r = (a[0] + a[1]) + (a[2] + a[3]);
+          if (row < k) {
+            if (d.flags & FU_WHOLE) {
+              L[d.c0 + row] = r;
+            } else {
+              pend = r;
+              pend_at = d.c0 + row;
+            }
+          } else if (row < d.h) {
+            L[d.u + row - k] = (L[b.r & 0xffffu] + L[b.r >> 16]) - r;
+          }
+          wave_lds_sync();
+        }
+      }
+      for (int q = 0; q < d.nbar; q++) {
+        lds_barrier();
+        if (pend_at >= 0) L[pend_at] = pend;
+        pend_at = -1;
+      }
+    };
+    UnitLoad<T> b0, b1;
+    FrontUnit d0 = unit_at(units + u0);
+    load(b0, d0);
+    for (; u0 < last; u0 += 2) {  // two units a turn: lists have even lengths
+      const FrontUnit d1 = unit_at(units + u0 + 1);
+      load(b1, d1);
+      work(b0, d0);
+      d0 = unit_at(units + min(u0 + 2, last));
+      load(b0, d0);
+      work(b1, d1);
+    }
+  }
+  lds_barrier();
+  T* X = L + n - top0;  // solution at the positions from top0 on
+  {
+    const UnitPtr units = unit_list(s.units_b);
+    int u0 = list_at(s.list_b, w);
+    const int last = list_at(s.list_b, w + 1) - 1;
+    T y0 = (T)0, acc[4 * UG];
+#pragma unroll
+    for (int q = 0; q < 4 * UG; q++) acc[q] = (T)0;
+    auto load = [&](UnitLoad<T>& b, const FrontUnit& d) {
+      const int rc = min(64 * d.chunk + lane, d.h - 1);
+      b.r = rpos[(uint32_t)(d.row0 + rc)];
+      load_panel(b, base + d.pan, d, rc);
+    };
+    auto work = [&](const UnitLoad<T>& b, const FrontUnit& d) {
+      {
+        const int row = 64 * d.chunk + lane, k = d.k;
+        T x = y0;
+        if (d.chunk != 0 || (d.flags & FU_FIRST)) {
+          const int p = (int)b.r;
+          x = L[row >= k && p >= top0 ? n + p - top0 : p];
+          x = row < k ? x : row < d.h ? -x : (T)0;
+          if (d.chunk == 0) y0 = x;  // holds every y of the front (k <= 64)
+        }
+        if (d.flags & FU_BEGIN) {
+#pragma unroll
+          for (int q = 0; q < 4 * UG; q++) acc[q] = (T)0;
+        }
+#pragma unroll
+        for (int q = 0; q < UG; q++) {
+          const T xq = row >= 4 * (d.g0 + q) ? x : (T)0;
+#pragma unroll
+          for (int j = 0; j < 4; j++) acc[4 * q + j] = fused(b.v[q].get(j), xq, acc[4 * q + j]);
+        }
+        if (d.flags & FU_END) {
+          const T r = reduce_scatter<T, 4 * UG>(acc, lane);
+          constexpr int per = 64 / (4 * UG);
+          const int col = 4 * d.g0 + lane / per;
+          if (lane % per == 0 && col < k && col < 4 * d.g1) (d.c0 < top0 ? L : X)[d.c0 + col] = r;
+          wave_lds_sync();
+        }
+      }
+      for (int q = 0; q < d.nbar; q++) lds_barrier();
+    };
+    UnitLoad<T> b0, b1;
+    FrontUnit d0 = unit_at(units + u0);
+    load(b0, d0);
+    for (; u0 < last; u0 += 2) {  // two units a turn: lists have even lengths
+      const FrontUnit d1 = unit_at(units + u0 + 1);
+      load(b1, d1);
+      work(b0, d0);
+      d0 = unit_at(units + min(u0 + 2, last));
+      load(b0, d0);
+      work(b1, d1);
+    }
+  }
+  lds_barrier();
+  for (int p = t; p < n; p += 64 * NW) sol[s.vec + p] = (double)(p < top0 ? L[p] : X[p]);
+}
+
+}  // namespace
+
+template <typename T>
+void launch_front_scatter(T* tiles, const FrontSub* subs, int nsub, const int32_t* inds, const int32_t* occ_ptr,
+                          const int32_t* occ_pos, const int32_t* a_ptr, const int32_t* a_col, const double* a_val,
+                          hipStream_t st) {
+  if (nsub <= 0) return;
+  hipLaunchKernelGGL(k_front_scatter<T>, dim3(nsub, 4), dim3(256), 0, st, tiles, subs, inds, occ_ptr, occ_pos,
+                     a_ptr, a_col, a_val);
+}
+
+template <typename T>
+void launch_front_factor(T* tiles, T* schur, const FrontSub* subs, int nsub, int h, int maxcount, bool wide, int* flag,
+                         hipStream_t st) {
+  if (nsub <= 0 || maxcount <= 0) return;
+  const dim3 g(nsub, maxcount);
+  // One wavefront per small front where there are thousands: the pivot block
+  // is a chain that only one wavefront works on (512 subdomains of 5440
+  // unknowns, FP64: 11.7 ms in all, 13.2 ms with four wavefronts throughout).
+  // Sixteen per wide front where there are fewer than the GPU has room for at
+  // four (the same, 343 subdomains: 5.9 ms, 6.1 ms without).
+  const int64_t fronts = (int64_t)maxcount * nsub;
+  if (fronts > 4096)
+    hipLaunchKernelGGL((k_front_factor<T, 2, 1>), g, dim3(64), 0, st, tiles, schur, subs, h, flag);
+  else
+    hipLaunchKernelGGL((k_front_factor<T, 2, 4>), g, dim3(256), 0, st, tiles, schur, subs, h, flag);
+  if (wide && fronts > 512)
+    hipLaunchKernelGGL((k_front_factor<T, 4, 4>), g, dim3(256), 0, st, tiles, schur, subs, h, flag);
+  else if (wide)
+    hipLaunchKernelGGL((k_front_factor<T, 4, 16>), g, dim3(1024), 0, st, tiles, schur, subs, h, flag);
+}
+
+template <typename T>
+void prepare_front_solve(int maxwork) {
+  const int bytes = maxwork * (int)sizeof(T);
+  if (bytes > 64 * 1024) {
+    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&k_front_solve<T, 8>),
+                              hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
+    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&k_front_solve<T, 16>),
+                              hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
+  }
+}
+
+template <typename T>
+void launch_front_solve(const T* tiles, const FrontSub* subs, int nsub, int nw, int maxwork, const int32_t* inds,
+                        const double* r, double* sol, hipStream_t st, const double* skip) {
+  if (nsub <= 0) return;
+  const size_t lds = (size_t)maxwork * sizeof(T);
+  if (nw == 16)
+    hipLaunchKernelGGL((k_front_solve<T, 16>), dim3(nsub), dim3(1024), lds, st, tiles, subs, inds, r, sol, skip);
+  else
+    hipLaunchKernelGGL((k_front_solve<T, 8>), dim3(nsub), dim3(512), lds, st, tiles, subs, inds, r, sol, skip);
+}
+
+#define DOUG_INSTANTIATE_FRONTS(T)                                                                              \
+  template void launch_front_scatter<T>(T*, const FrontSub*, int, const int32_t*, const int32_t*,               \
+                                        const int32_t*, const int32_t*, const int32_t*, const double*,          \
+                                        hipStream_t);                                                           \
+  template void launch_front_factor<T>(T*, T*, const FrontSub*, int, int, int, bool, int*, hipStream_t);        \
+  template void prepare_front_solve<T>(int);                                                                    \
+  template void launch_front_solve<T>(const T*, const FrontSub*, int, int, int, const int32_t*, const double*,  \
+                                      double*, hipStream_t, const double*);
+DOUG_INSTANTIATE_FRONTS(double)
+DOUG_INSTANTIATE_FRONTS(float)
+#undef DOUG_INSTANTIATE_FRONTS
+
+}  // namespace doug

@@ -7,7 +7,7 @@
 // results are compared bit-for-bit with a sequential CPU loop (SpMV,
 // restriction, overlap sum, vector updates) keep products and sums as
 // separate roundings.
-#include "doug_kernels.hpp"
+#include "doug_tile.hpp"
 #include <algorithm>
 
 #pragma clang fp contract(off)
@@ -17,29 +17,6 @@ namespace doug {
 namespace {
 
 constexpr int LD = kTile + 1;  // padded LDS row stride (elements)
-
-// Matrix-core tile product for each element type.  Both forms take A[l%16][l/16]
-// and B[l/16][l%16] from lane l.  Result register r of lane l holds
-//   f64 16x16x4: D[l/16 + 4r][l%16]   (single-row groups strided by 4)
-//   f32 16x16x4: D[4(l/16) + r][l%16] (groups of four consecutive rows)
-template <typename T>
-struct Mma;
-template <>
-struct Mma<double> {
-  typedef double v4 __attribute__((ext_vector_type(4)));
-  static __device__ __forceinline__ v4 op(double a, double b, v4 c) {
-    return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
-  }
-  static __device__ __forceinline__ int row(int lane, int r) { return (lane >> 4) + 4 * r; }
-};
-template <>
-struct Mma<float> {
-  typedef float v4 __attribute__((ext_vector_type(4)));
-  static __device__ __forceinline__ v4 op(float a, float b, v4 c) {
-    return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
-  }
-  static __device__ __forceinline__ int row(int lane, int r) { return 4 * (lane >> 4) + r; }
-};
 
 // element offset of tile (i, k) from the block's base; k inside row i's envelope
 __device__ __forceinline__ int64_t toff(const BlockDesc& b, int i, int k) {
@@ -111,14 +88,6 @@ __device__ __forceinline__ void mma_ab(typename Mma<T>::v4 (&acc)[2][2], const T
     acc[1][0] = Mma<T>::op(a1, b0, acc[1][0]);
     acc[1][1] = Mma<T>::op(a1, b1, acc[1][1]);
   }
-}
-
-template <typename V>
-__device__ __forceinline__ void zero_acc(V (&acc)[2][2]) {
-#pragma unroll
-  for (int a = 0; a < 2; a++)
-#pragma unroll
-    for (int b = 0; b < 2; b++) acc[a][b] = V{0, 0, 0, 0};
 }
 
 // element (row, col) held by accumulator (bi, bj, r) of this lane
@@ -218,13 +187,6 @@ __device__ __forceinline__ void mma16_ab(typename Mma<T>::v4& acc, const T* a, i
   const int li = lane & 15, lk = lane >> 4;
 #pragma unroll
   for (int kk = 0; kk < 4; kk++) acc = Mma<T>::op(a[li * la + 4 * kk + lk], b[(4 * kk + lk) * lb + li], acc);
-}
-
-// orders this wavefront's LDS writes before its later LDS reads of them
-__device__ __forceinline__ void wave_lds_sync() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
 // one wavefront's staging: a 16x16 block (stride 17), then 16 reciprocals
@@ -2347,16 +2309,6 @@ DOUG_INSTANTIATE(float)
 // lists, ascending).  Row li of block b is unknown inds[s0 + li]; column c of
 // A is local column q - s0 for the occurrence q of c inside [s0, s0 + s),
 // found by scanning c's short list.  One workgroup per block.
-
-__device__ __forceinline__ int local_col(const int32_t* __restrict__ occ_ptr,
-                                         const int32_t* __restrict__ occ_pos, int c, int s0, int s) {
-  for (int k = occ_ptr[c]; k < occ_ptr[c + 1]; k++) {
-    const int q = occ_pos[k];
-    if (q >= s0 + s) break;
-    if (q >= s0) return q - s0;
-  }
-  return -1;
-}
 
 // First tile column of each tile row's envelope: min over the row's lower
 // entries of their tile column; `fc` holds the tile row index on entry.

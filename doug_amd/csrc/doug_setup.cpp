@@ -1251,7 +1251,7 @@ struct RankNode {
 struct RankScratch {
   int n = 0;
   std::vector<RankNode> nd;
-  std::vector<int> floc;  // -1 between uses (block_rcm_serial scratch)
+  std::vector<int> floc;  // -1 between uses (block_rcm scratch)
   int tick = 0;
   explicit RankScratch(int n_) : n(n_), nd((size_t)n_), floc((size_t)n_, -1) {}
 };
@@ -1277,14 +1277,6 @@ void block_rcm(const Csr& A, const std::vector<int>& starts, const std::vector<i
       for (int b = t; b < nb; b += nth) rcm_block(A, inds, starts[b], starts[b + 1] - starts[b], out, floc, buf);
     });
   for (auto& x : th) x.join();
-}
-
-void block_rcm_serial(const Csr& A, const std::vector<int>& starts, const std::vector<int>& inds,
-                      std::vector<int>& out, std::vector<int>& floc) {
-  out.assign(inds.begin(), inds.end());
-  RcmBuf buf;
-  for (int b = 0; b + 1 < (int)starts.size(); b++)
-    rcm_block(A, inds, starts[b], starts[b + 1] - starts[b], out, floc, buf);
 }
 
 // ---------------------------------------------------------------------------
@@ -1732,7 +1724,7 @@ void rank_local(const Csr& As, const std::vector<double>& val, const std::vector
 void virtual_ranks(const Csr& As, const std::vector<double>& val, const std::vector<int>& eptn,
                    int nranks, int ol_dist, int ol_sub,
                    int nsub_per_rank, int radius1, int minasize1, int maxasize1, double strong1,
-                   RankSetup& out, const Csr* rcm_graph, RankWorkspaces* ws, bool keep_local,
+                   RankSetup& out, RankWorkspaces* ws, bool keep_local,
                    const std::vector<int>* pos) {
   const int n = As.nrows;
   std::vector<std::vector<int>> own((size_t)nranks);
@@ -1747,7 +1739,7 @@ void virtual_ranks(const Csr& As, const std::vector<double>& val, const std::vec
   for (int r = 0; r < nranks; r++) out.own_off[r + 1] = out.own_off[r] + (int)own[r].size();
   out.order.resize((size_t)n);
   std::vector<Aggregates> inner((size_t)nranks), full((size_t)nranks);
-  std::vector<std::vector<int>> sst((size_t)nranks), sin((size_t)nranks), dsin((size_t)nranks);
+  std::vector<std::vector<int>> sst((size_t)nranks), sin((size_t)nranks);
   // own local indices in ascending global order, and the own nodes listed in
   // the inner and full aggregates of each rank
   std::vector<std::vector<int>> by_global((size_t)nranks);
@@ -1829,7 +1821,6 @@ void virtual_ranks(const Csr& As, const std::vector<double>& val, const std::vec
           if (pst[q + 1] > pst[q]) ps2.push_back(pst[q + 1]);
         add_layers_all(R.A, ps2, pnd, ol_sub, sst[r], sin[r]);
         for (int& v : sin[r]) v = R.lg[v];
-        if (rcm_graph) block_rcm_serial(*rcm_graph, sst[r], sin[r], dsin[r], S.floc);
         if (keep_local) {
           // the outer layer's rows are the last ones: A_ghost fills them
           const int first = R.A.nrows - R.nrecv;
@@ -1867,7 +1858,6 @@ void virtual_ranks(const Csr& As, const std::vector<double>& val, const std::vec
   }
   out.sstarts.assign((size_t)off_sub[nranks] + 1, 0);
   out.sinds.assign((size_t)off_ent[nranks], 0);
-  out.dinds.assign(rcm_graph ? (size_t)off_ent[nranks] : 0, 0);
   // first listed node of each rank in either list
   std::vector<int> node_off[2] = {std::vector<int>((size_t)nranks + 1, 0),
                                   std::vector<int>((size_t)nranks + 1, 0)};
@@ -1904,7 +1894,6 @@ void virtual_ranks(const Csr& As, const std::vector<double>& val, const std::vec
         }
         for (size_t q = 1; q < sst[r].size(); q++) out.sstarts[off_sub[r] + q] = off_ent[r] + sst[r][q];
         std::copy(sin[r].begin(), sin[r].end(), out.sinds.begin() + off_ent[r]);
-        if (rcm_graph) std::copy(dsin[r].begin(), dsin[r].end(), out.dinds.begin() + off_ent[r]);
       }
     });
   for (auto& x : th2) x.join();

@@ -118,10 +118,6 @@ void set_setup_thread_cap(int cap);
 struct RankWorkspaces;
 void block_rcm(const Csr& A, const std::vector<int>& starts, const std::vector<int>& inds,
                std::vector<int>& out, RankWorkspaces* ws = nullptr);
-// block_rcm on the calling thread with the caller's scratch `floc`
-// (A.nrows entries, all -1 on entry and on exit).
-void block_rcm_serial(const Csr& A, const std::vector<int>& starts, const std::vector<int>& inds,
-                      std::vector<int>& out, std::vector<int>& floc);
 
 // Project graph partitioner (stands in for METIS): recursive bisection of a
 // symmetric adjacency (0-based CSR, no self loops) into nparts parts of
@@ -170,7 +166,6 @@ struct RankSetup {
   std::vector<RankLocal> ranks;       // numbering only: each local matrix is released after use
   Aggregates inner, full;             // global numbering
   std::vector<int> sstarts, sinds;    // subdomains with their layers, global ids
-  std::vector<int> dinds;             // sinds, each subdomain in block_rcm order (if asked)
   // every rank's own nodes in its local order, rank after rank (own_off[r]
   // is rank r's first position): the process-major node order
   std::vector<int> order, own_off;
@@ -189,8 +184,7 @@ struct RankWorkspaces {
   void clear();
 };
 
-// With `rcm_graph`, each rank also orders its subdomains by block_rcm over
-// that graph (out.dinds), inside the rank's worker.  With `keep_local` every
+// With `keep_local` every
 // rank keeps its local matrix with A_ghost's rows and its own aggregates
 // (ranks_coarse_space's input); `pos` (optional) gives the position of each
 // of As's entries in the caller's matrix, recorded in RankLocal::A.src (As's
@@ -198,8 +192,8 @@ struct RankWorkspaces {
 void virtual_ranks(const Csr& As, const std::vector<double>& val, const std::vector<int>& eptn,
                    int nranks, int ol_dist, int ol_sub,
                    int nsub_per_rank, int radius1, int minasize1, int maxasize1, double strong1,
-                   RankSetup& out, const Csr* rcm_graph = nullptr, RankWorkspaces* ws = nullptr,
-                   bool keep_local = false, const std::vector<int>* pos = nullptr);
+                   RankSetup& out, RankWorkspaces* ws = nullptr, bool keep_local = false,
+                   const std::vector<int>* pos = nullptr);
 
 // The coarse space of a DOUG run on several processes
 // (CoarsePreconditioner_smooth_Init, CoarsePreconditioner_smooth.F90:47-89,

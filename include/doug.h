@@ -62,10 +62,10 @@ typedef struct {
   int32_t num_iters, reserved;
 } doug_params;
 
-/* Sizes and timings of the last doug_setup (seconds).  factor_bytes and
- * factor_tiles count the stored subdomain factor tiles (64x64, inside each
- * factor's envelope); factor_flops is the matrix-core work of their
- * factorisation. */
+/* Sizes and timings of the last doug_setup (seconds).  factor_bytes counts
+ * the stored subdomain factors (frontal panels, or the 64x64 tiles inside
+ * each factor's envelope) and factor_tiles the same in units of 4096 entries;
+ * factor_flops is the work of their factorisation. */
 typedef struct {
   int32_t n, nagr_fine, nagr_coarse, nsub, ncoarse, overlap, smoothers;
   int64_t nnz, sub_total, factor_bytes, coarse_factor_bytes;
@@ -74,7 +74,8 @@ typedef struct {
   int64_t factor_tiles;
   double factor_flops;
   /* device bytes the context keeps after the set-up for the next one (the
-   * coarse build's temporaries; 0 with DOUG_OPT_KEEP_SETUP_TEMPS 0) */
+   * coarse build's temporaries and the subdomain factorisation's update
+   * matrices; 0 with DOUG_OPT_KEEP_SETUP_TEMPS 0) */
   int64_t temp_bytes;
 } doug_info;
 
@@ -293,16 +294,18 @@ int doug_get_tuning(const doug_ctx *ctx, doug_tuning *out);
  * updates, SpMV, scalar read-back) from one captured HIP graph.
  * DOUG_OPT_SPMV_SHAPE (0..5) and DOUG_OPT_TRSV_ORDER (0/1) set what
  * doug_autotune would choose, see doug_tuning.  DOUG_OPT_LOCAL_ORDER
- * (default 1) places each subdomain's unknowns in its factor in reverse
- * Cuthill-McKee order, which narrows the stored tile envelope; 0 keeps the
- * index-set order.  It needs a new doug_setup and changes rounding only.
+ * (default 1) places each subdomain's unknowns in its factor in nested
+ * dissection order, for frontal factors, or, where a subdomain is too large
+ * for them, in reverse Cuthill-McKee order, which narrows the stored tile
+ * envelope; 0 keeps the index-set order (envelopes).  It needs a new
+ * doug_setup and changes rounding only.
  * DOUG_OPT_DEVICE_COARSE (default 1): build the smoothed restriction and the
  * Galerkin coarse matrix on the GPU (same bits as the host build, which 0
  * selects); applies to smoothers = 1 at the next doug_setup.
  * DOUG_OPT_BATCH_TILES (1 or 2, default 2): off-diagonal tiles the batched
  * envelope solve stages per step (what doug_autotune sets).
- * DOUG_OPT_DEVICE_BLOCKS (default 1): take the subdomain factors' tile
- * envelopes and entries on the GPU from the uploaded matrix (same tiles as
+ * DOUG_OPT_DEVICE_BLOCKS (default 1): take the subdomain factors' (tile
+ * envelopes and) entries on the GPU from the uploaded matrix (same tiles as
  * the host scatter map, which 0 selects; a matrix holding a duplicate
  * (i, j) pair always uses the host map); at the next doug_setup.
  * DOUG_OPT_KEEP_SETUP_TEMPS (default 1): keep the coarse build's device
@@ -336,9 +339,9 @@ int doug_set_option(doug_ctx *ctx, int32_t option, int64_t value);
 int doug_value_grad_device(doug_ctx *ctx, const double *dlam, const double *dx, double *dgrad);
 
 /* Several right-hand sides in one pass.  After doug_setup, doug_prepare_batch
- * allocates the multi-vector workspaces; the subdomain factors are the
- * single-column path's tile envelopes (L_i below the diagonal, inv(L_ii) on
- * it).  Each preconditioner apply is then one multi-vector restriction, two
+ * allocates the multi-vector workspaces and forms the subdomain factors in
+ * tile envelopes (L_i below the diagonal, inv(L_ii) on it) where the
+ * single-column path has frontal ones.  Each preconditioner apply is then one multi-vector restriction, two
  * chunked GEMMs on the coarse inverse factor, one launch of the batched
  * forward/backward envelope solve for every subdomain and all columns (tile x
  * panel products on the matrix cores, each factor tile read once per apply

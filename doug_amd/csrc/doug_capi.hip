@@ -1113,7 +1113,7 @@ static int build_fronts(doug_ctx* ctx, const Csr& M, const std::vector<int>& sta
     ctx->front_scratch = {q, sch_bytes};
   }
   T* d_schur = (T*)ctx->front_scratch.first;
-  HIPCHK(hipMemsetAsync(*d_tiles, 0, (size_t)base * sizeof(T), st));
+  HIPCHK(hipMemsetAsync(*d_tiles, 0, ((size_t)base) * sizeof(T), st));
   if (!host_map) {
     launch_front_scatter(*d_tiles, ctx->d_fsub, nb, ctx->lists.inds, ctx->lists.occ_ptr, ctx->lists.occ_pos, ctx->d_ptr,
                          ctx->d_col, ctx->d_val, st);
@@ -2102,8 +2102,8 @@ static int device_fine(doug_ctx* ctx, hipEvent_t ev0, hipEvent_t ev1) {
     // frontal factors: 2.7 times fewer entries than the envelopes on cubes of
     // 18^3 unknowns, 3.7 times on squares of 66^2; as long as the solve's work
     // vector fits a workgroup's LDS
-    const int64_t max_work = 160 * 1024 / (ctx->precision == DOUG_PREC_FP32_FACTORS ? 4 : 8) - 64;
     const bool f32 = ctx->precision == DOUG_PREC_FP32_FACTORS;
+    const int64_t max_work = 160 * 1024 / (f32 ? 4 : 8) - 64 - (f32 ? 0 : 64 * kFrontWavesMax);
     // eight wavefronts where two workgroups share a CU (512 subdomains, FP64:
     // 806 us, 852 us with sixteen), sixteen where there is a CU for each (9
     // subdomains: 113 us, 122 us with eight)
@@ -2112,7 +2112,8 @@ static int device_fine(doug_ctx* ctx, hipEvent_t ev0, hipEvent_t ev1) {
     bool sizes = true;
     for (size_t b = 0; b + 1 < ctx->sstarts.size(); b++)
       sizes = sizes && ctx->sstarts[b + 1] - ctx->sstarts[b] <= kMaxTrsvTiles * kTile;
-    ctx->fronts = sizes && build_front_patterns(A, ctx->sstarts, ctx->sinds, max_work, ctx->front_nw, f32 ? 8 : 4,
+    ctx->fronts = sizes && build_front_patterns(A, ctx->sstarts, ctx->sinds, max_work, ctx->front_nw,
+                                                f32 ? kFrontUnitGroups32 : kFrontUnitGroups64,
                                                 pats, pat, dinds);
     if (!ctx->fronts) block_rcm(A, ctx->sstarts, ctx->sinds, dinds, &ctx->rank_ws);
   } else {
@@ -2176,9 +2177,9 @@ static int device_fine(doug_ctx* ctx, hipEvent_t ev0, hipEvent_t ev1) {
   if ((rc = set_trsv_order(ctx, ctx->trsv_order))) return rc;
   if (ctx->fronts) {
     if (ctx->precision == DOUG_PREC_FP32_FACTORS)
-      prepare_front_solve<float>(ctx->maxwork);
+      prepare_front_solve<float>(ctx->front_nw, ctx->maxwork);
     else
-      prepare_front_solve<double>(ctx->maxwork);
+      prepare_front_solve<double>(ctx->front_nw, ctx->maxwork);
   }
   return DOUG_OK;
 }

@@ -38,10 +38,10 @@ void launch_front_factor(T* tiles, T* schur, const FrontSub* subs, int nsub, int
                          hipStream_t st);
 // Solve of every subdomain by nw wavefronts each: gathers r(inds), writes the solution to sol (FP64,
 // concatenated layout).  maxwork: the largest pattern's work vector; call
-// prepare_front_solve<T>(maxwork) once before.  skip (device, optional): the
+// prepare_front_solve<T>(nw, maxwork) once before.  skip (device, optional): the
 // launch does nothing when *skip != 0.
 template <typename T>
-void prepare_front_solve(int maxwork);
+void prepare_front_solve(int nw, int maxwork);
 template <typename T>
 void launch_front_solve(const T* tiles, const FrontSub* subs, int nsub, int nw, int maxwork, const int32_t* inds,
                         const double* r, double* sol, hipStream_t st, const double* skip = nullptr);

@@ -249,9 +249,11 @@ struct Space {
   }
 };
 
-// cost of a front in the solve: its elements and a fixed part for its chain
-// of loads (in elements that stream meanwhile)
-int64_t front_cost(const Front& f) { return front_panel_elems(f.k, f.m) + 1500; }
+// cost of a front in the solve: its units (a unit costs what its loads do,
+// filled or not)
+int64_t front_cost(const Front& f, int ug) {
+  return (int64_t)((f.k + f.m + 63) / 64) * std::max(1, (f.k + 4 * ug - 1) / (4 * ug));
+}
 
 // A share of a front: 64-row chunks (forward) or column groups (backward).
 struct Item {
@@ -391,7 +393,7 @@ bool make_pattern(const Graph& g, int64_t max_work, int nw, int ug, FrontPattern
   // wavefronts; what is above them goes level by level
   std::vector<int64_t> cost((size_t)nf);
   for (int f = 0; f < nf; f++) {
-    cost[f] = front_cost(F[f]);
+    cost[f] = front_cost(F[f], ug);
     for (int c : F[f].child)
       if (c >= 0) cost[f] += cost[c];
   }
@@ -413,7 +415,7 @@ bool make_pattern(const Graph& g, int64_t max_work, int nw, int ug, FrontPattern
       sum += cost[f];
     }
     const int64_t worst = *std::max_element(load, load + nw);
-    if (roots.empty() || (5 * nw * worst <= 6 * sum) || (int)roots.size() >= 6 * nw) break;
+    if (roots.empty() || 10 * nw * worst <= 11 * sum || (int)roots.size() >= 6 * nw) break;
     const int f = roots.front();
     if (F[f].child[0] < 0 && F[f].child[1] < 0) break;  // a leaf is the heaviest
     top[f] = 1;
@@ -583,7 +585,7 @@ bool make_pattern(const Graph& g, int64_t max_work, int nw, int ug, FrontPattern
     std::vector<int> byw;
     for (int f = q; f < e; f++) byw.push_back(f);
     std::sort(byw.begin(), byw.end(), [&](int a, int b) {
-      const int64_t x = front_cost(F[a]), y = front_cost(F[b]);
+      const int64_t x = front_cost(F[a], ug), y = front_cost(F[b], ug);
       return x != y ? x > y : a < b;
     });
     fw.at(pf, 0);
@@ -594,7 +596,7 @@ bool make_pattern(const Graph& g, int64_t max_work, int nw, int ug, FrontPattern
         int w = 0;
         for (int x = 1; x < nw; x++)
           if (load[x] < load[w]) w = x;
-        load[w] += front_cost(F[f]);
+        load[w] += front_cost(F[f], ug);
         put(fw, pf, w, f, 0, rows_of(f));
         put(bw, pb, w, f, 0, (F[f].k + 3) / 4);
       }

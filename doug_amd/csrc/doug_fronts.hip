@@ -28,36 +28,6 @@ __device__ __forceinline__ int panel_elem(int H, int row, int col) {
   return base + (j >> 1) * 2 * (H - 4 * g) + 2 * (row - 4 * g) + (j & 1);
 }
 
-// The four entries of column group g in one row: the panel is streamed once
-// per pass, so its loads are non-temporal.
-template <typename T>
-struct Quad;
-template <>
-struct Quad<float> {
-  typedef float v4 __attribute__((ext_vector_type(4)));
-  v4 a;
-  __device__ __forceinline__ void load(const float* pan, int H, int g, int row) {
-    // 32-bit offsets from a uniform base keep the addresses in one register
-    const uint32_t o = 16u * (uint32_t)(row + g * (H - 2 * g - 2));
-    a = __builtin_nontemporal_load(reinterpret_cast<const v4*>(reinterpret_cast<const char*>(pan) + o));
-  }
-  __device__ __forceinline__ float get(int j) const { return a[j]; }
-  __device__ __forceinline__ void zero() { a = v4{0, 0, 0, 0}; }
-};
-template <>
-struct Quad<double> {
-  typedef double v2 __attribute__((ext_vector_type(2)));
-  v2 a, b;
-  __device__ __forceinline__ void load(const double* pan, int H, int g, int row) {
-    const uint32_t o = 16u * (uint32_t)(2 * g * H - 4 * g * (g - 1) + row - 4 * g);
-    a = __builtin_nontemporal_load(reinterpret_cast<const v2*>(reinterpret_cast<const char*>(pan) + o));
-    b = __builtin_nontemporal_load(
-        reinterpret_cast<const v2*>(reinterpret_cast<const char*>(pan) + (o + 16u * (uint32_t)(H - 4 * g))));
-  }
-  __device__ __forceinline__ double get(int j) const { return j < 2 ? a[j & 1] : b[j & 1]; }
-  __device__ __forceinline__ void zero() { a = v2{0, 0}; b = v2{0, 0}; }
-};
-
 __device__ __forceinline__ float lane_value(float v, int l) {
   return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), l));
 }
@@ -476,9 +446,6 @@ __global__ __launch_bounds__(64 * NW) void k_front_factor(T* tiles, T* schur, co
 // solve, one right-hand side
 // ------------------------------------------------------------------------
 
-__device__ __forceinline__ float fused(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
-__device__ __forceinline__ double fused(double a, double b, double c) { return __builtin_fma(a, b, c); }
-
 // A lane's 32-bit value as another lane of its row of 16 sees it (DPP).
 template <int CTRL>
 __device__ __forceinline__ float lane_swap(float v) {
@@ -492,6 +459,7 @@ __device__ __forceinline__ double lane_swap(double v) {
 }
 constexpr int kDppXor1 = 0xB1, kDppXor2 = 0x4E;        // quad_perm
 constexpr int kDppXor8 = 0x128, kDppXor7 = 0x141;      // row_ror:8, row_half_mirror
+constexpr int kDppRor4 = 0x124;                        // row_ror:4
 
 // a + b after half the lanes have exchanged them: lanes of the lower half
 // (of each 64, or of each 32) return a's sum over the two halves, the others b's.
@@ -503,39 +471,25 @@ __device__ __forceinline__ float fold16(float a, float b) {
   const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(a), __float_as_uint(b), false, false);
   return __uint_as_float(r[0]) + __uint_as_float(r[1]);
 }
-__device__ __forceinline__ double fold32(double a, double b) {
-  const auto l = __builtin_amdgcn_permlane32_swap(__double2loint(a), __double2loint(b), false, false);
-  const auto h = __builtin_amdgcn_permlane32_swap(__double2hiint(a), __double2hiint(b), false, false);
-  return __hiloint2double(h[0], l[0]) + __hiloint2double(h[1], l[1]);
-}
-__device__ __forceinline__ double fold16(double a, double b) {
-  const auto l = __builtin_amdgcn_permlane16_swap(__double2loint(a), __double2loint(b), false, false);
-  const auto h = __builtin_amdgcn_permlane16_swap(__double2hiint(a), __double2hiint(b), false, false);
-  return __hiloint2double(h[0], l[0]) + __hiloint2double(h[1], l[1]);
-}
-template <int CTRL, typename T>
-__device__ __forceinline__ T fold_row(T a, T b, bool hi) {
-  const T keep = hi ? b : a, send = hi ? a : b;
+template <int CTRL>
+__device__ __forceinline__ float fold_row(float a, float b, bool hi) {
+  const float keep = hi ? b : a, send = hi ? a : b;
   return keep + lane_swap<CTRL>(send);
 }
 
-// v[0..N-1] (N = 16 or 32) summed over the 64 lanes: lane l returns the sum
-// of entry l / (64 / N).  Each halving hands one half of the entries to the
-// other half of the lanes; all exchanges are register-to-register.
-template <typename T, int N>
-__device__ __forceinline__ T reduce_scatter(T (&v)[N], int lane) {
+// v[0..31] summed over the 64 lanes: lane l returns the sum of entry l / 2.
+// Each halving hands one half of the entries to the other half of the lanes;
+// all exchanges are register-to-register.
+__device__ __forceinline__ float reduce_scatter(float (&v)[32], int lane) {
 #pragma unroll
-  for (int q = 0; q < N / 2; q++) v[q] = fold32(v[q], v[q + N / 2]);
+  for (int q = 0; q < 16; q++) v[q] = fold32(v[q], v[q + 16]);
 #pragma unroll
-  for (int q = 0; q < N / 4; q++) v[q] = fold16(v[q], v[q + N / 4]);
+  for (int q = 0; q < 8; q++) v[q] = fold16(v[q], v[q + 8]);
 #pragma unroll
-  for (int q = 0; q < N / 8; q++) v[q] = fold_row<kDppXor8>(v[q], v[q + N / 8], lane & 8);
+  for (int q = 0; q < 4; q++) v[q] = fold_row<kDppXor8>(v[q], v[q + 4], lane & 8);
 #pragma unroll
-  for (int q = 0; q < N / 16; q++) v[q] = fold_row<kDppXor7>(v[q], v[q + N / 16], lane & 4);
-  if (N == 32)
-    v[0] = fold_row<kDppXor2>(v[0], v[1 % N], lane & 2);
-  else
-    v[0] = v[0] + lane_swap<kDppXor2>(v[0]);
+  for (int q = 0; q < 2; q++) v[q] = fold_row<kDppXor7>(v[q], v[q + 2], lane & 4);
+  v[0] = fold_row<kDppXor2>(v[0], v[1], lane & 2);
   return v[0] + lane_swap<kDppXor1>(v[0]);
 }
 
@@ -577,48 +531,50 @@ __device__ __forceinline__ FrontUnit unit_at(UnitPtr p) {
   return u;
 }
 
-// column groups per unit: 64 rows of them are 8 KB in either precision
-template <typename T>
-constexpr int kUnitGroups = sizeof(T) == 4 ? 8 : 4;
+// The four entries of column group g in one row: the panel is streamed once
+// per pass, so its loads are non-temporal.
+typedef float F4 __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ F4 load_quad(const float* pan, int H, int g, int row) {
+  // 32-bit offsets from a uniform base keep the addresses in one register
+  const uint32_t o = 16u * (uint32_t)(row + g * (H - 2 * g - 2));
+  return __builtin_nontemporal_load(reinterpret_cast<const F4*>(reinterpret_cast<const char*>(pan) + o));
+}
 
 // The loads of one unit: its panel rows, the row records of its rows (lane =
 // row) and, forward, those of the front's columns (lane = column).  Always
 // the same number of loads (a group or row past the end repeats the last
 // one), so that the next unit's stay in flight while this one is used.
-template <typename T>
 struct UnitLoad {
-  Quad<T> v[kUnitGroups<T>];
+  F4 v[kFrontUnitGroups32];
   uint32_t r, c;
 };
-template <typename T>
-__device__ __forceinline__ void load_panel(UnitLoad<T>& b, const T* pan, const FrontUnit& d, int rc) {
+__device__ __forceinline__ void load_panel(UnitLoad& b, const float* pan, const FrontUnit& d, int rc) {
 #pragma unroll
-  for (int q = 0; q < kUnitGroups<T>; q++) {
+  for (int q = 0; q < kFrontUnitGroups32; q++) {
     const int g = min(d.g0 + q, d.g1 - 1);
-    b.v[q].load(pan, d.h, g, max(rc, 4 * g));
+    b.v[q] = load_quad(pan, d.h, g, max(rc, 4 * g));
   }
 }
 
-// Forward and backward substitution for one subdomain per workgroup, in the
-// factor's precision T; the right-hand side is gathered from (and the solution
+// Forward and backward substitution for one subdomain per workgroup, in FP32; the right-hand side is gathered from (and the solution
 // written to) FP64 vectors.  The work vector (positions, then update vectors
 // or the top fronts' solution) lives in LDS.  Nothing when *skip is set.
 // Forward: one front's panel times its right-hand side, a lane per row, the
 // columns' values broadcast from the lanes that gathered them.  Backward: the
 // panel's transpose times [y; -x], a lane per row, the columns' sums reduced
 // over the lanes at the end.
-// Each pass streams the panels once.  With hundreds of subdomains that is what
-// bounds it (512 of 5440 unknowns, FP64: 4.5 GB in 806 us, 5.6 TB/s; the
-// envelope factor's 12 GB took 1735 us); with few, the chain of fronts from a
-// leaf to the root does (9 of 2100 unknowns: 113 us, 310 us with envelopes).
-// Hence the unit lists: a wavefront's next panel rows are always on their way,
-// across barriers too, and the leaves' subtrees run side by side without any.
-template <typename T, int NW>
+// Each pass streams the panels once, which bounds it where there are hundreds
+// of subdomains (512 of 5440 unknowns: 2.2 GB in 493 us, 4.5 TB/s; envelopes,
+// 6 GB in 879 us).  Hence the unit lists: a wavefront's next panel rows are
+// always on their way, across barriers too, and the leaves' subtrees run side
+// by side without any.
+template <int NW>
 __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(4))) void k_front_solve(
-    const T* __restrict__ tiles, const FrontSub* __restrict__ subs, const int32_t* __restrict__ inds,
+    const float* __restrict__ tiles, const FrontSub* __restrict__ subs, const int32_t* __restrict__ inds,
     const double* __restrict__ rhs, double* __restrict__ sol, const double* skip) {
   if (skip && *skip != 0.0) return;
-  constexpr int UG = kUnitGroups<T>;
+  typedef float T;
+  constexpr int UG = kFrontUnitGroups32;
   extern __shared__ __align__(16) unsigned char front_dyn[];
   T* L = reinterpret_cast<T*>(front_dyn);
   const FrontSub s = subs[blockIdx.x];
@@ -640,13 +596,13 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(4))) vo
     // still read by the others, so it is written behind the next barrier
     T pend = (T)0;
     int pend_at = -1;
-    auto load = [&](UnitLoad<T>& b, const FrontUnit& d) {
+    auto load = [&](UnitLoad& b, const FrontUnit& d) {
       const int rc = min(64 * d.chunk + lane, d.h - 1);
       b.c = src[(uint32_t)(d.row0 + min(lane, d.h - 1))];
       b.r = src[(uint32_t)(d.row0 + rc)];
       load_panel(b, base + d.pan, d, rc);
     };
-    auto work = [&](const UnitLoad<T>& b, const FrontUnit& d) {
+    auto work = [&](const UnitLoad& b, const FrontUnit& d) {
       {
         const int row = 64 * d.chunk + lane, k = d.k;
         if (d.flags & FU_FIRST) {
@@ -659,7 +615,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(4))) vo
           const bool in = row >= 4 * (d.g0 + q);  // right of the diagonal there is nothing
 #pragma unroll
           for (int j = 0; j < 4; j++)
-            a[j] = fused(in ? b.v[q].get(j) : (T)0, lane_value(fv, 4 * (d.g0 + q) + j), a[j]);
+            a[j] = __builtin_fmaf(in ? b.v[q][j] : (T)0, lane_value(fv, 4 * (d.g0 + q) + j), a[j]);
         }
         if (d.flags & FU_END) {
           const T r = (a[0] + a[1]) + (a[2] + a[3]);
@@ -682,7 +638,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(4))) vo
         pend_at = -1;
       }
     };
-    UnitLoad<T> b0, b1;
+    UnitLoad b0, b1;
     FrontUnit d0 = unit_at(units + u0);
     load(b0, d0);
     for (; u0 < last; u0 += 2) {  // two units a turn: lists have even lengths
@@ -703,12 +659,12 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(4))) vo
     T y0 = (T)0, acc[4 * UG];
 #pragma unroll
     for (int q = 0; q < 4 * UG; q++) acc[q] = (T)0;
-    auto load = [&](UnitLoad<T>& b, const FrontUnit& d) {
+    auto load = [&](UnitLoad& b, const FrontUnit& d) {
       const int rc = min(64 * d.chunk + lane, d.h - 1);
       b.r = rpos[(uint32_t)(d.row0 + rc)];
       load_panel(b, base + d.pan, d, rc);
     };
-    auto work = [&](const UnitLoad<T>& b, const FrontUnit& d) {
+    auto work = [&](const UnitLoad& b, const FrontUnit& d) {
       {
         const int row = 64 * d.chunk + lane, k = d.k;
         T x = y0;
@@ -726,10 +682,10 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(4))) vo
         for (int q = 0; q < UG; q++) {
           const T xq = row >= 4 * (d.g0 + q) ? x : (T)0;
 #pragma unroll
-          for (int j = 0; j < 4; j++) acc[4 * q + j] = fused(b.v[q].get(j), xq, acc[4 * q + j]);
+          for (int j = 0; j < 4; j++) acc[4 * q + j] = __builtin_fmaf(b.v[q][j], xq, acc[4 * q + j]);
         }
         if (d.flags & FU_END) {
-          const T r = reduce_scatter<T, 4 * UG>(acc, lane);
+          const T r = reduce_scatter(acc, lane);
           constexpr int per = 64 / (4 * UG);
           const int col = 4 * d.g0 + lane / per;
           if (lane % per == 0 && col < k && col < 4 * d.g1) (d.c0 < top0 ? L : X)[d.c0 + col] = r;
@@ -738,7 +694,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(4))) vo
       }
       for (int q = 0; q < d.nbar; q++) lds_barrier();
     };
-    UnitLoad<T> b0, b1;
+    UnitLoad b0, b1;
     FrontUnit d0 = unit_at(units + u0);
     load(b0, d0);
     for (; u0 < last; u0 += 2) {  // two units a turn: lists have even lengths
@@ -752,6 +708,274 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(4))) vo
   }
   lds_barrier();
   for (int p = t; p < n; p += 64 * NW) sol[s.vec + p] = (double)(p < top0 ? L[p] : X[p]);
+}
+
+// ---- FP64: the same on the matrix cores ----
+//
+// v_mfma_f64_4x4x4 takes A[i][k] of block b from lane i + 4 b + 16 k, B[k][j]
+// from lane j + 4 b + 16 k, and holds D[i][j] in lane j + 4 b + 16 i.  One
+// column of B is enough here; all four are the same.
+__device__ __forceinline__ double mma4(double a, double b, double c) {
+  return __builtin_amdgcn_mfma_f64_4x4x4f64(a, b, c, 0, 0, 0);
+}
+__device__ __forceinline__ double pick4(const double (&v)[4], int i) {
+  const double a = (i & 1) ? v[1] : v[0], b = (i & 1) ? v[3] : v[2];
+  return (i & 2) ? b : a;
+}
+
+// A unit's descriptor on its way through the vector path: fetched ahead of the
+// loads that the units before it issue, it is there when they still are not.
+struct RawUnit {
+  uint32_t a __attribute__((ext_vector_type(4)));
+  uint32_t b __attribute__((ext_vector_type(2)));
+};
+__device__ __forceinline__ RawUnit raw_unit(const FrontUnit* p, int i) {
+  typedef uint32_t v4 __attribute__((ext_vector_type(4)));
+  typedef uint32_t v2 __attribute__((ext_vector_type(2)));
+  const Global<v4> q = global(reinterpret_cast<const v4*>(p));
+  RawUnit r;
+  r.a = q[(uint32_t)(2 * i)];
+  r.b = *(const v2 __attribute__((address_space(1)))*)(q + (uint32_t)(2 * i + 1));
+  return r;
+}
+__device__ __forceinline__ FrontUnit unit_of(const RawUnit& r) {
+  const uint32_t a2 = uniform(r.a[2]), a3 = uniform(r.a[3]), b0 = uniform(r.b[0]);
+  FrontUnit u;
+  u.pan = uniform(r.a[0]);
+  u.row0 = uniform(r.a[1]);
+  u.h = (uint16_t)a2;
+  u.k = (uint16_t)(a2 >> 16);
+  u.c0 = (uint16_t)a3;
+  u.u = (uint16_t)(a3 >> 16);
+  u.g0 = (uint8_t)b0;
+  u.g1 = (uint8_t)(b0 >> 8);
+  u.chunk = (uint8_t)(b0 >> 16);
+  u.flags = (uint8_t)(b0 >> 24);
+  u.nbar = (uint16_t)uniform(r.b[1]);
+  return u;
+}
+
+// The units of one wavefront, two a turn (lists have even lengths): the loads
+// of the unit after next are issued as soon as a unit's registers are free,
+// before its barriers.
+template <typename Load, typename F, typename G, typename H>
+__device__ __forceinline__ void walk_units(const FrontUnit* units, int u, int end, F&& load, G&& work, H&& barriers) {
+  Load q0, q1;
+  RawUnit r0 = raw_unit(units, u), r1 = raw_unit(units, u + 1);
+  FrontUnit d0 = unit_of(r0), d1 = unit_of(r1);
+  r0 = raw_unit(units, min(u + 2, end - 1));
+  load(q0, d0);
+  __builtin_amdgcn_sched_barrier(0);
+  r1 = raw_unit(units, min(u + 3, end - 1));
+  load(q1, d1);
+  __builtin_amdgcn_sched_barrier(0);
+  for (; u < end; u += 2) {
+    work(q0, d0);
+    int n = d0.nbar;
+    d0 = unit_of(r0);
+    r0 = raw_unit(units, min(u + 4, end - 1));
+    load(q0, d0);
+    __builtin_amdgcn_sched_barrier(0);
+    barriers(n);
+    work(q1, d1);
+    n = d1.nbar;
+    d1 = unit_of(r1);
+    r1 = raw_unit(units, min(u + 5, end - 1));
+    load(q1, d1);
+    __builtin_amdgcn_sched_barrier(0);
+    barriers(n);
+  }
+}
+
+// Byte offset in an FP64 panel of H rows of the columns 4 g + 2 j, 4 g + 2 j + 1
+// of a row.
+__device__ __forceinline__ uint32_t panel_offset(int H, int g, int j, int row) {
+  return 16u * (uint32_t)(2 * g * H - 4 * g * (g - 1) + row - 4 * g + (j ? H - 4 * g : 0));
+}
+typedef double Two __attribute__((ext_vector_type(2)));
+// Buffer loads of a panel: an offset past its end gives zeros and loads nothing.
+typedef uint32_t U4 __attribute__((ext_vector_type(4)));
+constexpr uint32_t kNothing = 0x80000000u;
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t panel_buffer(const double* p, int bytes) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<double*>(p), 0, bytes, 0x00027000);
+}
+__device__ __forceinline__ Two panel_load(__amdgpu_buffer_rsrc_t b, uint32_t offset) {
+  const U4 v = __builtin_amdgcn_raw_buffer_load_b128(b, (int)offset, 0, 0);
+  return __builtin_bit_cast(Two, v);
+}
+
+// Bytes of a panel's first g1 column groups.
+__device__ __forceinline__ int panel_bytes(int H, int g1) { return 32 * (g1 * H - 2 * g1 * (g1 - 1)); }
+
+// A product step takes 16 rows of four columns, so that a unit of 64 rows and
+// 16 columns is 16 of them, with neither broadcasts (forward) nor sums over
+// lanes (backward): in the vector form above these cost more than the
+// products.  A 16-byte load gives a lane two columns of a row, one for each of
+// two steps: forward of row l % 16 the pair l / 16 of eight columns, backward
+// of row 4 (l / 4 % 4) + l / 16 the pair l % 4.  The operands that all rows
+// (columns) share go through 64 entries of LDS per wavefront behind the work
+// vector.  Lanes outside the front, or right of its diagonal, load nothing and
+// get zeros: what bounds the kernel where subdomains are few is the 64 bytes a
+// cycle that a CU loads, and half of a unit is such lanes on average.
+// 512 subdomains of 5440 unknowns: 805 us, 5.6 TB/s (the vector form 804,
+// envelopes 1735); 343 of 4600: 395 us (414, 950); 64 of 4300 in two
+// dimensions: 171 us (188, 709); 9 of 2100: 110 us (113, 310).
+template <int NW>
+__global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(4))) void k_front_solve_mma(
+    const double* __restrict__ tiles, const FrontSub* __restrict__ subs, int maxwork,
+    const int32_t* __restrict__ inds, const double* __restrict__ rhs, double* __restrict__ sol, const double* skip) {
+  if (skip && *skip != 0.0) return;
+  constexpr int UG = kFrontUnitGroups64;
+  extern __shared__ __align__(16) unsigned char front_dyn[];
+  double* L = reinterpret_cast<double*>(front_dyn);
+  const FrontSub s = subs[blockIdx.x];
+  const int t = threadIdx.x, lane = t & 63, w = __builtin_amdgcn_readfirstlane(t >> 6);
+  const int lo = lane & 3, mid = (lane >> 2) & 3, hi = lane >> 4;
+  double* stage = L + maxwork + 64 * w;
+  const double* base = tiles + s.base;
+  const int n = s.n, top0 = s.top0;
+  if (n == 0) return;
+  const Global<uint32_t> src = global(s.src);
+  const Global<uint16_t> rpos = global(s.rpos);
+  for (int p = t; p < n; p += 64 * NW) L[p] = rhs[inds[s.vec + p]];
+  if (t == 0) L[n] = 0.0;
+  lds_barrier();
+  struct Load {
+    Two a[UG / 2][4];
+    uint32_t r, c;
+  };
+  {
+    // y of a front that several wavefronts share: its right-hand side is
+    // still read by the others, so it is written behind the next barrier
+    double acc[4] = {0.0, 0.0, 0.0, 0.0}, pend = 0.0;
+    int pend_at = -1;
+    const int mine = 16 * lo + 4 * mid + hi;  // the row of a chunk whose sum this lane ends with
+    auto load = [&](Load& q, const FrontUnit& d) {
+      const auto pan = panel_buffer(base + d.pan, panel_bytes(d.h, d.g1));
+#pragma unroll
+      for (int x = 0; x < UG / 2; x++) {
+        const int g = d.g0 + 2 * x + (hi >> 1), row = 64 * d.chunk + (lane & 15);
+        const uint32_t o = panel_offset(d.h, g, hi & 1, row);
+        const int first = g < d.g1 ? 4 * g : d.h;
+#pragma unroll
+        for (int y = 0; y < 4; y++)
+          q.a[x][y] = panel_load(pan, row + 16 * y >= first && row + 16 * y < d.h ? o + 256u * y : kNothing);
+      }
+      q.c = src[(uint32_t)(d.row0 + min(lane, d.h - 1))];
+      q.r = src[(uint32_t)(d.row0 + min(64 * d.chunk + mine, d.h - 1))];
+    };
+    auto work = [&](const Load& q, const FrontUnit& d) {
+      const int k = d.k;
+      if (d.flags & FU_FIRST) {
+        double f = 0.0;
+        if (lane < k) f = L[d.c0 + lane] + (L[q.c & 0xffffu] + L[q.c >> 16]);
+        stage[lane] = f;
+        wave_lds_sync();
+      }
+      if (d.flags & FU_BEGIN) acc[0] = acc[1] = acc[2] = acc[3] = 0.0;
+      const int left = d.h - 64 * d.chunk;
+#pragma unroll
+      for (int x = 0; x < UG / 2; x++)
+        if (x == 0 || d.g0 + 2 * x < d.g1) {
+          const int g = d.g0 + 2 * x + (hi >> 1);  // past g1 there are zeros in `stage`
+          const Two f = *reinterpret_cast<const Two*>(stage + 4 * g + 2 * (hi & 1));
+#pragma unroll
+          for (int y = 0; y < 4; y++)
+            if (y == 0 || 16 * y < left) {
+              const Two a = q.a[x][y];
+              acc[y] = mma4(a[0], f[0], acc[y]);
+              acc[y] = mma4(a[1], f[1], acc[y]);
+            }
+        }
+      if (d.flags & FU_END) {
+        const int row = 64 * d.chunk + mine;
+        const double r = pick4(acc, lo);
+        if (row < k) {
+          if (d.flags & FU_WHOLE) {
+            L[d.c0 + row] = r;
+          } else {
+            pend = r;
+            pend_at = d.c0 + row;
+          }
+        } else if (row < d.h) {
+          L[d.u + row - k] = (L[q.r & 0xffffu] + L[q.r >> 16]) - r;
+        }
+        wave_lds_sync();
+      }
+    };
+    auto barriers = [&](int count) {
+      for (int i = 0; i < count; i++) {
+        lds_barrier();
+        if (pend_at >= 0) L[pend_at] = pend;
+        pend_at = -1;
+      }
+    };
+    walk_units<Load>(s.units_f, list_at(s.list_f, w), list_at(s.list_f, w + 1), load, work, barriers);
+  }
+  lds_barrier();
+  double* X = L + n - top0;  // solution at the positions from top0 on
+  {
+    double acc[UG] = {0.0, 0.0, 0.0, 0.0}, y0 = 0.0;
+    auto load = [&](Load& q, const FrontUnit& d) {
+      const auto pan = panel_buffer(base + d.pan, panel_bytes(d.h, d.g1));
+#pragma unroll
+      for (int x = 0; x < UG / 2; x++) {
+        const int g = d.g0 + 2 * x + (lo >> 1), row = 64 * d.chunk + 4 * mid + hi;
+        const uint32_t o = panel_offset(d.h, g, lo & 1, row);
+        const int first = g < d.g1 ? 4 * g : d.h;
+#pragma unroll
+        for (int y = 0; y < 4; y++)
+          q.a[x][y] = panel_load(pan, row + 16 * y >= first && row + 16 * y < d.h ? o + 256u * y : kNothing);
+      }
+      q.r = rpos[(uint32_t)(d.row0 + min(64 * d.chunk + lane, d.h - 1))];
+    };
+    auto work = [&](const Load& q, const FrontUnit& d) {
+      const int k = d.k;
+      {
+        const int row = 64 * d.chunk + lane;
+        double x = y0;
+        if (d.chunk != 0 || (d.flags & FU_FIRST)) {
+          const int p = (int)q.r;
+          x = L[row >= k && p >= top0 ? n + p - top0 : p];
+          x = row < k ? x : row < d.h ? -x : 0.0;
+          if (d.chunk == 0) y0 = x;  // holds every y of the front (k <= 64)
+        }
+        stage[lane] = x;
+        wave_lds_sync();
+      }
+      if (d.flags & FU_BEGIN) {
+#pragma unroll
+        for (int x = 0; x < UG; x++) acc[x] = 0.0;
+      }
+      const int left = d.h - 64 * d.chunk;
+#pragma unroll
+      for (int y = 0; y < 4; y++)
+        if (y == 0 || 16 * y < left) {
+          const double v = stage[16 * y + 4 * mid + hi];
+#pragma unroll
+          for (int x = 0; x < UG / 2; x++) {
+            const Two a = q.a[x][y];
+            acc[2 * x] = mma4(a[0], v, acc[2 * x]);
+            acc[2 * x + 1] = mma4(a[1], v, acc[2 * x + 1]);
+          }
+        }
+      wave_lds_sync();
+      if (d.flags & FU_END) {
+        double r = pick4(acc, lo);
+        r += lane_swap<kDppXor8>(r);
+        r += lane_swap<kDppRor4>(r);
+        const int col = 4 * d.g0 + 8 * (lo >> 1) + 2 * hi + (lo & 1);
+        if (mid == 0 && col < k && col < 4 * d.g1) (d.c0 < top0 ? L : X)[d.c0 + col] = r;
+        wave_lds_sync();
+      }
+    };
+    auto barriers = [&](int count) {
+      for (int i = 0; i < count; i++) lds_barrier();
+    };
+    walk_units<Load>(s.units_b, list_at(s.list_b, w), list_at(s.list_b, w + 1), load, work, barriers);
+  }
+  lds_barrier();
+  for (int p = t; p < n; p += 64 * NW) sol[s.vec + p] = p < top0 ? L[p] : X[p];
 }
 
 }  // namespace
@@ -786,26 +1010,43 @@ void launch_front_factor(T* tiles, T* schur, const FrontSub* subs, int nsub, int
     hipLaunchKernelGGL((k_front_factor<T, 4, 16>), g, dim3(1024), 0, st, tiles, schur, subs, h, flag);
 }
 
+// LDS of a solve by nw wavefronts
 template <typename T>
-void prepare_front_solve(int maxwork) {
-  const int bytes = maxwork * (int)sizeof(T);
-  if (bytes > 64 * 1024) {
-    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&k_front_solve<T, 8>),
-                              hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
-    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&k_front_solve<T, 16>),
-                              hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
-  }
+static int front_solve_lds(int nw, int maxwork) {
+  return (maxwork + (sizeof(T) == 8 ? 64 * nw : 0)) * (int)sizeof(T);
+}
+
+template <typename T>
+void prepare_front_solve(int nw, int maxwork) {
+  const int bytes = front_solve_lds<T>(nw, maxwork);
+  if (bytes <= 64 * 1024) return;
+  const void* k;
+  if constexpr (sizeof(T) == 8)
+    k = nw == 16 ? reinterpret_cast<const void*>(&k_front_solve_mma<16>)
+                 : reinterpret_cast<const void*>(&k_front_solve_mma<8>);
+  else
+    k = nw == 16 ? reinterpret_cast<const void*>(&k_front_solve<16>)
+                 : reinterpret_cast<const void*>(&k_front_solve<8>);
+  (void)hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
 }
 
 template <typename T>
 void launch_front_solve(const T* tiles, const FrontSub* subs, int nsub, int nw, int maxwork, const int32_t* inds,
                         const double* r, double* sol, hipStream_t st, const double* skip) {
   if (nsub <= 0) return;
-  const size_t lds = (size_t)maxwork * sizeof(T);
-  if (nw == 16)
-    hipLaunchKernelGGL((k_front_solve<T, 16>), dim3(nsub), dim3(1024), lds, st, tiles, subs, inds, r, sol, skip);
-  else
-    hipLaunchKernelGGL((k_front_solve<T, 8>), dim3(nsub), dim3(512), lds, st, tiles, subs, inds, r, sol, skip);
+  const size_t lds = (size_t)front_solve_lds<T>(nw, maxwork);
+  const dim3 g(nsub), b(64 * nw);
+  if constexpr (sizeof(T) == 8) {
+    if (nw == 16)
+      hipLaunchKernelGGL(k_front_solve_mma<16>, g, b, lds, st, tiles, subs, maxwork, inds, r, sol, skip);
+    else
+      hipLaunchKernelGGL(k_front_solve_mma<8>, g, b, lds, st, tiles, subs, maxwork, inds, r, sol, skip);
+  } else {
+    if (nw == 16)
+      hipLaunchKernelGGL(k_front_solve<16>, g, b, lds, st, tiles, subs, inds, r, sol, skip);
+    else
+      hipLaunchKernelGGL(k_front_solve<8>, g, b, lds, st, tiles, subs, inds, r, sol, skip);
+  }
 }
 
 #define DOUG_INSTANTIATE_FRONTS(T)                                                                              \
@@ -813,7 +1054,7 @@ void launch_front_solve(const T* tiles, const FrontSub* subs, int nsub, int nw, 
                                         const int32_t*, const int32_t*, const int32_t*, const double*,          \
                                         hipStream_t);                                                           \
   template void launch_front_factor<T>(T*, T*, const FrontSub*, int, int, int, bool, int*, hipStream_t);        \
-  template void prepare_front_solve<T>(int);                                                                    \
+  template void prepare_front_solve<T>(int, int);                                                                   \
   template void launch_front_solve<T>(const T*, const FrontSub*, int, int, int, const int32_t*, const double*,  \
                                       double*, hipStream_t, const double*);
 DOUG_INSTANTIATE_FRONTS(double)

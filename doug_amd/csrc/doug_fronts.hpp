@@ -12,6 +12,8 @@ namespace doug {
 
 constexpr int kFrontCols = 64;    // columns of a front at most
 constexpr int kFrontWavesMax = 16;  // wavefronts of the solve's workgroup: 8 or 16
+// column groups per unit of the solve, FP32 and FP64: 64 rows of them are 8 KB
+constexpr int kFrontUnitGroups32 = 8, kFrontUnitGroups64 = 4;
 
 // One front: columns at positions c0 .. c0+k-1 of the elimination order and
 // m boundary rows (later positions, ascending).  Its panel holds, for the

@@ -163,7 +163,9 @@ struct doug_ctx {
   LocalLists batch_lists;
   double* d_btiles = nullptr;
   float* d_btiles32 = nullptr;
-  int front_nw = 8;  // wavefronts per subdomain in the single-vector solve
+  int front_nw = 8;      // wavefronts per workgroup in the single-vector solve
+  int front_groups = 1;  // workgroups per subdomain
+  double* d_updates = nullptr;  // updates between them
   doug_tuning tuning{};
   double* d_tiles = nullptr;   // FP64 factors
   float* d_tiles32 = nullptr;  // FP32 factors (DOUG_PREC_FP32_FACTORS)
@@ -1039,6 +1041,13 @@ static int build_fronts(doug_ctx* ctx, const Csr& M, const std::vector<int>& sta
   std::vector<uint32_t> src;
   std::vector<FrontUnit> uf, ub;
   std::vector<int32_t> hp, lf, lb;
+  struct BOff {
+    size_t uf, ub, lf, lb, gp, uo, ui;
+  };
+  std::vector<BOff> boff;
+  std::vector<FrontUnit> buf, bub;
+  std::vector<int32_t> blf, blb, gpos, gtop, uoff;
+  std::vector<uint16_t> uidx;
   std::vector<double> flops;
   for (const FrontPattern& P : pats) {
     off.push_back(Off{fr.size(), rpos.size(), col.size(), hp.size(), hl.size(), uf.size(), ub.size(), lf.size(),
@@ -1053,6 +1062,15 @@ static int build_fronts(doug_ctx* ctx, const Csr& M, const std::vector<int>& sta
     ub.insert(ub.end(), P.units_b.begin(), P.units_b.end());
     lf.insert(lf.end(), P.list_f.begin(), P.list_f.end());
     lb.insert(lb.end(), P.list_b.begin(), P.list_b.end());
+    boff.push_back(BOff{buf.size(), bub.size(), blf.size(), blb.size(), gpos.size(), uoff.size(), uidx.size()});
+    buf.insert(buf.end(), P.bunits_f.begin(), P.bunits_f.end());
+    bub.insert(bub.end(), P.bunits_b.begin(), P.bunits_b.end());
+    blf.insert(blf.end(), P.blist_f.begin(), P.blist_f.end());
+    blb.insert(blb.end(), P.blist_b.begin(), P.blist_b.end());
+    gpos.insert(gpos.end(), P.gpos.begin(), P.gpos.end());
+    gtop.insert(gtop.end(), P.gtop.begin(), P.gtop.end());
+    uoff.insert(uoff.end(), P.uoff.begin(), P.uoff.end());
+    uidx.insert(uidx.end(), P.uidx.begin(), P.uidx.end());
     double f = 0.0;
     for (const Front& q : P.fronts)
       f += (double)q.k * q.k * q.k * 2.0 / 3.0 + 4.0 * q.k * q.k * q.m + 1.0 * q.k * q.m * q.m;
@@ -1068,6 +1086,16 @@ static int build_fronts(doug_ctx* ctx, const Csr& M, const std::vector<int>& sta
       (rc = upload(ctx, &d_uf, uf)) || (rc = upload(ctx, &d_ub, ub)) || (rc = upload(ctx, &d_lf, lf)) ||
       (rc = upload(ctx, &d_lb, lb)))
     return rc;
+  FrontUnit *d_buf = nullptr, *d_bub = nullptr;
+  int32_t *d_blf = nullptr, *d_blb = nullptr, *d_gpos = nullptr, *d_gtop = nullptr, *d_uoff = nullptr;
+  uint16_t* d_uidx = nullptr;
+  if (ctx->front_groups > 1 &&
+      ((rc = upload(ctx, &d_buf, buf)) || (rc = upload(ctx, &d_bub, bub)) || (rc = upload(ctx, &d_blf, blf)) ||
+       (rc = upload(ctx, &d_blb, blb)) || (rc = upload(ctx, &d_gpos, gpos)) ||
+       (rc = upload(ctx, &d_gtop, gtop)) || (rc = upload(ctx, &d_uoff, uoff)) ||
+       (rc = upload(ctx, &d_uidx, uidx))))
+    return rc;
+  int64_t updates = 0;
   std::vector<FrontSub>& subs = ctx->h_fsub;
   subs.assign((size_t)nb, FrontSub{});
   int64_t base = 0, sch = 0;
@@ -1079,10 +1107,13 @@ static int build_fronts(doug_ctx* ctx, const Csr& M, const std::vector<int>& sta
   for (int b = 0; b < nb; b++) {
     const FrontPattern& P = pats[pat[b]];
     const Off& o = off[pat[b]];
+    const BOff& bo = boff[pat[b]];
     const int nh = (int)P.hptr.size() - 1;
     subs[b] = FrontSub{base, (int64_t)starts[b], sch, d_fr + o.fr, d_rpos + o.rec, d_src + o.rec,
                        d_col + o.col, d_hp + o.hp, d_hl + o.hl, d_uf + o.uf, d_ub + o.ub, d_lf + o.lf,
-                       d_lb + o.lb, P.n, P.top0, P.work(), nh};
+                       d_lb + o.lb, d_buf + bo.uf, d_bub + bo.ub, d_blf + bo.lf, d_blb + bo.lb, d_gpos + bo.gp,
+                       d_gtop + bo.gp, d_uoff + bo.uo, d_uidx + bo.ui, updates, P.n, P.top0, P.work(), nh};
+    updates += (int64_t)P.uidx.size();
     base += P.elems;
     sch += (P.schur + 15) / 16 * 16;
     f += flops[pat[b]];
@@ -1097,7 +1128,7 @@ static int build_fronts(doug_ctx* ctx, const Csr& M, const std::vector<int>& sta
   }
   *total_elems = base;
   if (chol_flops) *chol_flops = f;
-  if ((rc = upload(ctx, &ctx->d_fsub, subs))) return rc;
+  if ((rc = upload(ctx, &ctx->d_fsub, subs)) || (rc = dalloc(ctx, &ctx->d_updates, (size_t)updates))) return rc;
   if ((rc = dalloc(ctx, d_tiles, (size_t)base))) return rc;
   const size_t sch_bytes = (size_t)std::max<int64_t>(sch, 1) * sizeof(T);
   if (ctx->front_scratch.second < sch_bytes) {
@@ -2104,17 +2135,27 @@ static int device_fine(doug_ctx* ctx, hipEvent_t ev0, hipEvent_t ev1) {
     // vector fits a workgroup's LDS
     const bool f32 = ctx->precision == DOUG_PREC_FP32_FACTORS;
     const int64_t max_work = 160 * 1024 / (f32 ? 4 : 8) - 64 - (f32 ? 0 : 64 * kFrontWavesMax);
-    // eight wavefronts where two workgroups share a CU (512 subdomains, FP64:
-    // 806 us, 852 us with sixteen), sixteen where there is a CU for each (9
-    // subdomains: 113 us, 122 us with eight)
+    // eight wavefronts where a CU takes several subdomains (512, FP64: 806 us,
+    // 852 us with sixteen), sixteen where there is a CU for each (9 subdomains:
+    // 113 us, 122 us with eight)
     ctx->front_nw = ctx->nsub > 256 ? 8 : 16;
     // (the envelope solve's size limit holds for either: the batched solve uses it)
     bool sizes = true;
     for (size_t b = 0; b + 1 < ctx->sstarts.size(); b++)
       sizes = sizes && ctx->sstarts[b + 1] - ctx->sstarts[b] <= kMaxTrsvTiles * kTile;
-    ctx->fronts = sizes && build_front_patterns(A, ctx->sstarts, ctx->sinds, max_work, ctx->front_nw,
-                                                f32 ? kFrontUnitGroups32 : kFrontUnitGroups64,
-                                                pats, pat, dinds);
+    // two, four or eight workgroups per subdomain as long as each has a CU: 9
+    // subdomains of 2100 unknowns took 110 us with one, 74 us with four and
+    // 61 us with eight, 64 of 4300 171, 108 and (two rounds) 129 us, 100 of
+    // 4300 121 us with one, 96 us with two and 122 us with four, 225 137 us
+    // with one and 184 us with two
+    ctx->front_groups = 1;
+    while (!f32 && 2 * ctx->front_groups * ctx->nsub <= 256 && ctx->front_groups < kFrontGroupsMax)
+      ctx->front_groups *= 2;
+    const int units = f32 ? kFrontUnitGroups32 : kFrontUnitGroups64;
+    for (; sizes && !ctx->fronts && ctx->front_groups > 0; ctx->front_groups /= 2)
+      if ((ctx->fronts = build_front_patterns(A, ctx->sstarts, ctx->sinds, max_work, ctx->front_nw, ctx->front_groups,
+                                              units, pats, pat, dinds)))
+        break;
     if (!ctx->fronts) block_rcm(A, ctx->sstarts, ctx->sinds, dinds, &ctx->rank_ws);
   } else {
     dinds = ctx->sinds;
@@ -2575,11 +2616,11 @@ static void enqueue_subdomain_solves(doug_ctx* ctx, const double* r, double* sub
   }
   if (ctx->fronts) {
     if (ctx->precision == DOUG_PREC_FP32_FACTORS)
-      launch_front_solve(ctx->d_tiles32, ctx->d_fsub_solve, ctx->nsub, ctx->front_nw, ctx->maxwork, ctx->lists.inds, r, subsol,
-                         ctx->stream, skip);
+      launch_front_solve(ctx->d_tiles32, ctx->d_fsub_solve, ctx->nsub, ctx->front_nw, ctx->front_groups, ctx->maxwork,
+                         ctx->lists.inds, r, ctx->d_updates, subsol, ctx->stream, skip);
     else
-      launch_front_solve(ctx->d_tiles, ctx->d_fsub_solve, ctx->nsub, ctx->front_nw, ctx->maxwork, ctx->lists.inds, r, subsol,
-                         ctx->stream, skip);
+      launch_front_solve(ctx->d_tiles, ctx->d_fsub_solve, ctx->nsub, ctx->front_nw, ctx->front_groups, ctx->maxwork,
+                         ctx->lists.inds, r, ctx->d_updates, subsol, ctx->stream, skip);
     return;
   }
   if (ctx->precision == DOUG_PREC_FP32_FACTORS)

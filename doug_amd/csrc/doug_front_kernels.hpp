@@ -21,6 +21,10 @@ struct FrontSub {
   const uint16_t* hlist;
   const FrontUnit *units_f, *units_b;
   const int32_t *list_f, *list_b;
+  const FrontUnit *bunits_f, *bunits_b;  // subtrees of several workgroups
+  const int32_t *blist_f, *blist_b, *gpos, *gtop, *uoff;
+  const uint16_t* uidx;
+  int64_t ub;  // first of its entries between the workgroups' updates
   int32_t n, top0, work, nheights;
 };
 
@@ -36,14 +40,15 @@ void launch_front_scatter(T* tiles, const FrontSub* subs, int nsub, const int32_
 template <typename T>
 void launch_front_factor(T* tiles, T* schur, const FrontSub* subs, int nsub, int h, int maxcount, bool wide, int* flag,
                          hipStream_t st);
-// Solve of every subdomain by nw wavefronts each: gathers r(inds), writes the solution to sol (FP64,
+// Solve of every subdomain by `groups` workgroups of nw wavefronts each
+// (several in FP64 only; `updates` then holds what they hand over): gathers r(inds), writes the solution to sol (FP64,
 // concatenated layout).  maxwork: the largest pattern's work vector; call
 // prepare_front_solve<T>(nw, maxwork) once before.  skip (device, optional): the
 // launch does nothing when *skip != 0.
 template <typename T>
 void prepare_front_solve(int nw, int maxwork);
 template <typename T>
-void launch_front_solve(const T* tiles, const FrontSub* subs, int nsub, int nw, int maxwork, const int32_t* inds,
-                        const double* r, double* sol, hipStream_t st, const double* skip = nullptr);
+void launch_front_solve(const T* tiles, const FrontSub* subs, int nsub, int nw, int groups, int maxwork, const int32_t* inds,
+                        const double* r, double* updates, double* sol, hipStream_t st, const double* skip = nullptr);
 
 }  // namespace doug

@@ -268,11 +268,10 @@ struct ItemLists {
     if (cell.size() < (phase + 1) * nw) cell.resize((phase + 1) * nw);
     return cell[phase * nw + (size_t)w];
   }
-  // each wavefront's units, a barrier between two phases
+  // each wavefront's units, a barrier behind each phase, appended
   void flatten(const std::vector<Front>& F, int ug, bool fwd, std::vector<FrontUnit>& units,
                std::vector<int32_t>& list) const {
-    list.assign(1, 0);
-    units.clear();
+    if (list.empty()) list.push_back(0);
     const size_t phases = cell.size() / nw;
     for (int w = 0; w < nw; w++) {
       const size_t first = units.size();
@@ -328,9 +327,10 @@ struct ItemLists {
   }
 };
 
-bool make_pattern(const Graph& g, int64_t max_work, int nw, int ug, FrontPattern& P) {
-  const int n = g.n();
+bool make_pattern(const Graph& g, int64_t max_work, int nw, int groups, int ug, FrontPattern& P) {
+  const int n = g.n(), nwb = nw * groups;  // nwb wavefronts for the bottom subtrees
   P.n = n;
+  P.groups = groups;
   Dissector D(g);
   D.run(0, n, 0);
   // fronts in postorder, at most kFrontCols columns each: a longer separator
@@ -389,62 +389,91 @@ bool make_pattern(const Graph& g, int64_t max_work, int nw, int ug, FrontPattern
     F[f].m = (uint16_t)rows[f].size();
     if ((int)F[f].k + F[f].m > 64 * 250) return false;
   }
-  // bottom subtrees, one wavefront each, until they share out evenly over the
-  // wavefronts; what is above them goes level by level
   std::vector<int64_t> cost((size_t)nf);
   for (int f = 0; f < nf; f++) {
     cost[f] = front_cost(F[f], ug);
     for (int c : F[f].child)
       if (c >= 0) cost[f] += cost[c];
   }
-  std::vector<int> roots;
-  for (int f = 0; f < nf; f++)
-    if (parent[f] < 0) roots.push_back(f);
   auto heavier = [&](int a, int b) { return cost[a] != cost[b] ? cost[a] > cost[b] : a < b; };
-  std::vector<char> top((size_t)nf, 0);
-  std::vector<int> wave((size_t)nf, 0);
-  while (true) {
-    std::sort(roots.begin(), roots.end(), heavier);
-    int64_t load[kFrontWavesMax] = {}, sum = 0;
-    for (int f : roots) {
-      int w = 0;
-      for (int q = 1; q < nw; q++)
-        if (load[q] < load[w]) w = q;
-      load[w] += cost[f];
-      wave[f] = w;
-      sum += cost[f];
+  // Cuts the subtrees at `roots` until `ways` shares differ by less than
+  // num / den of their mean, or `most` subtrees: share[f] of each that is left,
+  // cut[f] = mark of the fronts above them.
+  auto cut_up = [&](std::vector<int>& roots, int ways, int num, int den, int most, std::vector<char>& cut,
+                    std::vector<int>& share) {
+    while (true) {
+      std::sort(roots.begin(), roots.end(), heavier);
+      int64_t load[kFrontWavesMax] = {}, sum = 0;
+      for (int f : roots) {
+        int w = 0;
+        for (int q = 1; q < ways; q++)
+          if (load[q] < load[w]) w = q;
+        load[w] += cost[f];
+        share[f] = w;
+        sum += cost[f];
+      }
+      const int64_t worst = *std::max_element(load, load + ways);
+      if (roots.empty() || den * ways * worst <= num * sum || (int)roots.size() >= most) break;
+      const int f = roots.front();
+      if (F[f].child[0] < 0 && F[f].child[1] < 0) break;  // a leaf is the heaviest
+      cut[f] = 1;
+      roots.erase(roots.begin());
+      for (int c : F[f].child)
+        if (c >= 0) roots.push_back(c);
     }
-    const int64_t worst = *std::max_element(load, load + nw);
-    if (roots.empty() || 10 * nw * worst <= 11 * sum || (int)roots.size() >= 6 * nw) break;
-    const int f = roots.front();
-    if (F[f].child[0] < 0 && F[f].child[1] < 0) break;  // a leaf is the heaviest
-    top[f] = 1;
-    roots.erase(roots.begin());
-    for (int c : F[f].child)
-      if (c >= 0) roots.push_back(c);
+  };
+  // groups: whole subtrees each; the apex above them is the last workgroup's
+  std::vector<int> group((size_t)nf, 0), wave((size_t)nf, 0);
+  std::vector<char> apex((size_t)nf, 0), top((size_t)nf, 0), is_root((size_t)nf, 0);
+  std::vector<int> all_roots;
+  for (int f = 0; f < nf; f++)
+    if (parent[f] < 0) all_roots.push_back(f);
+  if (groups > 1) cut_up(all_roots, groups, 12, 10, 4 * groups, apex, group);
+  std::vector<std::vector<int>> roots((size_t)groups);
+  for (int f : all_roots) roots[group[f]].push_back(f);
+  for (int f = nf - 1; f >= 0; f--)
+    if (!apex[f] && parent[f] >= 0 && !apex[parent[f]]) group[f] = group[parent[f]];
+  // in a group: bottom subtrees, one wavefront each; what is above them goes
+  // level by level
+  for (auto& r : roots) {
+    cut_up(r, nw, 11, 10, 6 * nw, top, wave);
+    for (int f : r) is_root[f] = 1;
   }
-  // new numbering: bottom subtrees in postorder, then the top fronts by height
+  // new numbering: the groups' bottom subtrees in postorder, then their top
+  // fronts by level, then the apex by level
   std::vector<int> seq, height((size_t)nf, 0), level((size_t)nf, -1);
-  std::vector<char> is_root((size_t)nf, 0);
-  for (int f : roots) is_root[f] = 1;
   for (int f = nf - 1; f >= 0; f--)  // a bottom front runs with its subtree's root
-    if (!top[f] && !is_root[f]) wave[f] = wave[parent[f]];
-  int levels = 0;
+    if (!apex[f] && !top[f] && !is_root[f]) wave[f] = wave[parent[f]];
+  std::vector<int> levels((size_t)groups + 1, 0);  // of each group, of the apex
   for (int f = 0; f < nf; f++) {
-    if (top[f]) level[f] = 0;
+    const bool up = top[f] || apex[f];
+    if (up) level[f] = 0;
     for (int c : F[f].child)
       if (c >= 0) {
         height[f] = std::max(height[f], height[c] + 1);
-        if (top[f] && top[c]) level[f] = std::max(level[f], level[c] + 1);
+        if (up && (top[c] || apex[c]) && apex[f] == apex[c]) level[f] = std::max(level[f], level[c] + 1);
       }
-    if (top[f]) levels = std::max(levels, level[f] + 1);
+    int& l = levels[apex[f] ? groups : group[f]];
+    if (up) l = std::max(l, level[f] + 1);
   }
-  for (int f = 0; f < nf; f++)
-    if (!top[f]) seq.push_back(f);
-  const int nbottom = (int)seq.size();
-  for (int l = 0; l < levels; l++)
+  std::vector<int> first_of(2 * (size_t)groups + 2, 0);  // fronts: bottoms of group g, tops of group g, apex, end
+  for (int q = 0; q < groups; q++) {
+    first_of[q] = (int)seq.size();
     for (int f = 0; f < nf; f++)
-      if (top[f] && level[f] == l) seq.push_back(f);
+      if (!apex[f] && !top[f] && group[f] == q) seq.push_back(f);
+  }
+  const int nbottom = (int)seq.size();
+  for (int q = 0; q < groups; q++) {
+    first_of[groups + q] = (int)seq.size();
+    for (int l = 0; l < levels[q]; l++)
+      for (int f = 0; f < nf; f++)
+        if (top[f] && group[f] == q && level[f] == l) seq.push_back(f);
+  }
+  first_of[2 * groups] = (int)seq.size();
+  for (int l = 0; l < levels[groups]; l++)
+    for (int f = 0; f < nf; f++)
+      if (apex[f] && level[f] == l) seq.push_back(f);
+  first_of[2 * groups + 1] = nf;
   std::vector<int> newid((size_t)nf), newpos((size_t)n);
   P.order.resize((size_t)n);
   P.colfront.resize((size_t)n);
@@ -482,7 +511,7 @@ bool make_pattern(const Graph& g, int64_t max_work, int nw, int ug, FrontPattern
     R[q].resize(f.m);
     for (int r = 0; r < f.m; r++) R[q][r] = (uint16_t)newpos[rows[o][r]];
     lv[q] = level[o];
-    wv[q] = wave[o];
+    wv[q] = group[o] * nw + wave[o];
     hv[q] = height[o];
     G[q] = f;
   }
@@ -494,14 +523,14 @@ bool make_pattern(const Graph& g, int64_t max_work, int nw, int ug, FrontPattern
   Space space;
   space.take(1);  // the zero entry
   {
-    Space own[kFrontWavesMax];
+    Space own[kFrontWavesMax * kFrontGroupsMax];
     for (int q = 0; q < nbottom; q++) {
       Space& s = own[wv[q]];
       u[q] = s.take(F[q].m);
       for (int c : F[q].child)
         if (c >= 0) s.give(u[c], F[c].m);
     }
-    for (int w = 0; w < nw; w++) {
+    for (int w = 0; w < nwb; w++) {
       const int64_t b = space.top;
       space.top += own[w].top;
       for (auto& h : own[w].hole) space.give(b + h.first, h.second - h.first);
@@ -510,7 +539,7 @@ bool make_pattern(const Graph& g, int64_t max_work, int nw, int ug, FrontPattern
     }
     for (int q = nbottom; q < nf;) {
       int e = q;
-      while (e < nf && lv[e] == lv[q]) e++;
+      while (e < nf && lv[e] == lv[q]) e++;  // (of two groups, too)
       for (int f = q; f < e; f++) u[f] = space.take(F[f].m);
       for (int f = q; f < e; f++)
         for (int c : F[f].child)
@@ -568,58 +597,83 @@ bool make_pattern(const Graph& g, int64_t max_work, int nw, int ug, FrontPattern
     P.schur = sp.top;
   }
   // work lists
-  ItemLists fw{nw, {}}, bw{nw, {}};
   auto rows_of = [&](int f) { return (F[f].k + F[f].m + 63) / 64; };
   auto put = [&](ItemLists& l, size_t phase, int w, int f, int first, int count) {
     if (count > 0) l.at(phase, w).push_back(Item{f, first, count});
   };
-  for (int q = 0; q < nbottom; q++) {
-    put(fw, 0, wv[q], q, 0, rows_of(q));
-    const int r = nbottom - 1 - q;
-    put(bw, (size_t)levels, wv[r], r, 0, (F[r].k + 3) / 4);
-  }
-  for (int q = nbottom; q < nf;) {
-    int e = q;
-    while (e < nf && lv[e] == lv[q]) e++;
-    const size_t pf = (size_t)lv[q] + 1, pb = (size_t)(levels - 1 - lv[q]);
-    std::vector<int> byw;
-    for (int f = q; f < e; f++) byw.push_back(f);
-    std::sort(byw.begin(), byw.end(), [&](int a, int b) {
-      const int64_t x = front_cost(F[a], ug), y = front_cost(F[b], ug);
-      return x != y ? x > y : a < b;
-    });
-    fw.at(pf, 0);
-    bw.at(pb, 0);
-    if (e - q >= nw) {  // whole fronts, heaviest first to the least loaded
-      int64_t load[kFrontWavesMax] = {};
-      for (int f : byw) {
-        int w = 0;
-        for (int x = 1; x < nw; x++)
-          if (load[x] < load[w]) w = x;
-        load[w] += front_cost(F[f], ug);
-        put(fw, pf, w, f, 0, rows_of(f));
-        put(bw, pb, w, f, 0, (F[f].k + 3) / 4);
-      }
-    } else {  // each front split over its share of the wavefronts
-      int w0 = 0;
-      const int cnt = e - q;
-      for (int i = 0; i < cnt; i++) {
-        const int share = nw / cnt + (i < nw % cnt ? 1 : 0), f = byw[i];
-        const int nc = rows_of(f), ng = (F[f].k + 3) / 4;
-        for (int x = 0; x < share; x++) {
-          const int b = nc * x / share, c = nc * (x + 1) / share, gb = ng * x / share, gc = ng * (x + 1) / share;
-          put(fw, pf, w0 + x, f, b, c - b);
-          put(bw, pb, w0 + x, f, gb, gc - gb);
+  // the fronts [from, to), one level after the other from phase `first` on,
+  // backward the other way round from phase 0
+  auto put_levels = [&](ItemLists& fw, ItemLists& bw, int from, int to, size_t first, int count) {
+    for (int q = from; q < to;) {
+      int e = q;
+      while (e < to && lv[e] == lv[q]) e++;
+      const size_t pf = (size_t)lv[q] + first, pb = (size_t)(count - 1 - lv[q]);
+      std::vector<int> byw;
+      for (int f = q; f < e; f++) byw.push_back(f);
+      std::sort(byw.begin(), byw.end(), [&](int a, int b) {
+        const int64_t x = front_cost(F[a], ug), y = front_cost(F[b], ug);
+        return x != y ? x > y : a < b;
+      });
+      fw.at(pf, 0);
+      bw.at(pb, 0);
+      if (e - q >= nw) {  // whole fronts, heaviest first to the least loaded
+        int64_t load[kFrontWavesMax] = {};
+        for (int f : byw) {
+          int w = 0;
+          for (int x = 1; x < nw; x++)
+            if (load[x] < load[w]) w = x;
+          load[w] += front_cost(F[f], ug);
+          put(fw, pf, w, f, 0, rows_of(f));
+          put(bw, pb, w, f, 0, (F[f].k + 3) / 4);
         }
-        w0 += share;
+      } else {  // each front split over its share of the wavefronts
+        int w0 = 0;
+        const int cnt = e - q;
+        for (int i = 0; i < cnt; i++) {
+          const int share = nw / cnt + (i < nw % cnt ? 1 : 0), f = byw[i];
+          const int nc = rows_of(f), ng = (F[f].k + 3) / 4;
+          for (int x = 0; x < share; x++) {
+            const int b = nc * x / share, c = nc * (x + 1) / share, gb = ng * x / share, gc = ng * (x + 1) / share;
+            put(fw, pf, w0 + x, f, b, c - b);
+            put(bw, pb, w0 + x, f, gb, gc - gb);
+          }
+          w0 += share;
+        }
       }
+      q = e;
     }
-    q = e;
+  };
+  for (int g = 0; g < groups; g++) {
+    ItemLists fw{nw, {}}, bw{nw, {}};
+    for (int q = first_of[g]; q < (g + 1 < groups ? first_of[g + 1] : nbottom); q++)
+      put(fw, 0, wv[q] - g * nw, q, 0, rows_of(q));
+    put_levels(fw, bw, first_of[groups + g], first_of[groups + g + 1], 1, levels[g]);
+    for (int q = (g + 1 < groups ? first_of[g + 1] : nbottom) - 1; q >= first_of[g]; q--)
+      put(bw, (size_t)levels[g], wv[q] - g * nw, q, 0, (F[q].k + 3) / 4);
+    fw.at((size_t)levels[g], 0);
+    bw.at((size_t)levels[g], 0);
+    fw.flatten(F, ug, true, groups > 1 ? P.bunits_f : P.units_f, groups > 1 ? P.blist_f : P.list_f);
+    bw.flatten(F, ug, false, groups > 1 ? P.bunits_b : P.units_b, groups > 1 ? P.blist_b : P.list_b);
   }
-  fw.at((size_t)levels, 0);
-  bw.at((size_t)levels, 0);
-  fw.flatten(F, ug, true, P.units_f, P.list_f);
-  bw.flatten(F, ug, false, P.units_b, P.list_b);
+  if (groups > 1) {
+    ItemLists fw{nw, {}}, bw{nw, {}};
+    put_levels(fw, bw, first_of[2 * groups], nf, 0, levels[groups]);
+    fw.flatten(F, ug, true, P.units_f, P.list_f);
+    bw.flatten(F, ug, false, P.units_b, P.list_b);
+    auto position = [&](int q) { return q < nf ? (int)F[q].c0 : n; };
+    for (int q = 0; q <= groups; q++) {
+      P.gpos.push_back(q < groups ? position(first_of[q]) : P.top0);
+      P.gtop.push_back(position(first_of[groups + q]));
+    }
+    P.uoff.assign(1, 0);
+    for (int g = 0; g < groups; g++) {
+      for (int q = first_of[2 * groups]; q < nf; q++)
+        for (int c : F[q].child)
+          if (c >= 0 && c < first_of[2 * groups] && wv[c] / nw == g)
+            for (int r = 0; r < F[c].m; r++) P.uidx.push_back((uint16_t)(F[c].u + r));
+      P.uoff.push_back((int32_t)P.uidx.size());
+    }
+  }
   return true;
 }
 
@@ -687,7 +741,8 @@ int64_t front_entry(const FrontPattern& p, int lo, int hi, bool dbl) {
 }
 
 bool build_front_patterns(const Csr& A, const std::vector<int>& starts, const std::vector<int>& inds,
-                          int64_t max_work, int nw, int ug, std::vector<FrontPattern>& patterns, std::vector<int>& pat,
+                          int64_t max_work, int nw, int groups, int ug,
+                          std::vector<FrontPattern>& patterns, std::vector<int>& pat,
                           std::vector<int>& out) {
   const int nb = (int)starts.size() - 1;
   pat.assign((size_t)nb, -1);
@@ -726,7 +781,7 @@ bool build_front_patterns(const Csr& A, const std::vector<int>& starts, const st
               mine = known.back().get();
             }
           }
-          if (mine && !make_pattern(mine->g, max_work, nw, ug, mine->p)) {
+          if (mine && !make_pattern(mine->g, max_work, nw, groups, ug, mine->p)) {
             std::lock_guard<std::mutex> lk(mu);
             ok = false;
             return;

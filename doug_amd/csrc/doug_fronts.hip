@@ -760,6 +760,7 @@ __device__ __forceinline__ FrontUnit unit_of(const RawUnit& r) {
 // before its barriers.
 template <typename Load, typename F, typename G, typename H>
 __device__ __forceinline__ void walk_units(const FrontUnit* units, int u, int end, F&& load, G&& work, H&& barriers) {
+  if (u >= end) return;
   Load q0, q1;
   RawUnit r0 = raw_unit(units, u), r1 = raw_unit(units, u + 1);
   FrontUnit d0 = unit_of(r0), d1 = unit_of(r1);
@@ -817,18 +818,30 @@ __device__ __forceinline__ int panel_bytes(int H, int g1) { return 32 * (g1 * H 
 // vector.  Lanes outside the front, or right of its diagonal, load nothing and
 // get zeros: what bounds the kernel where subdomains are few is the 64 bytes a
 // cycle that a CU loads, and half of a unit is such lanes on average.
-// 512 subdomains of 5440 unknowns: 805 us, 5.6 TB/s (the vector form 804,
-// envelopes 1735); 343 of 4600: 395 us (414, 950); 64 of 4300 in two
-// dimensions: 171 us (188, 709); 9 of 2100: 110 us (113, 310).
-template <int NW>
+// 512 subdomains of 5440 unknowns: 803 us, 5.6 TB/s, bound by HBM (the vector
+// form 804, envelopes 1735); 343 of 4600: 395 us (414, 950).
+//
+// Where subdomains are at most half as many as the CUs, two, four or eight
+// workgroups share one, each with subtrees of its own: stage 1 takes these
+// forward, stage 2 the few fronts above them in both directions and stage 3
+// the subtrees backward; y and the updates in between go through global
+// memory.  Stage 0 is all of it in one workgroup.  64 subdomains of 4300
+// unknowns in two dimensions: 35 + 38 + 34 us (171 us in one workgroup each,
+// the vector form 188, envelopes 709); 9 of 2100: 15 + 30 + 17 us (110, 113,
+// 310).
+enum { kWhole = 0, kSubtreesForward = 1, kApex = 2, kSubtreesBackward = 3 };
+template <int NW, int STAGE>
 __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(4))) void k_front_solve_mma(
-    const double* __restrict__ tiles, const FrontSub* __restrict__ subs, int maxwork,
-    const int32_t* __restrict__ inds, const double* __restrict__ rhs, double* __restrict__ sol, const double* skip) {
+    const double* __restrict__ tiles, const FrontSub* __restrict__ subs, int groups, int maxwork,
+    const int32_t* __restrict__ inds, const double* __restrict__ rhs, double* updates, double* sol,
+    const double* skip) {
   if (skip && *skip != 0.0) return;
   constexpr int UG = kFrontUnitGroups64;
   extern __shared__ __align__(16) unsigned char front_dyn[];
   double* L = reinterpret_cast<double*>(front_dyn);
-  const FrontSub s = subs[blockIdx.x];
+  constexpr bool kGroup = STAGE == kSubtreesForward || STAGE == kSubtreesBackward;
+  const int grp = kGroup ? (int)blockIdx.x % groups : 0;
+  const FrontSub s = subs[kGroup ? (int)blockIdx.x / groups : (int)blockIdx.x];
   const int t = threadIdx.x, lane = t & 63, w = __builtin_amdgcn_readfirstlane(t >> 6);
   const int lo = lane & 3, mid = (lane >> 2) & 3, hi = lane >> 4;
   double* stage = L + maxwork + 64 * w;
@@ -837,14 +850,31 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(4))) vo
   if (n == 0) return;
   const Global<uint32_t> src = global(s.src);
   const Global<uint16_t> rpos = global(s.rpos);
-  for (int p = t; p < n; p += 64 * NW) L[p] = rhs[inds[s.vec + p]];
-  if (t == 0) L[n] = 0.0;
+  double* X = L + n - top0;  // solution at the positions from top0 on
+  // this workgroup's positions: [p0, p1), and its subtrees' top fronts [p2, p3)
+  const int apex0 = STAGE == kWhole ? n : list_at(s.gtop, groups);
+  const int p0 = kGroup ? list_at(s.gpos, grp) : STAGE == kApex ? apex0 : 0;
+  const int p1 = kGroup ? list_at(s.gpos, grp + 1) : n;
+  const int p2 = kGroup ? list_at(s.gtop, grp) : n, p3 = kGroup ? list_at(s.gtop, grp + 1) : n;
+  auto own = [&](auto&& f) {
+    for (int p = p0 + t; p < p1; p += 64 * NW) f(p);
+    for (int p = p2 + t; p < p3; p += 64 * NW) f(p);
+  };
+  if (STAGE == kSubtreesBackward) {
+    own([&](int p) { L[p] = sol[s.vec + p]; });
+    for (int p = apex0 + t; p < n; p += 64 * NW) X[p] = sol[s.vec + p];
+  } else {
+    own([&](int p) { L[p] = rhs[inds[s.vec + p]]; });
+    if (t == 0) L[n] = 0.0;
+  }
+  if (STAGE == kApex)
+    for (int q = t; q < list_at(s.uoff, groups); q += 64 * NW) L[s.uidx[q]] = updates[s.ub + q];
   lds_barrier();
   struct Load {
     Two a[UG / 2][4];
     uint32_t r, c;
   };
-  {
+  if constexpr (STAGE != kSubtreesBackward) {
     // y of a front that several wavefronts share: its right-hand side is
     // still read by the others, so it is written behind the next barrier
     double acc[4] = {0.0, 0.0, 0.0, 0.0}, pend = 0.0;
@@ -910,11 +940,18 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(4))) vo
         pend_at = -1;
       }
     };
-    walk_units<Load>(s.units_f, list_at(s.list_f, w), list_at(s.list_f, w + 1), load, work, barriers);
+    const int32_t* list = STAGE == kSubtreesForward ? s.blist_f + NW * grp : s.list_f;
+    walk_units<Load>(STAGE == kSubtreesForward ? s.bunits_f : s.units_f, list_at(list, w), list_at(list, w + 1), load,
+                     work, barriers);
   }
-  lds_barrier();
-  double* X = L + n - top0;  // solution at the positions from top0 on
-  {
+  if (STAGE == kSubtreesForward) {
+    lds_barrier();
+    own([&](int p) { sol[s.vec + p] = L[p]; });
+    for (int q = list_at(s.uoff, grp) + t; q < list_at(s.uoff, grp + 1); q += 64 * NW) updates[s.ub + q] = L[s.uidx[q]];
+    return;
+  }
+  if (STAGE != kSubtreesBackward) lds_barrier();
+  if constexpr (STAGE != kSubtreesForward) {
     double acc[UG] = {0.0, 0.0, 0.0, 0.0}, y0 = 0.0;
     auto load = [&](Load& q, const FrontUnit& d) {
       const auto pan = panel_buffer(base + d.pan, panel_bytes(d.h, d.g1));
@@ -972,10 +1009,12 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(4))) vo
     auto barriers = [&](int count) {
       for (int i = 0; i < count; i++) lds_barrier();
     };
-    walk_units<Load>(s.units_b, list_at(s.list_b, w), list_at(s.list_b, w + 1), load, work, barriers);
+    const int32_t* list = STAGE == kSubtreesBackward ? s.blist_b + NW * grp : s.list_b;
+    walk_units<Load>(STAGE == kSubtreesBackward ? s.bunits_b : s.units_b, list_at(list, w), list_at(list, w + 1), load,
+                     work, barriers);
   }
   lds_barrier();
-  for (int p = t; p < n; p += 64 * NW) sol[s.vec + p] = p < top0 ? L[p] : X[p];
+  own([&](int p) { sol[s.vec + p] = p < top0 ? L[p] : X[p]; });
 }
 
 }  // namespace
@@ -1020,32 +1059,46 @@ template <typename T>
 void prepare_front_solve(int nw, int maxwork) {
   const int bytes = front_solve_lds<T>(nw, maxwork);
   if (bytes <= 64 * 1024) return;
-  const void* k;
-  if constexpr (sizeof(T) == 8)
-    k = nw == 16 ? reinterpret_cast<const void*>(&k_front_solve_mma<16>)
-                 : reinterpret_cast<const void*>(&k_front_solve_mma<8>);
-  else
-    k = nw == 16 ? reinterpret_cast<const void*>(&k_front_solve<16>)
-                 : reinterpret_cast<const void*>(&k_front_solve<8>);
-  (void)hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
+  auto allow = [bytes](auto kernel) {
+    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
+  };
+  if constexpr (sizeof(T) == 8) {
+    allow(&k_front_solve_mma<8, kWhole>);
+    allow(&k_front_solve_mma<16, kWhole>);
+    allow(&k_front_solve_mma<16, kSubtreesForward>);
+    allow(&k_front_solve_mma<16, kApex>);
+    allow(&k_front_solve_mma<16, kSubtreesBackward>);
+  } else {
+    allow(&k_front_solve<8>);
+    allow(&k_front_solve<16>);
+  }
 }
 
 template <typename T>
-void launch_front_solve(const T* tiles, const FrontSub* subs, int nsub, int nw, int maxwork, const int32_t* inds,
-                        const double* r, double* sol, hipStream_t st, const double* skip) {
+void launch_front_solve(const T* tiles, const FrontSub* subs, int nsub, int nw, int groups, int maxwork,
+                        const int32_t* inds, const double* r, double* updates, double* sol, hipStream_t st,
+                        const double* skip) {
   if (nsub <= 0) return;
   const size_t lds = (size_t)front_solve_lds<T>(nw, maxwork);
-  const dim3 g(nsub), b(64 * nw);
+  const dim3 b(64 * nw);
   if constexpr (sizeof(T) == 8) {
-    if (nw == 16)
-      hipLaunchKernelGGL(k_front_solve_mma<16>, g, b, lds, st, tiles, subs, maxwork, inds, r, sol, skip);
-    else
-      hipLaunchKernelGGL(k_front_solve_mma<8>, g, b, lds, st, tiles, subs, maxwork, inds, r, sol, skip);
+    auto go = [&](auto kernel, int blocks) {
+      hipLaunchKernelGGL(kernel, dim3(blocks), b, lds, st, tiles, subs, groups, maxwork, inds, r, updates, sol, skip);
+    };
+    if (groups > 1) {  // nw is 16
+      go(k_front_solve_mma<16, kSubtreesForward>, nsub * groups);
+      go(k_front_solve_mma<16, kApex>, nsub);
+      go(k_front_solve_mma<16, kSubtreesBackward>, nsub * groups);
+    } else if (nw == 16) {
+      go(k_front_solve_mma<16, kWhole>, nsub);
+    } else {
+      go(k_front_solve_mma<8, kWhole>, nsub);
+    }
   } else {
     if (nw == 16)
-      hipLaunchKernelGGL(k_front_solve<16>, g, b, lds, st, tiles, subs, inds, r, sol, skip);
+      hipLaunchKernelGGL(k_front_solve<16>, dim3(nsub), b, lds, st, tiles, subs, inds, r, sol, skip);
     else
-      hipLaunchKernelGGL(k_front_solve<8>, g, b, lds, st, tiles, subs, inds, r, sol, skip);
+      hipLaunchKernelGGL(k_front_solve<8>, dim3(nsub), b, lds, st, tiles, subs, inds, r, sol, skip);
   }
 }
 
@@ -1055,8 +1108,8 @@ void launch_front_solve(const T* tiles, const FrontSub* subs, int nsub, int nw, 
                                         hipStream_t);                                                           \
   template void launch_front_factor<T>(T*, T*, const FrontSub*, int, int, int, bool, int*, hipStream_t);        \
   template void prepare_front_solve<T>(int, int);                                                                   \
-  template void launch_front_solve<T>(const T*, const FrontSub*, int, int, int, const int32_t*, const double*,  \
-                                      double*, hipStream_t, const double*);
+  template void launch_front_solve<T>(const T*, const FrontSub*, int, int, int, int, const int32_t*,            \
+                                      const double*, double*, double*, hipStream_t, const double*);
 DOUG_INSTANTIATE_FRONTS(double)
 DOUG_INSTANTIATE_FRONTS(float)
 #undef DOUG_INSTANTIATE_FRONTS

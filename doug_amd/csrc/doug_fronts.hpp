@@ -12,6 +12,7 @@ namespace doug {
 
 constexpr int kFrontCols = 64;    // columns of a front at most
 constexpr int kFrontWavesMax = 16;  // wavefronts of the solve's workgroup: 8 or 16
+constexpr int kFrontGroupsMax = 8;  // workgroups that share a subdomain's subtrees
 // column groups per unit of the solve, FP32 and FP64: 64 rows of them are 8 KB
 constexpr int kFrontUnitGroups32 = 8, kFrontUnitGroups64 = 4;
 
@@ -82,6 +83,15 @@ struct FrontPattern {
   std::vector<uint16_t> hlist;
   std::vector<FrontUnit> units_f, units_b;   // wavefront w: units[list[w] .. list[w + 1])
   std::vector<int32_t> list_f, list_b;
+  // With several groups the lists above hold the apex only; workgroup g takes
+  // subtrees, their bottom fronts at the positions [gpos[g], gpos[g + 1]) and
+  // top ones at [gtop[g], gtop[g + 1]), its wavefront w list nw g + w of these.
+  // uidx: the work indices of the updates that the apex takes from them, group
+  // by group.
+  int groups = 1;
+  std::vector<FrontUnit> bunits_f, bunits_b;
+  std::vector<int32_t> blist_f, blist_b, gpos, gtop, uoff;
+  std::vector<uint16_t> uidx;
   int work() const { return n + usz; }
 };
 
@@ -100,9 +110,11 @@ int64_t front_entry(const FrontPattern& p, int lo, int hi, bool dbl);
 // each): pat[b] is subdomain b's pattern in `patterns`, out its blocks in
 // elimination order.  False, with nothing usable, when some subdomain's
 // structure exceeds the format (work indices of 16 bits, `max_work` entries
-// of work vector, panel offsets of 31 bits).  nw wavefronts, ug groups per unit.
+// of work vector, panel offsets of 31 bits).  nw wavefronts per workgroup,
+// `groups` workgroups for the subtrees, ug column groups per unit.
 bool build_front_patterns(const Csr& A, const std::vector<int>& starts, const std::vector<int>& inds,
-                          int64_t max_work, int nw, int ug, std::vector<FrontPattern>& patterns, std::vector<int>& pat,
+                          int64_t max_work, int nw, int groups, int ug,
+                          std::vector<FrontPattern>& patterns, std::vector<int>& pat,
                           std::vector<int>& out);
 
 }  // namespace doug

@@ -139,8 +139,33 @@ struct Run {
 
   // One pass; a wavefront runs to its next barrier before the next one starts.
   void pass(bool fwd, bool reversed, vector<double>& L) const {
-    const auto& units = fwd ? p.units_f : p.units_b;
-    const auto& list = fwd ? p.list_f : p.list_b;
+    if (p.groups == 1) return walk(fwd, reversed, fwd ? p.units_f : p.units_b, fwd ? p.list_f : p.list_b, L);
+    const vector<double> in = L;
+    const int n = p.n, nw = (int)p.blist_f.size() / p.groups, apex0 = p.gtop.back();
+    auto slot = [&](int q) { return (size_t)(q < p.top0 || fwd ? q : n + q - p.top0); };
+    // each group has a work vector of its own: its positions and, backward,
+    // the apex's solution; forward it leaves its y and its updates for the apex
+    auto subtrees = [&]() {
+      const vector<int32_t>& list = fwd ? p.blist_f : p.blist_b;
+      for (int g = 0; g < p.groups; g++) {
+        vector<double> own(L.size(), NAN);
+        for (int q = p.gpos[g]; q < p.gpos[g + 1]; q++) own[q] = in[q];
+        for (int q = p.gtop[g]; q < p.gtop[g + 1]; q++) own[q] = in[q];
+        if (fwd) own[n] = 0;
+        for (int q = apex0; !fwd && q < n; q++) own[slot(q)] = L[slot(q)];
+        walk(fwd, reversed, fwd ? p.bunits_f : p.bunits_b,
+             vector<int32_t>(list.begin() + g * nw, list.begin() + (g + 1) * nw + 1), own);
+        for (int q = p.gpos[g]; q < p.gpos[g + 1]; q++) L[slot(q)] = own[slot(q)];
+        for (int q = p.gtop[g]; q < p.gtop[g + 1]; q++) L[slot(q)] = own[slot(q)];
+        for (int q = p.uoff[g]; fwd && q < p.uoff[g + 1]; q++) L[p.uidx[q]] = own[p.uidx[q]];
+      }
+    };
+    if (fwd) subtrees();
+    walk(fwd, reversed, fwd ? p.units_f : p.units_b, fwd ? p.list_f : p.list_b, L);
+    if (!fwd) subtrees();
+  }
+  void walk(bool fwd, bool reversed, const vector<FrontUnit>& units, const vector<int32_t>& list,
+            vector<double>& L) const {
     const int nw = (int)list.size() - 1, n = p.n;
     vector<int> next(list.begin(), list.end() - 1), owed((size_t)nw, 0);
     vector<vector<double>> f((size_t)nw, vector<double>(64, 0.0)), acc(f), y0(f);
@@ -204,17 +229,29 @@ struct Run {
   }
 };
 
-static int check(const char* name, const Csr& A, int nw, int ug) {
+static int check(const char* name, const Csr& A, int nw, int groups, int ug) {
   const int n = A.nrows;
   vector<int> starts{0, n}, inds((size_t)n), pat, out, pos((size_t)n);
   for (int i = 0; i < n; i++) inds[i] = i;
   vector<FrontPattern> P;
-  if (!build_front_patterns(A, starts, inds, 65535, nw, ug, P, pat, out)) {
+  if (!build_front_patterns(A, starts, inds, 65535, nw, groups, ug, P, pat, out)) {
     printf("%s: refused\n", name);
     return 1;
   }
   for (int q = 0; q < n; q++) pos[out[q]] = q;
   const FrontPattern& p = P[0];
+  if (groups > 1) {  // the groups' positions follow one another, and each lists only its own fronts
+    if (p.gpos.front() != 0 || p.gpos.back() != p.top0 || p.gtop.front() != p.top0) return 1;
+    for (int w = 0; w < nw * groups; w++)
+      for (int i = p.blist_f[w]; i < p.blist_f[w + 1]; i++) {
+        const FrontUnit& u = p.bunits_f[i];
+        const vector<int32_t>& range = u.c0 < p.top0 ? p.gpos : p.gtop;
+        if (u.flags && (u.c0 < range[w / nw] || u.c0 + u.k > range[w / nw + 1])) {
+          printf("%s: a front outside its group\n", name);
+          return 1;
+        }
+      }
+  }
   for (bool dbl : {true, false}) {
     Run run{p, {}, {}, dbl};
     if (!run.factor(A, pos)) {
@@ -245,7 +282,7 @@ static int check(const char* name, const Csr& A, int nw, int ug) {
           if (A.col[e] == i) dmax = std::max(dmax, A.val[e]);
       const double bound = 2.3e-16 * n * 20.0 * dmax;
       if (!(std::sqrt(err / norm) <= bound)) {
-        printf("%s nw %d ug %d dbl %d reversed %d: error %g, bound %g\n", name, nw, ug, dbl, reversed,
+        printf("%s nw %d groups %d ug %d dbl %d reversed %d: error %g, bound %g\n", name, nw, groups, ug, dbl, reversed,
                std::sqrt(err / norm), bound);
         return 1;
       }
@@ -256,22 +293,22 @@ static int check(const char* name, const Csr& A, int nw, int ug) {
 
 int main() {
   int bad = 0;
-  for (int cfg = 0; cfg < 3; cfg++) {
-    const int nw = cfg == 1 ? 16 : 8, ug = cfg == 0 ? 8 : 4;
-    bad |= check("one node", grid(1, 1, 1), nw, ug);
-    bad |= check("two nodes", grid(1, 1, 2), nw, ug);
-    bad |= check("line of 33", grid(33, 1, 1), nw, ug);
-    bad |= check("line of 1000", grid(1000, 1, 1), nw, ug);
-    bad |= check("4 x 4 x 4", grid(4, 4, 4), nw, ug);
-    bad |= check("5 x 7 x 9", grid(5, 7, 9), nw, ug);
-    bad |= check("14 x 14 x 14", grid(14, 14, 14), nw, ug);
-    bad |= check("66 x 66", grid(66, 66, 1), nw, ug);
-    bad |= check("2 x 70 x 30", grid(2, 70, 30), nw, ug);
-    bad |= check("scattered", scattered(700, 3, 1, false), nw, ug);
-    bad |= check("seven components", scattered(900, 2, 7, false), nw, ug);
-    bad |= check("many components", scattered(600, 1, 200, false), nw, ug);
-    bad |= check("hub", scattered(800, 1, 5, true), nw, ug);
-    bad |= check("dense", scattered(200, 150, 1, true), nw, ug);
+  for (int cfg = 0; cfg < 6; cfg++) {
+    const int nw = cfg == 0 || cfg == 2 ? 8 : 16, ug = cfg == 0 ? 8 : 4, groups = cfg < 3 ? 1 : 1 << (cfg - 2);
+    bad |= check("one node", grid(1, 1, 1), nw, groups, ug);
+    bad |= check("two nodes", grid(1, 1, 2), nw, groups, ug);
+    bad |= check("line of 33", grid(33, 1, 1), nw, groups, ug);
+    bad |= check("line of 1000", grid(1000, 1, 1), nw, groups, ug);
+    bad |= check("4 x 4 x 4", grid(4, 4, 4), nw, groups, ug);
+    bad |= check("5 x 7 x 9", grid(5, 7, 9), nw, groups, ug);
+    bad |= check("14 x 14 x 14", grid(14, 14, 14), nw, groups, ug);
+    bad |= check("66 x 66", grid(66, 66, 1), nw, groups, ug);
+    bad |= check("2 x 70 x 30", grid(2, 70, 30), nw, groups, ug);
+    bad |= check("scattered", scattered(700, 3, 1, false), nw, groups, ug);
+    bad |= check("seven components", scattered(900, 2, 7, false), nw, groups, ug);
+    bad |= check("many components", scattered(600, 1, 200, false), nw, groups, ug);
+    bad |= check("hub", scattered(800, 1, 5, true), nw, groups, ug);
+    bad |= check("dense", scattered(200, 150, 1, true), nw, groups, ug);
   }
   // refused, not truncated, where the work vector does not fit
   {
@@ -279,7 +316,7 @@ int main() {
     vector<int> starts{0, A.nrows}, inds((size_t)A.nrows), pat, out;
     for (int i = 0; i < A.nrows; i++) inds[i] = i;
     vector<FrontPattern> P;
-    if (build_front_patterns(A, starts, inds, A.nrows + 10, 8, 8, P, pat, out)) {
+    if (build_front_patterns(A, starts, inds, A.nrows + 10, 8, 1, 8, P, pat, out)) {
       printf("a work vector too long was accepted\n");
       bad = 1;
     }

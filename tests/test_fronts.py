@@ -69,7 +69,8 @@ def test_solves_the_subdomains(kind, precision):
     eps = 1.2e-7 if precision else 2.3e-16
     bound = eps * max(n, 64) * 2.0 * A.diagonal().max()
     print(f"fronts {kind} precision={precision} n={n}", flush=True)
-    for parts in (1, 3) if n >= 3 else (1,):
+    # workgroups per subdomain: eight up to 32 subdomains, four up to 64, two up to 128
+    for parts in (1, 3, 50, 100, 150) if n >= 1500 else (1, 3) if n >= 3 else (1,):
         cut = np.linspace(0, n, parts + 1).astype(int)
         sets = [np.arange(cut[p], cut[p + 1]) for p in range(parts)]
         z = np.zeros(n)

@@ -2914,7 +2914,8 @@ static int pcg_core(doug_ctx* ctx, double tol, int maxit, int32_t* it_out, doubl
   // replayed from a captured HIP graph
   auto enqueue_iteration = [&](bool first) {
     enqueue_prec(ctx, ctx->d_r, ctx->d_z, true, done_flag);  // with rho = r.z and beta
-    launch_p_update(n, ctx->d_z, ctx->d_p, ctx->d_scal, first ? 1 : 0, st);
+    const int nrho = (n - 1) / (ctx->p.method == 0 ? kVecChunk : 256) + 1;
+    launch_p_update(n, ctx->d_z, ctx->d_p, ctx->d_scal, first ? 1 : 0, ctx->d_partial, nrho, st);
     enqueue_spmv(ctx, ctx->d_p, ctx->d_q);
     launch_dot(ctx->d_p, ctx->d_q, n, ctx->d_partial, nullptr, 2, ctx->d_scal, st);
     launch_xr_update(n, ctx->d_x, ctx->d_r, ctx->d_p, ctx->d_q, ctx->d_partial, ctx->d_scal, st, ctx->d_hist);

@@ -1,6 +1,5 @@
 // gfx950 kernels of the frontal subdomain factors (doug_fronts.hpp): scatter
-// of the matrix entries, the factorisation height by height, and the solves
-// for one and for several right-hand sides.
+// of the matrix entries, the factorisation height by height, and the solves.
 #include "doug_tile.hpp"
 #include "doug_front_kernels.hpp"
 
@@ -556,8 +555,9 @@ __device__ __forceinline__ void load_panel(UnitLoad& b, const float* pan, const 
   }
 }
 
-// Forward and backward substitution for one subdomain per workgroup, in FP32; the right-hand side is gathered from (and the solution
-// written to) FP64 vectors.  The work vector (positions, then update vectors
+// Forward and backward substitution for one subdomain per workgroup, in FP32;
+// the right-hand side is gathered from (and the solution written to) FP64
+// vectors.  The work vector (positions, then update vectors
 // or the top fronts' solution) lives in LDS.  Nothing when *skip is set.
 // Forward: one front's panel times its right-hand side, a lane per row, the
 // columns' values broadcast from the lanes that gathered them.  Backward: the

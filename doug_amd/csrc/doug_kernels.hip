@@ -877,10 +877,10 @@ __global__ void k_overlap_sum(int n, const int32_t* __restrict__ occ_ptr,
 
 // ------------------------------------------------------------------------
 // Deterministic reductions: a fixed tree per workgroup, then the partials
-// summed in a fixed order (k_reduce_finish, or the last workgroup of the
-// several-column kernels) before the scalar recurrence.
+// summed in a fixed order (k_reduce_finish, fold_partials, or the last
+// workgroup of the several-column kernels) before the scalar recurrence.
 // ------------------------------------------------------------------------
-enum { S_RHO = 0, S_RHO_PREV = 1, S_BETA = 2, S_PQ = 3, S_ALPHA = 4, S_RES = 5 };
+enum { S_RHO = 0, S_RHO_PREV = 1, S_BETA = 2, S_PQ = 3, S_ALPHA = 4, S_RES = 5, S_RHO_NEXT = 6 };
 // the single-vector PCG's convergence test on the device (see k_reduce_finish)
 enum { S_DONE = 8, S_ITER = 9, S_THR = 10, S_INIT = 11, S_MAXIT = 12, S_HCAP = 13 };
 
@@ -906,6 +906,7 @@ __device__ __forceinline__ double block_sum(double v, double* sh) {
 // writes (alpha, beta, residual) to out[3(it-1)..] for it <= S_HCAP, and
 // sets S_DONE once !(res / S_INIT > S_THR) or it >= S_MAXIT, the host's
 // test; after that the iteration's other kernels leave x and r alone.
+// Mode 4 is mode 3 where rho was folded into the p update: it becomes S_RHO.
 __global__ __launch_bounds__(1024) void k_reduce_finish(const double* __restrict__ partial, int count,
                                                         double* out, int mode, double* scal) {
   __shared__ double sh[16];
@@ -930,7 +931,12 @@ __global__ __launch_bounds__(1024) void k_reduce_finish(const double* __restrict
       scal[S_ALPHA] = scal[S_RHO] / s;
     } else if (!out) {
       scal[S_RES] = s;
-    } else if (scal[S_DONE] == 0.0) {
+    } else {
+      if (mode == 4) {
+        scal[S_RHO_PREV] = scal[S_RHO];
+        scal[S_RHO] = scal[S_RHO_NEXT];
+      }
+      if (scal[S_DONE] != 0.0) return;
       scal[S_RES] = s;
       const int it = (int)scal[S_ITER] + 1;
       scal[S_ITER] = it;
@@ -971,11 +977,52 @@ __global__ __launch_bounds__(256) void k_dot_chunks(const double* __restrict__ a
   if (threadIdx.x == 0) partial[blockIdx.x] = s;
 }
 
+// The sum of at most kFoldPartials partials by a workgroup of 256, in every
+// thread and in k_reduce_finish's order.  Up to that many (262,144 unknowns)
+// the kernel that needs a sum forms it itself, each workgroup again, instead
+// of waiting for a launch of one workgroup (4.2 us each, two an iteration):
+// solves of 16,384 unknowns 3.64 to 3.58 ms, of 250,000 14.21 to 14.09 ms.
+// Above, the partials are more than a workgroup should read again.
+__device__ __forceinline__ double fold_partials(const double* __restrict__ partial, int count, double* sh) {
+  const int t = threadIdx.x, lane = t & 63, w = t >> 6;
+  double v[kFoldPartials / 256];
+#pragma unroll
+  for (int j = 0; j < kFoldPartials / 256; j++) {
+    const int q = t + 256 * j;
+    v[j] = 0.0 + (q < count ? partial[q] : 0.0);
+  }
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1)
+#pragma unroll
+    for (int j = 0; j < kFoldPartials / 256; j++) v[j] += __shfl_xor(v[j], o);
+  if (lane == 0)
+#pragma unroll
+    for (int j = 0; j < kFoldPartials / 256; j++) sh[4 * j + w] = v[j];
+  __syncthreads();
+  double s = 0.0;
+#pragma unroll
+  for (int k = 0; k < kFoldPartials / 64; k++) s += sh[k];
+  return s;
+}
+
+// p = z + beta p; with `count` partials of r.z, rho and beta are formed here
+// (S_RHO stays the last iteration's until k_reduce_finish's mode 4).
 __global__ __launch_bounds__(256) void k_p_update_chunks(int n, const double* __restrict__ z,
-                                                         double* __restrict__ p,
-                                                         const double* __restrict__ scal, int first) {
+                                                         double* __restrict__ p, double* scal, int first,
+                                                         const double* __restrict__ partial, int count) {
+  __shared__ double sh[kFoldPartials / 64];
   const int i0 = blockIdx.x * kVecChunk + threadIdx.x;
-  const double beta = first ? 0.0 : scal[S_BETA];
+  double beta;
+  if (count > 0) {
+    const double s = fold_partials(partial, count, sh);
+    beta = s / scal[S_RHO];
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+      scal[S_BETA] = beta;
+      scal[S_RHO_NEXT] = s;
+    }
+  } else {
+    beta = scal[S_BETA];
+  }
   double zv[kVecPer], pv[kVecPer];
 #pragma unroll
   for (int k = 0; k < kVecPer; k++) {
@@ -991,16 +1038,27 @@ __global__ __launch_bounds__(256) void k_p_update_chunks(int n, const double* __
 }
 
 // x += alpha p, r -= alpha q and r.r partials; nothing once the device's
-// convergence test has passed (S_DONE).
+// convergence test has passed (S_DONE).  With `count` partials of p.q (not
+// where the r.r partials go), alpha is formed here.
 __global__ __launch_bounds__(256) void k_xr_update_chunks(int n, double* __restrict__ x,
                                                           double* __restrict__ r,
                                                           const double* __restrict__ p,
                                                           const double* __restrict__ q,
-                                                          const double* __restrict__ scal,
-                                                          double* partial) {
-  __shared__ double sh[4];
+                                                          double* scal, double* __restrict__ partial,
+                                                          const double* __restrict__ pq, int count) {
+  __shared__ double sh[4], fold[kFoldPartials / 64];
   if (scal[S_DONE] != 0.0) return;
-  const double alpha = scal[S_ALPHA];
+  double alpha;
+  if (count > 0) {
+    const double s = fold_partials(pq, count, fold);
+    alpha = scal[S_RHO_NEXT] / s;
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+      scal[S_PQ] = s;
+      scal[S_ALPHA] = alpha;
+    }
+  } else {
+    alpha = scal[S_ALPHA];
+  }
   const int i0 = blockIdx.x * kVecChunk + threadIdx.x;
   double xv[kVecPer], rv[kVecPer], pv[kVecPer], qv[kVecPer];
 #pragma unroll
@@ -2527,24 +2585,30 @@ void launch_overlap_sum(int n, const int32_t* occ_ptr, const int32_t* occ_pos, c
                      sol, rt_ptr, rt_col, rt_val, csol, z);
 }
 
+// both sums' partials fit (r.z has one per 256 unknowns, p.q one per 1024)
+static bool folds(int n) { return cdiv(n, 256) <= kFoldPartials; }
+
 void launch_dot(const double* a, const double* b, int n, double* partial, double* out, int mode,
                 double* scal, hipStream_t st) {
   const int nb = (int)cdiv(n, kVecChunk);
   hipLaunchKernelGGL(k_dot_chunks, dim3(nb), dim3(256), 0, st, a, b, n, partial);
+  if (mode != 3 && folds(n)) return;
   hipLaunchKernelGGL(k_reduce_finish, dim3(1), dim3(1024), 0, st, partial, nb, out, mode, scal);
 }
 
-void launch_p_update(int n, const double* z, double* p, const double* scal, int first,
-                     hipStream_t st) {
+void launch_p_update(int n, const double* z, double* p, double* scal, int first, const double* partial,
+                     int count, hipStream_t st) {
   hipLaunchKernelGGL(k_p_update_chunks, dim3(cdiv(n, kVecChunk)), dim3(256), 0, st, n, z, p, scal,
-                     first);
+                     first, partial, folds(n) ? count : 0);
 }
 
 void launch_xr_update(int n, double* x, double* r, const double* p, const double* q,
                       double* partial, double* scal, hipStream_t st, double* hist) {
   const int nb = (int)cdiv(n, kVecChunk);
-  hipLaunchKernelGGL(k_xr_update_chunks, dim3(nb), dim3(256), 0, st, n, x, r, p, q, scal, partial);
-  hipLaunchKernelGGL(k_reduce_finish, dim3(1), dim3(1024), 0, st, partial, nb, hist, 3, scal);
+  double* const rr = folds(n) ? partial + nb : partial;  // every workgroup still reads p.q's
+  hipLaunchKernelGGL(k_xr_update_chunks, dim3(nb), dim3(256), 0, st, n, x, r, p, q, scal, rr, partial,
+                     folds(n) ? nb : 0);
+  hipLaunchKernelGGL(k_reduce_finish, dim3(1), dim3(1024), 0, st, rr, nb, hist, folds(n) ? 4 : 3, scal);
 }
 
 void launch_overlap_sum_dot(int n, const int32_t* occ_ptr, const int32_t* occ_pos, const double* sol,
@@ -2554,7 +2618,7 @@ void launch_overlap_sum_dot(int n, const int32_t* occ_ptr, const int32_t* occ_po
   const int nb = (int)cdiv(n, 256);
   hipLaunchKernelGGL(k_overlap_sum_dot, dim3(nb), dim3(256), 0, st, n, occ_ptr, occ_pos, sol, rt_ptr,
                      rt_col, rt_val, csol, z, r, partial);
-  hipLaunchKernelGGL(k_reduce_finish, dim3(1), dim3(1024), 0, st, partial, nb, nullptr, 1, scal);
+  if (!folds(n)) hipLaunchKernelGGL(k_reduce_finish, dim3(1), dim3(1024), 0, st, partial, nb, nullptr, 1, scal);
 }
 
 void launch_copy(double* dst, const double* src, int n, hipStream_t st) {

@@ -13,6 +13,7 @@ constexpr int kMaxTrsvTiles = 256;     // subdomain size limit of the one-block 
 constexpr int kRedBlocks = 1024;       // fixed partial count of the grid reductions
 constexpr int kRedBlocksWide = 8192;   // grid of the column-pair reductions (partials per column)
 constexpr int kVecChunk = 1024;        // entries per workgroup of the PCG vector kernels
+constexpr int kFoldPartials = 1024;    // partials that the vector kernels sum themselves
 // partial sums the single-vector reductions of an n-vector need
 constexpr int64_t vec_partials(int64_t n) { return (n + 255) / 256 + kRedBlocks; }
 constexpr int kMaxRhs = 32;            // right-hand sides per batched solve
@@ -190,8 +191,11 @@ void launch_overlap_sum_dot(int n, const int32_t* occ_ptr, const int32_t* occ_po
 // vec_partials(n) doubles.
 void launch_dot(const double* a, const double* b, int n, double* partial, double* out, int mode,
                 double* scal, hipStream_t st);
-void launch_p_update(int n, const double* z, double* p, const double* scal, int first,
-                     hipStream_t st);
+// Up to 256 kFoldPartials unknowns launch_dot (modes 1 and 2) and
+// launch_overlap_sum_dot leave their sums to this (of the `count` partials of
+// r.z) and to launch_xr_update.
+void launch_p_update(int n, const double* z, double* p, double* scal, int first, const double* partial,
+                     int count, hipStream_t st);
 // With hist, the residual's finish keeps the iteration count, the
 // (alpha, beta, residual) history and the convergence flag on the device
 // (scal slots S_DONE.. of the kernels); x and r stay unchanged once set.

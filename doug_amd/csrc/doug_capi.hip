@@ -2147,9 +2147,10 @@ static int device_fine(doug_ctx* ctx, hipEvent_t ev0, hipEvent_t ev1) {
     // subdomains of 2100 unknowns took 110 us with one, 74 us with four and
     // 61 us with eight, 64 of 4300 171, 108 and (two rounds) 129 us, 100 of
     // 4300 121 us with one, 96 us with two and 122 us with four, 225 137 us
-    // with one and 184 us with two
+    // with one and 184 us with two (FP64; in FP32 64 of 4300 103 us with one
+    // and 75 us with four, 100 103 us with one and 88 us with two)
     ctx->front_groups = 1;
-    while (!f32 && 2 * ctx->front_groups * ctx->nsub <= 256 && ctx->front_groups < kFrontGroupsMax)
+    while (2 * ctx->front_groups * ctx->nsub <= 256 && ctx->front_groups < kFrontGroupsMax)
       ctx->front_groups *= 2;
     const int units = f32 ? kFrontUnitGroups32 : kFrontUnitGroups64;
     for (; sizes && !ctx->fronts && ctx->front_groups > 0; ctx->front_groups /= 2)

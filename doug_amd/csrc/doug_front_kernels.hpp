@@ -41,7 +41,7 @@ template <typename T>
 void launch_front_factor(T* tiles, T* schur, const FrontSub* subs, int nsub, int h, int maxcount, bool wide, int* flag,
                          hipStream_t st);
 // Solve of every subdomain by `groups` workgroups of nw wavefronts each
-// (several in FP64 only; `updates` then holds what they hand over): gathers r(inds), writes the solution to sol (FP64,
+// (`updates` holds what several hand over): gathers r(inds), writes the solution to sol (FP64,
 // concatenated layout).  maxwork: the largest pattern's work vector; call
 // prepare_front_solve<T>(nw, maxwork) once before.  skip (device, optional): the
 // launch does nothing when *skip != 0.

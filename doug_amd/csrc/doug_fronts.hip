@@ -568,29 +568,59 @@ __device__ __forceinline__ void load_panel(UnitLoad& b, const float* pan, const 
 // 6 GB in 879 us).  Hence the unit lists: a wavefront's next panel rows are
 // always on their way, across barriers too, and the leaves' subtrees run side
 // by side without any.
-template <int NW>
+//
+// Where subdomains are at most half as many as the CUs, two, four or eight
+// workgroups share one, each with subtrees of its own: stage 1 takes these
+// forward, stage 2 the few fronts above them in both directions and stage 3
+// the subtrees backward; y and the updates in between go through global
+// memory (as doubles, unrounded).  Stage 0 is all of it in one workgroup.
+// 64 subdomains of 5250 unknowns: 181 us (248 us in one workgroup each); of
+// 4300 in two dimensions 75 us (103); 4 of 4300: 57 us (95).
+enum { kWhole = 0, kSubtreesForward = 1, kApex = 2, kSubtreesBackward = 3 };
+template <int NW, int STAGE>
 __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(4))) void k_front_solve(
-    const float* __restrict__ tiles, const FrontSub* __restrict__ subs, const int32_t* __restrict__ inds,
-    const double* __restrict__ rhs, double* __restrict__ sol, const double* skip) {
+    const float* __restrict__ tiles, const FrontSub* __restrict__ subs, int groups,
+    const int32_t* __restrict__ inds, const double* __restrict__ rhs, double* updates, double* sol,
+    const double* skip) {
   if (skip && *skip != 0.0) return;
   typedef float T;
   constexpr int UG = kFrontUnitGroups32;
   extern __shared__ __align__(16) unsigned char front_dyn[];
   T* L = reinterpret_cast<T*>(front_dyn);
-  const FrontSub s = subs[blockIdx.x];
+  constexpr bool kGroup = STAGE == kSubtreesForward || STAGE == kSubtreesBackward;
+  const int grp = kGroup ? (int)blockIdx.x % groups : 0;
+  const FrontSub s = subs[kGroup ? (int)blockIdx.x / groups : (int)blockIdx.x];
   const int t = threadIdx.x, lane = t & 63, w = __builtin_amdgcn_readfirstlane(t >> 6);
   const T* base = tiles + s.base;
   const int n = s.n, top0 = s.top0;
   if (n == 0) return;
   const Global<uint32_t> src = global(s.src);
   const Global<uint16_t> rpos = global(s.rpos);
-  for (int p = t; p < n; p += 64 * NW) L[p] = (T)rhs[inds[s.vec + p]];
-  if (t == 0) L[n] = (T)0;
+  T* X = L + n - top0;  // solution at the positions from top0 on
+  // this workgroup's positions: [p0, p1), and its subtrees' top fronts [p2, p3)
+  const int apex0 = STAGE == kWhole ? n : list_at(s.gtop, groups);
+  const int p0 = kGroup ? list_at(s.gpos, grp) : STAGE == kApex ? apex0 : 0;
+  const int p1 = kGroup ? list_at(s.gpos, grp + 1) : n;
+  const int p2 = kGroup ? list_at(s.gtop, grp) : n, p3 = kGroup ? list_at(s.gtop, grp + 1) : n;
+  auto own = [&](auto&& f) {
+    for (int p = p0 + t; p < p1; p += 64 * NW) f(p);
+    for (int p = p2 + t; p < p3; p += 64 * NW) f(p);
+  };
+  if (STAGE == kSubtreesBackward) {
+    own([&](int p) { L[p] = (T)sol[s.vec + p]; });
+    for (int p = apex0 + t; p < n; p += 64 * NW) X[p] = (T)sol[s.vec + p];
+  } else {
+    own([&](int p) { L[p] = (T)rhs[inds[s.vec + p]]; });
+    if (t == 0) L[n] = (T)0;
+  }
+  if (STAGE == kApex)
+    for (int q = t; q < list_at(s.uoff, groups); q += 64 * NW) L[s.uidx[q]] = (T)updates[s.ub + q];
   lds_barrier();
-  {
-    const UnitPtr units = unit_list(s.units_f);
-    int u0 = list_at(s.list_f, w);
-    const int last = list_at(s.list_f, w + 1) - 1;
+  if constexpr (STAGE != kSubtreesBackward) {
+    const UnitPtr units = unit_list(STAGE == kSubtreesForward ? s.bunits_f : s.units_f);
+    const int32_t* list = STAGE == kSubtreesForward ? s.blist_f + NW * grp : s.list_f;
+    int u0 = list_at(list, w);
+    const int last = list_at(list, w + 1) - 1;
     T fv = (T)0, a[4] = {(T)0, (T)0, (T)0, (T)0};
     // y of a front that several wavefronts share: its right-hand side is
     // still read by the others, so it is written behind the next barrier
@@ -639,8 +669,11 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(4))) vo
       }
     };
     UnitLoad b0, b1;
-    FrontUnit d0 = unit_at(units + u0);
-    load(b0, d0);
+    FrontUnit d0{};
+    if (u0 < last) {  // a subdomain may have no fronts above its subtrees
+      d0 = unit_at(units + u0);
+      load(b0, d0);
+    }
     for (; u0 < last; u0 += 2) {  // two units a turn: lists have even lengths
       const FrontUnit d1 = unit_at(units + u0 + 1);
       load(b1, d1);
@@ -650,12 +683,19 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(4))) vo
       work(b1, d1);
     }
   }
-  lds_barrier();
-  T* X = L + n - top0;  // solution at the positions from top0 on
-  {
-    const UnitPtr units = unit_list(s.units_b);
-    int u0 = list_at(s.list_b, w);
-    const int last = list_at(s.list_b, w + 1) - 1;
+  if (STAGE == kSubtreesForward) {
+    lds_barrier();
+    own([&](int p) { sol[s.vec + p] = (double)L[p]; });
+    for (int q = list_at(s.uoff, grp) + t; q < list_at(s.uoff, grp + 1); q += 64 * NW)
+      updates[s.ub + q] = (double)L[s.uidx[q]];
+    return;
+  }
+  if (STAGE != kSubtreesBackward) lds_barrier();
+  if constexpr (STAGE != kSubtreesForward) {
+    const UnitPtr units = unit_list(STAGE == kSubtreesBackward ? s.bunits_b : s.units_b);
+    const int32_t* list = STAGE == kSubtreesBackward ? s.blist_b + NW * grp : s.list_b;
+    int u0 = list_at(list, w);
+    const int last = list_at(list, w + 1) - 1;
     T y0 = (T)0, acc[4 * UG];
 #pragma unroll
     for (int q = 0; q < 4 * UG; q++) acc[q] = (T)0;
@@ -695,8 +735,11 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(4))) vo
       for (int q = 0; q < d.nbar; q++) lds_barrier();
     };
     UnitLoad b0, b1;
-    FrontUnit d0 = unit_at(units + u0);
-    load(b0, d0);
+    FrontUnit d0{};
+    if (u0 < last) {  // a subdomain may have no fronts above its subtrees
+      d0 = unit_at(units + u0);
+      load(b0, d0);
+    }
     for (; u0 < last; u0 += 2) {  // two units a turn: lists have even lengths
       const FrontUnit d1 = unit_at(units + u0 + 1);
       load(b1, d1);
@@ -707,7 +750,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(4))) vo
     }
   }
   lds_barrier();
-  for (int p = t; p < n; p += 64 * NW) sol[s.vec + p] = (double)(p < top0 ? L[p] : X[p]);
+  own([&](int p) { sol[s.vec + p] = (double)(p < top0 ? L[p] : X[p]); });
 }
 
 // ---- FP64: the same on the matrix cores ----
@@ -821,15 +864,10 @@ __device__ __forceinline__ int panel_bytes(int H, int g1) { return 32 * (g1 * H 
 // 512 subdomains of 5440 unknowns: 803 us, 5.6 TB/s, bound by HBM (the vector
 // form 804, envelopes 1735); 343 of 4600: 395 us (414, 950).
 //
-// Where subdomains are at most half as many as the CUs, two, four or eight
-// workgroups share one, each with subtrees of its own: stage 1 takes these
-// forward, stage 2 the few fronts above them in both directions and stage 3
-// the subtrees backward; y and the updates in between go through global
-// memory.  Stage 0 is all of it in one workgroup.  64 subdomains of 4300
+// The stages are those of the vector form.  64 subdomains of 4300
 // unknowns in two dimensions: 35 + 38 + 34 us (171 us in one workgroup each,
 // the vector form 188, envelopes 709); 9 of 2100: 15 + 30 + 17 us (110, 113,
 // 310).
-enum { kWhole = 0, kSubtreesForward = 1, kApex = 2, kSubtreesBackward = 3 };
 template <int NW, int STAGE>
 __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(4))) void k_front_solve_mma(
     const double* __restrict__ tiles, const FrontSub* __restrict__ subs, int groups, int maxwork,
@@ -1069,8 +1107,11 @@ void prepare_front_solve(int nw, int maxwork) {
     allow(&k_front_solve_mma<16, kApex>);
     allow(&k_front_solve_mma<16, kSubtreesBackward>);
   } else {
-    allow(&k_front_solve<8>);
-    allow(&k_front_solve<16>);
+    allow(&k_front_solve<8, kWhole>);
+    allow(&k_front_solve<16, kWhole>);
+    allow(&k_front_solve<16, kSubtreesForward>);
+    allow(&k_front_solve<16, kApex>);
+    allow(&k_front_solve<16, kSubtreesBackward>);
   }
 }
 
@@ -1081,25 +1122,24 @@ void launch_front_solve(const T* tiles, const FrontSub* subs, int nsub, int nw, 
   if (nsub <= 0) return;
   const size_t lds = (size_t)front_solve_lds<T>(nw, maxwork);
   const dim3 b(64 * nw);
-  if constexpr (sizeof(T) == 8) {
-    auto go = [&](auto kernel, int blocks) {
-      hipLaunchKernelGGL(kernel, dim3(blocks), b, lds, st, tiles, subs, groups, maxwork, inds, r, updates, sol, skip);
+  auto go = [&](auto whole8, auto whole, auto forward, auto apex, auto backward, auto... work) {
+    auto one = [&](auto kernel, int blocks) {
+      hipLaunchKernelGGL(kernel, dim3(blocks), b, lds, st, tiles, subs, groups, work..., inds, r, updates, sol, skip);
     };
     if (groups > 1) {  // nw is 16
-      go(k_front_solve_mma<16, kSubtreesForward>, nsub * groups);
-      go(k_front_solve_mma<16, kApex>, nsub);
-      go(k_front_solve_mma<16, kSubtreesBackward>, nsub * groups);
-    } else if (nw == 16) {
-      go(k_front_solve_mma<16, kWhole>, nsub);
+      one(forward, nsub * groups);
+      one(apex, nsub);
+      one(backward, nsub * groups);
     } else {
-      go(k_front_solve_mma<8, kWhole>, nsub);
+      one(nw == 16 ? whole : whole8, nsub);
     }
-  } else {
-    if (nw == 16)
-      hipLaunchKernelGGL(k_front_solve<16>, dim3(nsub), b, lds, st, tiles, subs, inds, r, sol, skip);
-    else
-      hipLaunchKernelGGL(k_front_solve<8>, dim3(nsub), b, lds, st, tiles, subs, inds, r, sol, skip);
-  }
+  };
+  if constexpr (sizeof(T) == 8)
+    go(&k_front_solve_mma<8, kWhole>, &k_front_solve_mma<16, kWhole>, &k_front_solve_mma<16, kSubtreesForward>,
+       &k_front_solve_mma<16, kApex>, &k_front_solve_mma<16, kSubtreesBackward>, maxwork);
+  else
+    go(&k_front_solve<8, kWhole>, &k_front_solve<16, kWhole>, &k_front_solve<16, kSubtreesForward>,
+       &k_front_solve<16, kApex>, &k_front_solve<16, kSubtreesBackward>);
 }
 
 #define DOUG_INSTANTIATE_FRONTS(T)                                                                              \

@@ -293,8 +293,8 @@ static int check(const char* name, const Csr& A, int nw, int groups, int ug) {
 
 int main() {
   int bad = 0;
-  for (int cfg = 0; cfg < 6; cfg++) {
-    const int nw = cfg == 0 || cfg == 2 ? 8 : 16, ug = cfg == 0 ? 8 : 4, groups = cfg < 3 ? 1 : 1 << (cfg - 2);
+  for (int cfg = 0; cfg < 9; cfg++) {
+    const int nw = cfg == 0 || cfg == 2 ? 8 : 16, ug = cfg == 0 || cfg > 5 ? 8 : 4, groups = cfg < 3 ? 1 : 1 << (cfg < 6 ? cfg - 2 : cfg - 5);
     bad |= check("one node", grid(1, 1, 1), nw, groups, ug);
     bad |= check("two nodes", grid(1, 1, 2), nw, groups, ug);
     bad |= check("line of 33", grid(33, 1, 1), nw, groups, ug);

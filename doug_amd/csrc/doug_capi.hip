@@ -158,8 +158,8 @@ struct doug_ctx {
   std::vector<FrontSub> h_fsub;
   int maxwork = 0;  // largest work vector of a subdomain
   int64_t factor_elems = 0;
-  // the batched solve's envelope factors and lists (the ones above where the
-  // single-vector solve uses envelopes too)
+  // the batched solve's envelope factors and lists (the ones of the
+  // single-vector solve unless that has fronts), set by doug_prepare_batch
   LocalLists batch_lists;
   double* d_btiles = nullptr;
   float* d_btiles32 = nullptr;
@@ -3027,7 +3027,6 @@ static int next_pow2(int v) {
 // unknowns an application took 2.83 ms with either in FP32, and 4.6 ms against
 // 5.1 ms with fronts in FP64.
 static int batch_factors(doug_ctx* ctx) {
-  ctx->batch_lists = ctx->lists;
   ctx->d_btiles = ctx->d_tiles;
   ctx->d_btiles32 = ctx->d_tiles32;
   if (!ctx->fronts) return DOUG_OK;
@@ -3059,6 +3058,7 @@ int doug_prepare_batch(doug_ctx* ctx) {
   const int n = ctx->n, NR = kMaxRhs;
   hipStream_t st = ctx->stream;
   int rc;
+  ctx->batch_lists = ctx->lists;  // (without fine solves the overlap sum reads the identity lists)
   if (ctx->p.fine_method == 1) {
     if ((rc = batch_factors(ctx))) return rc;
     // panels of the envelope solves

@@ -3097,13 +3097,15 @@ int doug_prepare_batch(doug_ctx* ctx) {
 }
 
 // z = M^{-1} r for nrp columns (node-major, leading dimension nrp); with
-// rz_dot (nrp even) the overlap sum also forms rho = r.z per column
+// rz_dot (nrp even) the overlap sum also forms rho = r.z per column (without
+// a preconditioner a pass of its own)
 static void enqueue_prec_multi(doug_ctx* ctx, int nrp, const double* r, double* z, bool rz_dot = false) {
   const Params& p = ctx->p;
   hipStream_t st = ctx->stream;
   const int n = ctx->n, NR = nrp <= 16 ? 16 : 32;
   if (p.method == 0) {
     launch_copy(z, r, n * nrp, st);
+    if (rz_dot) launch_dot_multi(r, z, n, nrp, ctx->d_partialm, ctx->d_counterm, 1, ctx->d_scalm, st);
     return;
   }
   const bool coarse = ctx->has_coarse;

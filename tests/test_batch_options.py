@@ -51,3 +51,9 @@ def _compare(variant, nrhs):
                                      dict(method=5)])
 def test_columns_equal_the_single_vector_path(variant, nrhs):
     _compare(variant, nrhs)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("nrhs", [1, 2, 5])
+def test_without_a_preconditioner(nrhs):
+    _compare(dict(method=0), nrhs)

@@ -548,6 +548,7 @@ bool make_pattern(const Graph& g, int64_t max_work, int nw, int groups, int ug, 
     }
   }
   P.usz = (int)std::max<int64_t>(space.top, n - P.top0 + 1);
+  P.usz += (n + P.usz) % 2;  // what lies behind the work vector in LDS is read in 16-byte pieces
   if ((int64_t)n + P.usz > std::min<int64_t>(max_work, 65535)) return false;
   for (int q = 0; q < nf; q++) F[q].u = (uint16_t)(n + u[q]);
   // row records

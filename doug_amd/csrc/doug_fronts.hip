@@ -882,7 +882,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(4))) vo
   const FrontSub s = subs[kGroup ? (int)blockIdx.x / groups : (int)blockIdx.x];
   const int t = threadIdx.x, lane = t & 63, w = __builtin_amdgcn_readfirstlane(t >> 6);
   const int lo = lane & 3, mid = (lane >> 2) & 3, hi = lane >> 4;
-  double* stage = L + maxwork + 64 * w;
+  double* stage = L + maxwork + 64 * w;  // maxwork is even: 16-byte pieces
   const double* base = tiles + s.base;
   const int n = s.n, top0 = s.top0;
   if (n == 0) return;

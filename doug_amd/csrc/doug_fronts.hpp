@@ -44,8 +44,8 @@ constexpr int64_t front_panel_elems(int64_t k, int64_t m) {
 // Everything a subdomain's structure determines; subdomains of the same
 // local graph share one.
 //
-// Work vector of a solve: positions 0..n-1, then usz entries: entry n stays
-// zero, update vectors follow; in the backward pass the same entries hold
+// Work vector of a solve (of even length): positions 0..n-1, then usz entries:
+// entry n stays zero, update vectors follow; in the backward pass the same entries hold
 // the solution at the positions from top0 on (entry n + p - top0).
 // Row records: rpos, the position of each of the k + m rows; src, the work
 // indices of up to two children's update entries for the row (low and high

@@ -1220,7 +1220,7 @@ static int envelope_factors(doug_ctx* ctx, const std::vector<int>& dinds, const 
     ctx->maxnt = std::max(ctx->maxnt, d.nt);
     ctx->work_rows += (int64_t)d.nt * kTile;
   }
-  prepare_trsv<T>(ctx->maxnt);
+  HIPCHK(prepare_trsv<T>());
   return DOUG_OK;
 }
 
@@ -2134,7 +2134,7 @@ static int device_fine(doug_ctx* ctx, hipEvent_t ev0, hipEvent_t ev1) {
     // 18^3 unknowns, 3.7 times on squares of 66^2; as long as the solve's work
     // vector fits a workgroup's LDS
     const bool f32 = ctx->precision == DOUG_PREC_FP32_FACTORS;
-    const int64_t max_work = 160 * 1024 / (f32 ? 4 : 8) - 64 - (f32 ? 0 : 64 * kFrontWavesMax);
+    const int64_t max_work = kLdsBytes / (f32 ? 4 : 8) - 64 - (f32 ? 0 : 64 * kFrontWavesMax);
     // eight wavefronts where a CU takes several subdomains (512, FP64: 806 us,
     // 852 us with sixteen), sixteen where there is a CU for each (9 subdomains:
     // 113 us, 122 us with eight)
@@ -2217,12 +2217,8 @@ static int device_fine(doug_ctx* ctx, hipEvent_t ev0, hipEvent_t ev1) {
   info.factor_tiles = (elems + kTileElems - 1) / kTileElems;
   ctx->factor_elems = elems;
   if ((rc = set_trsv_order(ctx, ctx->trsv_order))) return rc;
-  if (ctx->fronts) {
-    if (ctx->precision == DOUG_PREC_FP32_FACTORS)
-      prepare_front_solve<float>(ctx->front_nw, ctx->maxwork);
-    else
-      prepare_front_solve<double>(ctx->front_nw, ctx->maxwork);
-  }
+  if (ctx->fronts)
+    HIPCHK(ctx->precision == DOUG_PREC_FP32_FACTORS ? prepare_front_solve<float>() : prepare_front_solve<double>());
   return DOUG_OK;
 }
 

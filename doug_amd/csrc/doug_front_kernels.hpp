@@ -43,10 +43,10 @@ void launch_front_factor(T* tiles, T* schur, const FrontSub* subs, int nsub, int
 // Solve of every subdomain by `groups` workgroups of nw wavefronts each
 // (`updates` holds what several hand over): gathers r(inds), writes the solution to sol (FP64,
 // concatenated layout).  maxwork: the largest pattern's work vector; call
-// prepare_front_solve<T>(nw, maxwork) once before.  skip (device, optional): the
+// prepare_front_solve<T>() once before on a device.  skip (device, optional): the
 // launch does nothing when *skip != 0.
 template <typename T>
-void prepare_front_solve(int nw, int maxwork);
+hipError_t prepare_front_solve();
 template <typename T>
 void launch_front_solve(const T* tiles, const FrontSub* subs, int nsub, int nw, int groups, int maxwork, const int32_t* inds,
                         const double* r, double* updates, double* sol, hipStream_t st, const double* skip = nullptr);

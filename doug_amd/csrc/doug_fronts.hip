@@ -1094,25 +1094,20 @@ static int front_solve_lds(int nw, int maxwork) {
 }
 
 template <typename T>
-void prepare_front_solve(int nw, int maxwork) {
-  const int bytes = front_solve_lds<T>(nw, maxwork);
-  if (bytes <= 64 * 1024) return;
-  auto allow = [bytes](auto kernel) {
-    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
+hipError_t prepare_front_solve() {
+  auto allow = [](auto... kernels) {
+    hipError_t first = hipSuccess;
+    for (hipError_t e : {allow_lds(kernels, kLdsBytes)...})
+      if (first == hipSuccess) first = e;
+    return first;
   };
-  if constexpr (sizeof(T) == 8) {
-    allow(&k_front_solve_mma<8, kWhole>);
-    allow(&k_front_solve_mma<16, kWhole>);
-    allow(&k_front_solve_mma<16, kSubtreesForward>);
-    allow(&k_front_solve_mma<16, kApex>);
-    allow(&k_front_solve_mma<16, kSubtreesBackward>);
-  } else {
-    allow(&k_front_solve<8, kWhole>);
-    allow(&k_front_solve<16, kWhole>);
-    allow(&k_front_solve<16, kSubtreesForward>);
-    allow(&k_front_solve<16, kApex>);
-    allow(&k_front_solve<16, kSubtreesBackward>);
-  }
+  if constexpr (sizeof(T) == 8)
+    return allow(&k_front_solve_mma<8, kWhole>, &k_front_solve_mma<16, kWhole>,
+                 &k_front_solve_mma<16, kSubtreesForward>, &k_front_solve_mma<16, kApex>,
+                 &k_front_solve_mma<16, kSubtreesBackward>);
+  else
+    return allow(&k_front_solve<8, kWhole>, &k_front_solve<16, kWhole>, &k_front_solve<16, kSubtreesForward>,
+                 &k_front_solve<16, kApex>, &k_front_solve<16, kSubtreesBackward>);
 }
 
 template <typename T>
@@ -1147,7 +1142,7 @@ void launch_front_solve(const T* tiles, const FrontSub* subs, int nsub, int nw, 
                                         const int32_t*, const int32_t*, const int32_t*, const double*,          \
                                         hipStream_t);                                                           \
   template void launch_front_factor<T>(T*, T*, const FrontSub*, int, int, int, bool, int*, hipStream_t);        \
-  template void prepare_front_solve<T>(int, int);                                                                   \
+  template hipError_t prepare_front_solve<T>();                                                                 \
   template void launch_front_solve<T>(const T*, const FrontSub*, int, int, int, int, const int32_t*,            \
                                       const double*, double*, double*, hipStream_t, const double*);
 DOUG_INSTANTIATE_FRONTS(double)

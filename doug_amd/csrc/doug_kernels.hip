@@ -2329,11 +2329,8 @@ void launch_map_index(int32_t* idx, int64_t n, const int32_t* map, hipStream_t s
 }
 
 template <typename T>
-void prepare_trsv(int maxnt) {
-  const int bytes = maxnt * kTile * (int)sizeof(T);
-  if (bytes > 64 * 1024)
-    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&k_trsv<T>),
-                              hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
+hipError_t prepare_trsv() {
+  return allow_lds(k_trsv<T>, kMaxTrsvTiles * kTile * (int)sizeof(T));
 }
 
 template <typename T>
@@ -2354,7 +2351,7 @@ void launch_trsv(const T* tiles, const BlockDesc* d, int nblocks, int maxnt, con
   template void launch_chol_offdiag<T>(T*, const BlockDesc*, int, int, int, hipStream_t, bool); \
   template void launch_trsv<T>(const T*, const BlockDesc*, int, int, const int32_t*,          \
                                const double*, double*, hipStream_t, const double*);           \
-  template void prepare_trsv<T>(int);
+  template hipError_t prepare_trsv<T>();
 DOUG_INSTANTIATE(double)
 DOUG_INSTANTIATE(float)
 #undef DOUG_INSTANTIATE

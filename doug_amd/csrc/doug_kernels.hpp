@@ -9,6 +9,7 @@ constexpr int kTile = 64;              // dense tile edge (one wavefront wide)
 constexpr int kTileElems = kTile * kTile;
 constexpr int kSpmvThreads = 256;      // CSR-stream block
 constexpr int kSpmvChunk = 2048;       // products staged in LDS per block
+constexpr int kLdsBytes = 160 * 1024;   // of a CU, all of which a workgroup may take
 constexpr int kMaxTrsvTiles = 256;     // subdomain size limit of the one-block solve (16384)
 constexpr int kRedBlocks = 1024;       // fixed partial count of the grid reductions
 constexpr int kRedBlocksWide = 8192;   // grid of the column-pair reductions (partials per column)
@@ -121,9 +122,9 @@ void launch_spmv(int nblocks_rows, const int32_t* rowblk, const int32_t* ptr, co
 // r(inds), solves L L^T u = r in the factor's precision, writes u to sol
 // (FP64, concatenated layout).
 // maxnt: the largest block's tile count (sets the dynamic LDS); call
-// prepare_trsv<T>(maxnt) once before the first launch for that size.
+// prepare_trsv<T>() once before the first launch on a device.
 template <typename T>
-void prepare_trsv(int maxnt);
+hipError_t prepare_trsv();
 template <typename T>
 // skip (device, optional): the launch does nothing when *skip != 0.
 void launch_trsv(const T* tiles, const BlockDesc* d, int nblocks, int maxnt, const int32_t* inds,

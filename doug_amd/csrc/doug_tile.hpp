@@ -55,5 +55,13 @@ __device__ __forceinline__ int local_col(const int32_t* __restrict__ occ_ptr,
   return -1;
 }
 
+// Lets a kernel's workgroups take this much dynamic LDS: the most that any
+// launch may ask for, since the limit belongs to the kernel and one context's
+// need would take away another's.
+template <typename K>
+hipError_t allow_lds(K* kernel, int bytes) {
+  return hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
+}
+
 }  // namespace
 }  // namespace doug

@@ -120,7 +120,8 @@ def _diffusion_order(N: int, device) -> torch.Tensor:
     """_diffusion_pattern's sort permutation, formed on `device`: a row's
     entries ascend from its -x neighbour over -y, -z, itself, +z and +y to +x,
     so each place follows from the cell (0.3 ms at N = 64 where sorting the
-    entries on the host took 19 ms)."""
+    entries on the host took 19 ms).  No shape depends on a value, so that it
+    runs on fake and meta tensors and waits for nothing."""
     c = torch.arange(N, device=device)
     x, y, z = c.view(N, 1, 1), c.view(1, N, 1), c.view(1, 1, N)
     m = N * N * (N - 1)  # faces of an axis, listed low to high and high to low
@@ -129,8 +130,11 @@ def _diffusion_order(N: int, device) -> torch.Tensor:
     place = [(m + fx - N * N, low.view(N, 1, 1)), (3 * m + fy - N, low.view(1, N, 1)),
              (5 * m + fz - 1, low.view(1, 1, N)), (6 * m + fx, one), (4 * m + fz, high.view(1, 1, N)),
              (2 * m + fy, high.view(1, N, 1)), (fx, high.view(N, 1, 1))]
-    at = torch.stack([p for p, _ in place], dim=-1)
-    return at[torch.stack([k.expand(N, N, N) for _, k in place], dim=-1)]
+    there = torch.stack([k.expand(N, N, N) for _, k in place], dim=-1).flatten()
+    count = 7 * N ** 3 - 6 * N * N
+    order = torch.empty(count + 1, dtype=torch.int64, device=device)  # the last for entries that do not exist
+    order[torch.where(there, there.cumsum(0) - 1, count)] = torch.stack([p for p, _ in place], dim=-1).flatten()
+    return order[:count]
 
 
 def diffusion3d_values(theta: torch.Tensor, N: int) -> torch.Tensor:

@@ -1839,6 +1839,20 @@ static int setup_host(doug_ctx* ctx) {
   return DOUG_OK;
 }
 
+// What each subdomain's solve streams: panel entries of its fronts, or its
+// envelope's tile rows.
+static std::vector<int64_t> solve_sizes(const doug_ctx* ctx) {
+  std::vector<int64_t> size;
+  if (ctx->fronts) {
+    for (size_t b = 0; b < ctx->h_fsub.size(); b++)
+      size.push_back((b + 1 < ctx->h_fsub.size() ? ctx->h_fsub[b + 1].base : ctx->factor_elems) -
+                     ctx->h_fsub[b].base);
+  } else {
+    for (const BlockDesc& d : ctx->h_sub) size.push_back(d.nt);
+  }
+  return size;
+}
+
 // Dispatch order of the subdomain solves: 0 as partitioned, 1 largest first
 // (longest-processing-time order, which shortens the tail when sizes vary).
 static int set_trsv_order(doug_ctx* ctx, int order) {
@@ -1846,11 +1860,9 @@ static int set_trsv_order(doug_ctx* ctx, int order) {
   ctx->d_sub_trsv = ctx->d_sub;
   ctx->d_fsub_solve = ctx->d_fsub;
   if (order == 1 && ctx->fronts) {
-    std::vector<int64_t> size(ctx->h_fsub.size());
-    std::vector<int> by((size_t)ctx->h_fsub.size());
+    const std::vector<int64_t> size = solve_sizes(ctx);
+    std::vector<int> by(size.size());
     std::iota(by.begin(), by.end(), 0);
-    for (size_t b = 0; b < size.size(); b++)
-      size[b] = (b + 1 < size.size() ? ctx->h_fsub[b + 1].base : ctx->factor_elems) - ctx->h_fsub[b].base;
     std::stable_sort(by.begin(), by.end(), [&](int a, int b) { return size[a] > size[b]; });
     std::vector<FrontSub> sorted;
     for (int b : by) sorted.push_back(ctx->h_fsub[b]);
@@ -3464,11 +3476,8 @@ int doug_autotune(doug_ctx* ctx, int32_t reps, doug_tuning* out) {
     if ((rc = set_trsv_order(ctx, 0)) ||
         (rc = time_launches(ctx, rt, [&]() { enqueue_subdomain_solves(ctx, ctx->d_r); }, &tu.trsv_ms[0])))
       return rc;
-    bool sorted = true;
-    for (int i = 1; i < ctx->nsub; i++)
-      sorted = sorted && (ctx->fronts ? ctx->h_fsub[i - 1].n >= ctx->h_fsub[i].n
-                                      : ctx->h_sub[i - 1].nt >= ctx->h_sub[i].nt);
-    if (!sorted) {
+    const std::vector<int64_t> size = solve_sizes(ctx);
+    if (!std::is_sorted(size.rbegin(), size.rend())) {
       if ((rc = set_trsv_order(ctx, 1)) ||
           (rc = time_launches(ctx, rt, [&]() { enqueue_subdomain_solves(ctx, ctx->d_r); }, &tu.trsv_ms[1])))
         return rc;

@@ -147,6 +147,7 @@ struct doug_ctx {
   BlockDesc* d_sub = nullptr;
   std::vector<BlockDesc> h_sub;
   int trsv_order = 0;               // 1: largest subdomain dispatched first
+  int batch_order = 0;              // the same for a batch with factors of its own (beside fronts)
   int trsm_kb = 2;                  // tiles per step of the batched envelope solve
   int trsm_cg = 1;                  // column layout of that solve (1..3, DOUG_OPT_BATCH_COLUMN_GROUPS)
   int local_order = 1;              // 1: reverse Cuthill-McKee inside each subdomain
@@ -1853,13 +1854,13 @@ static std::vector<int64_t> solve_sizes(const doug_ctx* ctx) {
   return size;
 }
 
-// Dispatch order of the subdomain solves: 0 as partitioned, 1 largest first
-// (longest-processing-time order, which shortens the tail when sizes vary).
-static int set_trsv_order(doug_ctx* ctx, int order) {
-  ctx->trsv_order = order;
+// The subdomains' descriptors in the chosen dispatch orders: 0 as partitioned,
+// 1 largest first (longest-processing-time order, which shortens the tail when
+// sizes vary).
+static int apply_orders(doug_ctx* ctx) {
   ctx->d_sub_trsv = ctx->d_sub;
   ctx->d_fsub_solve = ctx->d_fsub;
-  if (order == 1 && ctx->fronts) {
+  if (ctx->trsv_order == 1 && ctx->fronts) {
     const std::vector<int64_t> size = solve_sizes(ctx);
     std::vector<int> by(size.size());
     std::iota(by.begin(), by.end(), 0);
@@ -1870,7 +1871,7 @@ static int set_trsv_order(doug_ctx* ctx, int order) {
     if (rc) return rc;
     HIPCHK(hipStreamSynchronize(ctx->stream));  // `sorted` goes out of scope
   }
-  if (order == 0 || ctx->h_sub.empty()) return DOUG_OK;
+  if ((ctx->fronts ? ctx->batch_order : ctx->trsv_order) == 0 || ctx->h_sub.empty()) return DOUG_OK;
   std::vector<BlockDesc> sorted(ctx->h_sub);
   std::stable_sort(sorted.begin(), sorted.end(),
                    [](const BlockDesc& a, const BlockDesc& b) { return a.nt > b.nt; });
@@ -1878,6 +1879,11 @@ static int set_trsv_order(doug_ctx* ctx, int order) {
   if (rc) return rc;
   HIPCHK(hipStreamSynchronize(ctx->stream));  // `sorted` goes out of scope
   return DOUG_OK;
+}
+
+static int set_trsv_order(doug_ctx* ctx, int order) {
+  ctx->trsv_order = ctx->batch_order = order;
+  return apply_orders(ctx);
 }
 
 // Matrix, vectors, subdomain data and the subdomain factorisation (enqueued).
@@ -2228,7 +2234,7 @@ static int device_fine(doug_ctx* ctx, hipEvent_t ev0, hipEvent_t ev1) {
   info.factor_bytes = elems * (int64_t)esize;
   info.factor_tiles = (elems + kTileElems - 1) / kTileElems;
   ctx->factor_elems = elems;
-  if ((rc = set_trsv_order(ctx, ctx->trsv_order))) return rc;
+  if ((rc = apply_orders(ctx))) return rc;
   if (ctx->fronts)
     HIPCHK(ctx->precision == DOUG_PREC_FP32_FACTORS ? prepare_front_solve<float>() : prepare_front_solve<double>());
   return DOUG_OK;
@@ -3048,7 +3054,7 @@ static int batch_factors(doug_ctx* ctx) {
   rc = ctx->precision == DOUG_PREC_FP32_FACTORS
            ? envelope_factors(ctx, dinds, ctx->batch_lists, host_map, &ctx->d_btiles32, &elems, nullptr, nullptr, d_flag)
            : envelope_factors(ctx, dinds, ctx->batch_lists, host_map, &ctx->d_btiles, &elems, nullptr, nullptr, d_flag);
-  if (rc || (rc = set_trsv_order(ctx, ctx->trsv_order))) return rc;
+  if (rc || (rc = apply_orders(ctx))) return rc;
   HIPCHK(hipMemcpyAsync(&flag, d_flag, sizeof(int), hipMemcpyDeviceToHost, ctx->stream));
   HIPCHK(hipStreamSynchronize(ctx->stream));
   if (flag) return fail(ctx, DOUG_E_NUMERIC, "subdomain " + std::to_string(flag - 1) + " is not positive definite");
@@ -3357,7 +3363,7 @@ int doug_set_option(doug_ctx* ctx, int32_t option, int64_t value) {
     case DOUG_OPT_TRSV_ORDER:
       if (value != 0 && value != 1) return fail(ctx, DOUG_E_ARG, "subdomain order must be 0 or 1");
       if (!ctx->ready) {
-        ctx->trsv_order = (int)value;
+        ctx->trsv_order = ctx->batch_order = (int)value;
         return DOUG_OK;
       }
       drop_iteration_graph(ctx);
@@ -3508,6 +3514,21 @@ int doug_autotune(doug_ctx* ctx, int32_t reps, doug_tuning* out) {
   }
   ctx->trsm_kb = kb;
   ctx->trsm_cg = cg;
+  bool uneven = false;
+  for (size_t b = 1; b < ctx->h_sub.size(); b++) uneven = uneven || ctx->h_sub[b - 1].nt < ctx->h_sub[b].nt;
+  if (ctx->batch_ready && ctx->fronts && uneven) {
+    // the order above is the fronts': the batch's envelopes are timed by themselves
+    const int rt = std::max(2, reps / 8);
+    double ms[2];
+    for (int o = 0; o < 2; o++) {
+      ctx->batch_order = o;
+      if ((rc = apply_orders(ctx)) ||
+          (rc = time_launches(ctx, rt, [&]() { enqueue_prec_multi(ctx, kMaxRhs, ctx->d_Rm, ctx->d_Zm); }, &ms[o])))
+        return rc;
+    }
+    ctx->batch_order = ms[1] < ms[0] ? 1 : 0;
+    if ((rc = apply_orders(ctx))) return rc;
+  }
   tu.trsm_col_groups = cg;
   HIPCHK(hipStreamSynchronize(ctx->stream));
   tu.trsm_tiles_per_step = kb;

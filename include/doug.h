@@ -269,7 +269,8 @@ int doug_time_operator(doug_ctx *ctx, int32_t which, int32_t reps, double *ms);
  * every SpMV shape -- 128, 256 or 512 rows per workgroup, each with and
  * without XCD-contiguous block order --, the dispatch order of the
  * subdomain solves (as partitioned, or largest first when sizes differ) and,
- * after doug_prepare_batch, the tiles per step of the batched solve,
+ * after doug_prepare_batch, the tiles per step of the batched solve and its
+ * own dispatch order (not reported) where it has factors of its own,
  * `reps` launches each (<= 0: 20), and keeps the fastest.  All choices give
  * bit-identical results.  The choice stays with the context across later
  * doug_setup calls.  `out` may be NULL. */

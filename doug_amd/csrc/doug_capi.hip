@@ -2658,7 +2658,7 @@ static void enqueue_prec(doug_ctx* ctx, const double* r, double* z, const PrecWo
   const Params& p = ctx->p;
   if (p.method == 0) {
     launch_copy(z, r, ctx->n, ctx->stream);
-    if (dot) launch_dot(r, z, ctx->n, ctx->d_partial, nullptr, 1, ctx->d_scal, ctx->stream);
+    if (dot) launch_dot(r, z, ctx->n, ctx->d_partial, 1, ctx->d_scal, ctx->stream);
     return;
   }
   // prec2Level_solve (pcg.F90:191-208) with several processes, where the
@@ -2900,7 +2900,7 @@ static int pcg_core(doug_ctx* ctx, double tol, int maxit, int32_t* it_out, doubl
   // r = b - A x
   enqueue_spmv(ctx, ctx->d_x, ctx->d_tmp);
   launch_residual(n, ctx->d_b, ctx->d_tmp, ctx->d_r, st);
-  launch_dot(ctx->d_r, ctx->d_r, n, ctx->d_partial, nullptr, 3, ctx->d_scal, st);
+  launch_dot(ctx->d_r, ctx->d_r, n, ctx->d_partial, 3, ctx->d_scal, st);
   HIPCHK(hipMemcpyAsync(scal, ctx->d_scal, S_N * sizeof(double), hipMemcpyDeviceToHost, st));
   HIPCHK(hipStreamSynchronize(st));
   double init_norm = scal[S_RES];
@@ -2932,7 +2932,7 @@ static int pcg_core(doug_ctx* ctx, double tol, int maxit, int32_t* it_out, doubl
     const int nrho = (n - 1) / (ctx->p.method == 0 ? kVecChunk : 256) + 1;
     launch_p_update(n, ctx->d_z, ctx->d_p, ctx->d_scal, first ? 1 : 0, ctx->d_partial, nrho, st);
     enqueue_spmv(ctx, ctx->d_p, ctx->d_q);
-    launch_dot(ctx->d_p, ctx->d_q, n, ctx->d_partial, nullptr, 2, ctx->d_scal, st);
+    launch_dot(ctx->d_p, ctx->d_q, n, ctx->d_partial, 2, ctx->d_scal, st);
     launch_xr_update(n, ctx->d_x, ctx->d_r, ctx->d_p, ctx->d_q, ctx->d_partial, ctx->d_scal, st, ctx->d_hist);
   };
   hipEvent_t ev[2] = {nullptr, nullptr};

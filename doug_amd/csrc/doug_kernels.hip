@@ -899,8 +899,8 @@ __device__ __forceinline__ double block_sum(double v, double* sh) {
 // The second stage of the single-vector reductions: one workgroup sums the
 // `count` workgroup partials (thread t takes t, t + 1024, ... in order, each
 // wavefront's by a butterfly, the 16 wavefronts' in order) and applies the
-// scalar recurrence of `mode`: 0 the sum to out,
-// 1 rho = r.z with beta, 2 p.q with alpha, 3 the squared residual norm.
+// scalar recurrence of `mode`: 1 rho = r.z with beta, 2 p.q with alpha, 3 the
+// squared residual norm.
 // Mode 3 with out (a PCG iteration's residual) also keeps the iteration on
 // the device: unless S_DONE is set, it counts the iteration in S_ITER,
 // writes (alpha, beta, residual) to out[3(it-1)..] for it <= S_HCAP, and
@@ -920,9 +920,7 @@ __global__ __launch_bounds__(1024) void k_reduce_finish(const double* __restrict
   if (t == 0) {
     double s = 0.0;
     for (int k = 0; k < 16; k++) s += sh[k];
-    if (mode == 0) {
-      out[0] = s;
-    } else if (mode == 1) {  // rho = r.z
+    if (mode == 1) {  // rho = r.z
       scal[S_BETA] = s / scal[S_RHO];
       scal[S_RHO_PREV] = scal[S_RHO];
       scal[S_RHO] = s;
@@ -2585,12 +2583,11 @@ void launch_overlap_sum(int n, const int32_t* occ_ptr, const int32_t* occ_pos, c
 // both sums' partials fit (r.z has one per 256 unknowns, p.q one per 1024)
 static bool folds(int n) { return cdiv(n, 256) <= kFoldPartials; }
 
-void launch_dot(const double* a, const double* b, int n, double* partial, double* out, int mode,
-                double* scal, hipStream_t st) {
+void launch_dot(const double* a, const double* b, int n, double* partial, int mode, double* scal, hipStream_t st) {
   const int nb = (int)cdiv(n, kVecChunk);
   hipLaunchKernelGGL(k_dot_chunks, dim3(nb), dim3(256), 0, st, a, b, n, partial);
   if (mode != 3 && folds(n)) return;
-  hipLaunchKernelGGL(k_reduce_finish, dim3(1), dim3(1024), 0, st, partial, nb, out, mode, scal);
+  hipLaunchKernelGGL(k_reduce_finish, dim3(1), dim3(1024), 0, st, partial, nb, nullptr, mode, scal);
 }
 
 void launch_p_update(int n, const double* z, double* p, double* scal, int first, const double* partial,

@@ -190,11 +190,11 @@ void launch_overlap_sum_dot(int n, const int32_t* occ_ptr, const int32_t* occ_po
 // ---- PCG vector kernels with deterministic two-level reductions ----
 // scal layout (device doubles): see doug_capi.hip.  `partial` holds
 // vec_partials(n) doubles.
-void launch_dot(const double* a, const double* b, int n, double* partial, double* out, int mode,
-                double* scal, hipStream_t st);
-// Up to 256 kFoldPartials unknowns launch_dot (modes 1 and 2) and
-// launch_overlap_sum_dot leave their sums to this (of the `count` partials of
-// r.z) and to launch_xr_update.
+// The PCG's sum of `mode` into scal: 1 rho = r.z with beta, 2 p.q with alpha, 3
+// the squared residual norm.  Modes 1 and 2 (and launch_overlap_sum_dot) only
+// begin it up to 256 kFoldPartials unknowns: their partials stay in `partial`
+// for launch_p_update (`count` of them) and launch_xr_update, which follow.
+void launch_dot(const double* a, const double* b, int n, double* partial, int mode, double* scal, hipStream_t st);
 void launch_p_update(int n, const double* z, double* p, double* scal, int first, const double* partial,
                      int count, hipStream_t st);
 // With hist, the residual's finish keeps the iteration count, the

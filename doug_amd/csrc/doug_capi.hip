@@ -2171,10 +2171,8 @@ static int device_fine(doug_ctx* ctx, hipEvent_t ev0, hipEvent_t ev1) {
     while (2 * ctx->front_groups * ctx->nsub <= 256 && ctx->front_groups < kFrontGroupsMax)
       ctx->front_groups *= 2;
     const int units = f32 ? kFrontUnitGroups32 : kFrontUnitGroups64;
-    for (; sizes && !ctx->fronts && ctx->front_groups > 0; ctx->front_groups /= 2)
-      if ((ctx->fronts = build_front_patterns(A, ctx->sstarts, ctx->sinds, max_work, ctx->front_nw, ctx->front_groups,
-                                              units, pats, pat, dinds)))
-        break;
+    ctx->fronts = sizes && build_front_patterns(A, ctx->sstarts, ctx->sinds, max_work, ctx->front_nw, ctx->front_groups,
+                                                units, pats, pat, dinds, &ctx->front_groups);
     if (!ctx->fronts) block_rcm(A, ctx->sstarts, ctx->sinds, dinds, &ctx->rank_ws);
   } else {
     dinds = ctx->sinds;

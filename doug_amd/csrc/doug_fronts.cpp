@@ -7,6 +7,7 @@
 #include "doug_fronts.hpp"
 
 #include <algorithm>
+#include <atomic>
 #include <cstring>
 #include <memory>
 #include <mutex>
@@ -327,17 +328,26 @@ struct ItemLists {
   }
 };
 
-bool make_pattern(const Graph& g, int64_t max_work, int nw, int groups, int ug, FrontPattern& P) {
-  const int n = g.n(), nwb = nw * groups;  // nwb wavefronts for the bottom subtrees
-  P.n = n;
-  P.groups = groups;
+// The fronts of a graph in postorder and their boundary rows (in postorder
+// positions), whatever the work vector and the number of workgroups.
+struct Tree {
+  std::vector<int> listed;  // position -> node
+  std::vector<Front> fronts;
+  std::vector<int> parent;
+  std::vector<std::vector<uint16_t>> rows;
+};
+
+// False where a front or the graph exceeds the format.
+bool make_tree(const Graph& g, Tree& T) {
+  const int n = g.n();
+  if (n > 65535) return false;
   Dissector D(g);
   D.run(0, n, 0);
   // fronts in postorder, at most kFrontCols columns each: a longer separator
   // becomes a chain, cut into equal pieces
   std::vector<int> part_front(D.parts.size(), -1);  // last front of each part
-  std::vector<int> parent;
-  std::vector<Front>& F = P.fronts;
+  std::vector<int>& parent = T.parent;
+  std::vector<Front>& F = T.fronts;
   for (size_t q = 0; q < D.parts.size(); q++) {
     const Part& p = D.parts[q];
     int kid[2] = {-1, -1}, nk = 0;
@@ -359,13 +369,14 @@ bool make_pattern(const Graph& g, int64_t max_work, int nw, int groups, int ug, 
     part_front[q] = (int)F.size() - 1;
   }
   const int nf = (int)F.size();
-  if (nf > 65535 || n > 65535) return false;
+  if (nf > 65535) return false;
   // boundary rows in postorder positions: the children's and the columns'
   // later neighbours, as bit sets
   std::vector<int> pos((size_t)n);
   for (int p = 0; p < n; p++) pos[D.listed[p]] = p;
   const int words = (n + 63) / 64;
-  std::vector<std::vector<uint16_t>> rows((size_t)nf);
+  std::vector<std::vector<uint16_t>>& rows = T.rows;
+  rows.resize((size_t)nf);
   std::vector<uint64_t> bits((size_t)words);
   for (int f = 0; f < nf; f++) {
     const int c0 = F[f].c0, c1 = c0 + F[f].k;
@@ -389,6 +400,22 @@ bool make_pattern(const Graph& g, int64_t max_work, int nw, int groups, int ug, 
     F[f].m = (uint16_t)rows[f].size();
     if ((int)F[f].k + F[f].m > 64 * 250) return false;
   }
+  T.listed.swap(D.listed);
+  return true;
+}
+
+// The pattern of `groups` workgroups of nw wavefronts; false where its work
+// vector or panels do not fit.
+bool make_pattern(const Tree& T, int64_t max_work, int nw, int groups, int ug, FrontPattern& P) {
+  P = FrontPattern{};
+  const int n = (int)T.listed.size(), nwb = nw * groups;  // nwb wavefronts for the bottom subtrees
+  P.n = n;
+  P.groups = groups;
+  P.fronts = T.fronts;
+  std::vector<Front>& F = P.fronts;
+  const int nf = (int)F.size();
+  const std::vector<int>& parent = T.parent;
+  const std::vector<std::vector<uint16_t>>& rows = T.rows;
   std::vector<int64_t> cost((size_t)nf);
   for (int f = 0; f < nf; f++) {
     cost[f] = front_cost(F[f], ug);
@@ -486,7 +513,7 @@ bool make_pattern(const Graph& g, int64_t max_work, int nw, int groups, int ug, 
       for (int c = 0; c < f.k; c++) {
         newpos[f.c0 + c] = at;
         P.colfront[at] = (uint16_t)q;
-        P.order[at++] = D.listed[f.c0 + c];
+        P.order[at++] = T.listed[f.c0 + c];
       }
     }
     if (nbottom == nf) P.top0 = n;
@@ -744,65 +771,80 @@ int64_t front_entry(const FrontPattern& p, int lo, int hi, bool dbl) {
 bool build_front_patterns(const Csr& A, const std::vector<int>& starts, const std::vector<int>& inds,
                           int64_t max_work, int nw, int groups, int ug,
                           std::vector<FrontPattern>& patterns, std::vector<int>& pat,
-                          std::vector<int>& out) {
-  const int nb = (int)starts.size() - 1;
+                          std::vector<int>& out, int* chosen) {
+  const int nb = (int)starts.size() - 1, least = chosen ? 1 : groups;
   pat.assign((size_t)nb, -1);
   out.resize(inds.size());
   // the first block of a graph makes the pattern, the others of the same
   // graph (compared entry by entry) share it
   struct Known {
     Graph g;
+    Tree t;
     FrontPattern p;
   };
   std::vector<std::unique_ptr<Known>> known;
-  std::unordered_multimap<uint64_t, int> by_hash;
+  std::unordered_map<uint64_t, std::vector<int>> by_hash;
   std::mutex mu;
   bool ok = true;
+  int limit = groups;  // workgroups that suit every pattern so far
   const int nth = std::max(1, std::min(setup_threads(), nb));
-  {
+  auto parallel = [&](auto&& f) {
     std::vector<std::thread> th;
-    for (int t = 0; t < nth; t++)
-      th.emplace_back([&, t]() {
-        std::vector<int> floc((size_t)A.nrows, -1);
-        Graph g;
-        for (int b = t; b < nb; b += nth) {
-          const int s0 = starts[b], s = starts[b + 1] - s0;
-          const uint64_t h = local_graph(A, inds.data() + s0, s, floc.data(), g);
-          Known* mine = nullptr;
-          {
-            std::lock_guard<std::mutex> lk(mu);
-            if (!ok) return;
-            auto range = by_hash.equal_range(h);
-            for (auto it = range.first; it != range.second && pat[b] < 0; ++it)
-              if (known[it->second]->g.ptr == g.ptr && known[it->second]->g.adj == g.adj) pat[b] = it->second;
-            if (pat[b] < 0) {
-              pat[b] = (int)known.size();
-              known.emplace_back(new Known{g, {}});
-              by_hash.emplace(h, pat[b]);
-              mine = known.back().get();
-            }
-          }
-          if (mine && !make_pattern(mine->g, max_work, nw, groups, ug, mine->p)) {
-            std::lock_guard<std::mutex> lk(mu);
-            ok = false;
-            return;
-          }
-        }
-      });
+    for (int t = 0; t < nth; t++) th.emplace_back(f, t);
     for (auto& x : th) x.join();
+  };
+  parallel([&](int t) {
+    std::vector<int> floc((size_t)A.nrows, -1);
+    Graph g;
+    for (int b = t; b < nb; b += nth) {
+      const int s0 = starts[b], s = starts[b + 1] - s0;
+      const uint64_t h = local_graph(A, inds.data() + s0, s, floc.data(), g);
+      Known* mine = nullptr;
+      int count;
+      {
+        std::lock_guard<std::mutex> lk(mu);
+        if (!ok) return;
+        std::vector<int>& like = by_hash[h];
+        for (size_t k = 0; k < like.size() && pat[b] < 0; k++)
+          if (known[like[k]]->g.ptr == g.ptr && known[like[k]]->g.adj == g.adj) pat[b] = like[k];
+        if (pat[b] < 0) {
+          pat[b] = (int)known.size();
+          like.push_back(pat[b]);
+          known.emplace_back(new Known{g, {}, {}});
+          mine = known.back().get();
+        }
+        count = limit;
+      }
+      if (!mine) continue;
+      bool fits = make_tree(mine->g, mine->t);
+      while (fits && !(fits = make_pattern(mine->t, max_work, nw, count, ug, mine->p)) && count > least)
+        fits = true, count /= 2;
+      std::lock_guard<std::mutex> lk(mu);
+      ok = ok && fits;
+      limit = std::min(limit, count);
+    }
+  });
+  // the others follow the one that takes the fewest workgroups
+  for (; ok; limit /= 2) {
+    std::atomic<int> next{0};
+    std::atomic<bool> fits{true};
+    parallel([&](int) {
+      for (int k = next++; k < (int)known.size() && fits; k = next++)
+        if (known[k]->p.groups != limit && !make_pattern(known[k]->t, max_work, nw, limit, ug, known[k]->p)) fits = false;
+    });
+    if (fits) break;
+    ok = limit > least;
   }
   if (!ok) return false;
+  if (chosen) *chosen = limit;
   patterns.clear();
   for (auto& k : known) patterns.push_back(std::move(k->p));
-  std::vector<std::thread> th;
-  for (int t = 0; t < nth; t++)
-    th.emplace_back([&, t]() {
-      for (int b = t; b < nb; b += nth) {
-        const std::vector<int32_t>& o = patterns[pat[b]].order;
-        for (size_t p = 0; p < o.size(); p++) out[starts[b] + p] = inds[starts[b] + o[p]];
-      }
-    });
-  for (auto& x : th) x.join();
+  parallel([&](int t) {
+    for (int b = t; b < nb; b += nth) {
+      const std::vector<int32_t>& o = patterns[pat[b]].order;
+      for (size_t p = 0; p < o.size(); p++) out[starts[b] + p] = inds[starts[b] + o[p]];
+    }
+  });
   return true;
 }
 

@@ -111,10 +111,13 @@ int64_t front_entry(const FrontPattern& p, int lo, int hi, bool dbl);
 // elimination order.  False, with nothing usable, when some subdomain's
 // structure exceeds the format (work indices of 16 bits, `max_work` entries
 // of work vector, panel offsets of 31 bits).  nw wavefronts per workgroup,
-// `groups` workgroups for the subtrees, ug column groups per unit.
+// `groups` workgroups for the subtrees, ug column groups per unit.  With
+// `chosen`, half as many workgroups for all, a quarter and so on down to one
+// where `groups` do not fit: the dissections, nearly all of the work, serve
+// each try.
 bool build_front_patterns(const Csr& A, const std::vector<int>& starts, const std::vector<int>& inds,
                           int64_t max_work, int nw, int groups, int ug,
                           std::vector<FrontPattern>& patterns, std::vector<int>& pat,
-                          std::vector<int>& out);
+                          std::vector<int>& out, int* chosen = nullptr);
 
 }  // namespace doug

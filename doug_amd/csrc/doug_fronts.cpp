@@ -819,6 +819,7 @@ bool build_front_patterns(const Csr& A, const std::vector<int>& starts, const st
       bool fits = make_tree(mine->g, mine->t);
       while (fits && !(fits = make_pattern(mine->t, max_work, nw, count, ug, mine->p)) && count > least)
         fits = true, count /= 2;
+      if (count == least) mine->t = Tree{};  // nothing smaller will be asked for
       std::lock_guard<std::mutex> lk(mu);
       ok = ok && fits;
       limit = std::min(limit, count);

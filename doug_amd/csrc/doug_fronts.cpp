@@ -58,16 +58,17 @@ struct Dissector {
   }
 
   // breadth-first order from root inside part `id`; lev holds the starts of
-  // its levels and the end
+  // its levels and the end.  What is found loses its label until the end: one
+  // array to look up for each edge (a mark beside the label, without branches,
+  // took 1.4 times as long).
   int search(int root, int id) {
     ++stamp;
     int* q = bfs.data();
-    int* mk = mark.data();
-    const int* lb = lab.data();
+    int* lb = lab.data();
     const int* ptr = g.ptr.data();
     const int* adj = g.adj.data();
     q[0] = root;
-    mk[root] = stamp;
+    lb[root] = -2;
     int b = 0, top = 1;
     lev.clear();
     lev.push_back(0);
@@ -77,15 +78,19 @@ struct Dissector {
         const int v = q[k];
         for (int p = ptr[v]; p < ptr[v + 1]; p++) {
           const int u = adj[p];
-          const int fresh = (mk[u] != stamp) & (lb[u] == id);
-          q[top] = u;
-          top += fresh;
-          mk[u] = fresh ? stamp : mk[u];
+          if (lb[u] == id) {
+            lb[u] = -2;
+            q[top++] = u;
+          }
         }
       }
       lev.push_back(e);
       if (top == e) break;
       b = e;
+    }
+    for (int k = 0; k < top; k++) {
+      lb[q[k]] = id;
+      mark[q[k]] = stamp;
     }
     return top;
   }
@@ -98,12 +103,21 @@ struct Dissector {
     return (int)parts.size() - 1;
   }
 
-  // verts[b, e), all labelled `id`
-  int run(int b, int e, int id) {
+  // verts[b, e), all labelled `id`.  With `known`, the first `known` of them
+  // are what search(verts[b], id) finds, in its order, and lev holds its levels.
+  int run(int b, int e, int id, int known = 0) {
     const int n = e - b;
     if (n <= kLeaf) return leaf(b, e);
-    int reached = search(verts[b], id);
+    int reached = known;
+    if (known > 0) {
+      ++stamp;
+      std::copy(verts.begin() + b, verts.begin() + b + known, bfs.begin());
+      for (int k = 0; k < known; k++) mark[bfs[k]] = stamp;
+    } else {
+      reached = search(verts[b], id);
+    }
     int na = 0, nb = 0, nc = n;  // nc: nodes of the component to cut
+    int near = 0;                // nodes before the separator
     std::vector<int> sep, rest;
     comp.clear();
     if (reached < n) {
@@ -184,6 +198,11 @@ struct Dissector {
           verts[b + na++] = v;
       }
       for (int v : sep) lab[v] = -1;
+      // the nearer side's own search from the same root goes over the same
+      // levels, the last one without the separator
+      near = na;
+      lev.resize((size_t)best + 1);
+      if (near > l0) lev.push_back(near);
     }
     {  // the components that were not cut: the next one to the lighter side
       size_t at = 0;
@@ -203,7 +222,7 @@ struct Dissector {
     for (int k = b; k < b + na; k++) lab[verts[k]] = ia;
     for (int k = b + na; k < b + na + nb; k++) lab[verts[k]] = ib;
     const int mid = b + na, end = mid + nb;
-    const int ca = run(b, mid, ia), cb = nb > 0 ? run(mid, end, ib) : -1;
+    const int ca = run(b, mid, ia, near), cb = nb > 0 ? run(mid, end, ib) : -1;
     std::sort(sep.begin(), sep.end());
     Part p{(int)listed.size(), (int)sep.size(), {ca, cb}};
     listed.insert(listed.end(), sep.begin(), sep.end());
@@ -707,9 +726,14 @@ bool make_pattern(const Tree& T, int64_t max_work, int nw, int groups, int ug, F
 
 // Local graph of block [s0, s0 + s): neighbours inside the block, without
 // self loops, symmetric (reverse edges are added where the matrix lacks
-// them); returns a hash of it.
-uint64_t local_graph(const Csr& A, const int* inds, int s, int* floc, Graph& g) {
-  for (int li = 0; li < s; li++) floc[inds[li]] = li;
+// them); returns a hash of it.  `floc` is scratch, -1 between calls: it spans
+// the block's numbers alone, which for a box of a grid is a small part of the
+// matrix's (a whole array per thread costs more page faults than work).
+uint64_t local_graph(const Csr& A, const int* inds, int s, std::vector<int>& floc, Graph& g) {
+  const int first = s > 0 ? *std::min_element(inds, inds + s) : 0;
+  const int span = s > 0 ? *std::max_element(inds, inds + s) - first + 1 : 0;  // floc[span]: outside
+  if (floc.size() <= (size_t)span) floc.assign((size_t)span + 1, -1);
+  for (int li = 0; li < s; li++) floc[inds[li] - first] = li;
   g.ptr.assign((size_t)s + 1, 0);
   size_t cap = 0;
   for (int li = 0; li < s; li++) cap += (size_t)(A.ptr[inds[li] + 1] - A.ptr[inds[li]]);
@@ -721,7 +745,7 @@ uint64_t local_graph(const Csr& A, const int* inds, int s, int* floc, Graph& g) 
   for (int li = 0; li < s; li++) {
     const int gi = inds[li], b = top;
     for (int p = A.ptr[gi]; p < A.ptr[gi + 1]; p++) {
-      const int lj = floc[col[p]];
+      const int lj = floc[std::min((unsigned)(col[p] - first), (unsigned)span)];
       adj[top] = lj;
       top += (lj >= 0) & (lj != li);
     }
@@ -734,7 +758,7 @@ uint64_t local_graph(const Csr& A, const int* inds, int s, int* floc, Graph& g) 
       hash = (hash ^ m) * 0x9e3779b97f4a7c15ull;
     }
   }
-  for (int li = 0; li < s; li++) floc[inds[li]] = -1;
+  for (int li = 0; li < s; li++) floc[inds[li] - first] = -1;
   g.adj.resize((size_t)top);
   if (fwd != rev) {  // unsymmetric structure: every edge in both directions
     Graph t;
@@ -794,26 +818,32 @@ bool build_front_patterns(const Csr& A, const std::vector<int>& starts, const st
     for (auto& x : th) x.join();
   };
   parallel([&](int t) {
-    std::vector<int> floc((size_t)A.nrows, -1);
+    std::vector<int> floc;
     Graph g;
     for (int b = t; b < nb; b += nth) {
       const int s0 = starts[b], s = starts[b + 1] - s0;
-      const uint64_t h = local_graph(A, inds.data() + s0, s, floc.data(), g);
+      const uint64_t h = local_graph(A, inds.data() + s0, s, floc, g);
       Known* mine = nullptr;
-      int count;
-      {
-        std::lock_guard<std::mutex> lk(mu);
-        if (!ok) return;
-        std::vector<int>& like = by_hash[h];
-        for (size_t k = 0; k < like.size() && pat[b] < 0; k++)
-          if (known[like[k]]->g.ptr == g.ptr && known[like[k]]->g.adj == g.adj) pat[b] = like[k];
-        if (pat[b] < 0) {
-          pat[b] = (int)known.size();
-          like.push_back(pat[b]);
-          known.emplace_back(new Known{g, {}, {}});
-          mine = known.back().get();
+      int count = 0;
+      for (size_t seen = 0; pat[b] < 0; seen++) {  // the graphs of this hash one by one, compared outside the lock
+        const Known* like = nullptr;
+        int at = 0;
+        {
+          std::lock_guard<std::mutex> lk(mu);
+          if (!ok) return;
+          std::vector<int>& all = by_hash[h];
+          if (seen < all.size()) {
+            at = all[seen];
+            like = known[at].get();
+          } else {
+            pat[b] = (int)known.size();
+            all.push_back(pat[b]);
+            known.emplace_back(new Known{std::move(g), {}, {}});
+            mine = known.back().get();
+            count = limit;
+          }
         }
-        count = limit;
+        if (like && like->g.ptr == g.ptr && like->g.adj == g.adj) pat[b] = at;
       }
       if (!mine) continue;
       bool fits = make_tree(mine->g, mine->t);

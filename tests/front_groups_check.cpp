@@ -1,6 +1,7 @@
 // build_front_patterns with a choice of workgroups: it takes the largest count
 // that fits every subdomain, with the patterns that this count gives when asked
-// for outright, and refuses where none fits.  Returns the number of failures.
+// for outright, and refuses where none fits; and its patterns do not depend on
+// the matrix's numbering.  Returns the number of failures.
 #include "doug_fronts.hpp"
 
 #include <algorithm>
@@ -106,6 +107,43 @@ int main() {
           bad++;
         }
       }
+  }
+  // other numbers for the nodes, in reverse and scattered over four times as
+  // many rows, leave the local graphs and so the patterns as they are
+  {
+    std::vector<int> starts;
+    const Csr A = boxes({{7, 8, 9}, {1, 1, 1}, {30, 21, 1}, {7, 8, 9}, {2, 3, 4}}, starts);
+    const int n = A.nrows;
+    std::vector<int> inds((size_t)n);
+    for (int i = 0; i < n; i++) inds[i] = i;
+    for (int way = 0; way < 2; way++) {
+      Csr B;
+      B.nrows = B.ncols = 4 * n;
+      std::vector<int> to((size_t)n), from((size_t)(4 * n), -1);
+      for (int i = 0; i < n; i++) to[i] = way == 0 ? 4 * n - 1 - i : (int)((int64_t)i * 1031 % n) * 4 + 3;
+      for (int i = 0; i < n; i++) from[to[i]] = i;
+      B.ptr.assign(1, 0);
+      for (int i = 0; i < 4 * n; i++) {
+        if (from[i] >= 0)
+          for (int e = A.ptr[from[i]]; e < A.ptr[from[i] + 1]; e++) B.col.push_back(to[A.col[e]]);
+        else  // rows of no subdomain, with neighbours in several
+          for (int c = 0; c < 3; c++) B.col.push_back((i + c) % (4 * n));
+        B.ptr.push_back((int)B.col.size());
+      }
+      B.val.assign(B.col.size(), 1.0);
+      std::vector<FrontPattern> p, q;
+      std::vector<int> pat, out, pat2, out2;
+      if (!build_front_patterns(A, starts, inds, 65534, 16, 2, 8, p, pat, out) ||
+          !build_front_patterns(B, starts, to, 65534, 16, 2, 8, q, pat2, out2))
+        return 1;
+      bool same = true;
+      for (int i = 0; i < n; i++) same = same && to[out[i]] == out2[i];
+      for (size_t b = 0; b < pat.size(); b++) same = same && bytes(p[pat[b]]) == bytes(q[pat2[b]]);
+      if (!same) {
+        printf("numbering %d: other patterns\n", way);
+        bad++;
+      }
+    }
   }
   return bad;
 }

@@ -158,6 +158,7 @@ struct doug_ctx {
   bool fronts = false;
   FrontSub *d_fsub = nullptr, *d_fsub_solve = nullptr;  // as partitioned; in dispatch order
   std::vector<FrontSub> h_fsub;
+  std::vector<int> front_like;  // subdomains of one local graph have one number (or -1)
   int maxwork = 0;  // largest work vector of a subdomain
   int64_t factor_elems = 0;
   // the batched solve's envelope factors and lists (the ones of the
@@ -2166,7 +2167,13 @@ static int device_fine(doug_ctx* ctx, hipEvent_t ev0, hipEvent_t ev1) {
     const int units = f32 ? kFrontUnitGroups32 : kFrontUnitGroups64;
     ctx->fronts = sizes && build_front_patterns(A, ctx->sstarts, ctx->sinds, max_work, ctx->front_nw, ctx->front_groups,
                                                 units, pats, pat, dinds, &ctx->front_groups);
-    if (!ctx->fronts) block_rcm(A, ctx->sstarts, ctx->sinds, dinds, &ctx->rank_ws);
+    if (ctx->fronts) {
+      ctx->front_like = pat;
+      for (int& k : ctx->front_like)
+        if (pats[k].mirrored) k = -1;
+    } else {
+      block_rcm(A, ctx->sstarts, ctx->sinds, dinds);
+    }
   } else {
     dinds = ctx->sinds;
     if (p.fine_method == 2)  // Gauss-Seidel sweeps the rows in ascending order
@@ -3036,7 +3043,7 @@ static int batch_factors(doug_ctx* ctx) {
   ctx->d_btiles32 = ctx->d_tiles32;
   if (!ctx->fronts) return DOUG_OK;
   std::vector<int> dinds;
-  block_rcm(ctx->A, ctx->sstarts, ctx->sinds, dinds, &ctx->rank_ws);
+  block_rcm(ctx->A, ctx->sstarts, ctx->sinds, dinds, &ctx->front_like);
   int *d_flag, flag = 0, rc;
   if ((rc = make_lists(ctx, dinds, ctx->batch_lists)) || (rc = dalloc(ctx, &d_flag, 1))) return rc;
   HIPCHK(hipMemsetAsync(d_flag, 0, sizeof(int), ctx->stream));

@@ -726,10 +726,10 @@ bool make_pattern(const Tree& T, int64_t max_work, int nw, int groups, int ug, F
 
 // Local graph of block [s0, s0 + s): neighbours inside the block, without
 // self loops, symmetric (reverse edges are added where the matrix lacks
-// them); returns a hash of it.  `floc` is scratch, -1 between calls: it spans
+// them, and `mirrored` is set); returns a hash of it.  `floc` is scratch, -1 between calls: it spans
 // the block's numbers alone, which for a box of a grid is a small part of the
 // matrix's (a whole array per thread costs more page faults than work).
-uint64_t local_graph(const Csr& A, const int* inds, int s, std::vector<int>& floc, Graph& g) {
+uint64_t local_graph(const Csr& A, const int* inds, int s, std::vector<int>& floc, Graph& g, bool& mirrored) {
   const int first = s > 0 ? *std::min_element(inds, inds + s) : 0;
   const int span = s > 0 ? *std::max_element(inds, inds + s) - first + 1 : 0;  // floc[span]: outside
   if (floc.size() <= (size_t)span) floc.assign((size_t)span + 1, -1);
@@ -760,7 +760,8 @@ uint64_t local_graph(const Csr& A, const int* inds, int s, std::vector<int>& flo
   }
   for (int li = 0; li < s; li++) floc[inds[li] - first] = -1;
   g.adj.resize((size_t)top);
-  if (fwd != rev) {  // unsymmetric structure: every edge in both directions
+  mirrored = fwd != rev;
+  if (mirrored) {  // unsymmetric structure: every edge in both directions
     Graph t;
     t.ptr.assign((size_t)s + 1, 0);
     for (int v = 0; v < s; v++)
@@ -803,6 +804,7 @@ bool build_front_patterns(const Csr& A, const std::vector<int>& starts, const st
   // graph (compared entry by entry) share it
   struct Known {
     Graph g;
+    bool mirrored;
     Tree t;
     FrontPattern p;
   };
@@ -822,7 +824,8 @@ bool build_front_patterns(const Csr& A, const std::vector<int>& starts, const st
     Graph g;
     for (int b = t; b < nb; b += nth) {
       const int s0 = starts[b], s = starts[b + 1] - s0;
-      const uint64_t h = local_graph(A, inds.data() + s0, s, floc, g);
+      bool mirrored;
+      const uint64_t h = local_graph(A, inds.data() + s0, s, floc, g, mirrored);
       Known* mine = nullptr;
       int count = 0;
       for (size_t seen = 0; pat[b] < 0; seen++) {  // the graphs of this hash one by one, compared outside the lock
@@ -838,12 +841,12 @@ bool build_front_patterns(const Csr& A, const std::vector<int>& starts, const st
           } else {
             pat[b] = (int)known.size();
             all.push_back(pat[b]);
-            known.emplace_back(new Known{std::move(g), {}, {}});
+            known.emplace_back(new Known{std::move(g), mirrored, {}, {}});
             mine = known.back().get();
             count = limit;
           }
         }
-        if (like && like->g.ptr == g.ptr && like->g.adj == g.adj) pat[b] = at;
+        if (like && like->mirrored == mirrored && like->g.ptr == g.ptr && like->g.adj == g.adj) pat[b] = at;
       }
       if (!mine) continue;
       bool fits = make_tree(mine->g, mine->t);
@@ -869,7 +872,10 @@ bool build_front_patterns(const Csr& A, const std::vector<int>& starts, const st
   if (!ok) return false;
   if (chosen) *chosen = limit;
   patterns.clear();
-  for (auto& k : known) patterns.push_back(std::move(k->p));
+  for (auto& k : known) {
+    patterns.push_back(std::move(k->p));
+    patterns.back().mirrored = k->mirrored;
+  }
   parallel([&](int t) {
     for (int b = t; b < nb; b += nth) {
       const std::vector<int32_t>& o = patterns[pat[b]].order;

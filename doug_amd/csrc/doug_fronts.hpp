@@ -72,6 +72,7 @@ enum {
 
 struct FrontPattern {
   int n = 0, top0 = 0, usz = 0;
+  bool mirrored = false;  // edges were added in reverse: its subdomains' own structures may differ
   int64_t elems = 0;   // panel elements
   int64_t schur = 0;   // set-up work elements
   std::vector<int32_t> order;      // position -> index in the subdomain's list

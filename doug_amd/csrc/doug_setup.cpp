@@ -5,10 +5,12 @@
 #include <algorithm>
 #include <atomic>
 #include <cmath>
+#include <memory>
 #include <numeric>
 #include <queue>
 #include <tuple>
 #include <thread>
+#include <unordered_map>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
@@ -1107,8 +1109,9 @@ struct RcmBuf {
   LocalGraph g;
 };
 
-// One block [s0, s0 + s) of `inds` into `out`; `floc` is -1 on entry and exit.
-void rcm_block(const Csr& A, const std::vector<int>& inds, int s0, int s, std::vector<int>& out,
+// One block [s0, s0 + s) of `inds`: the places of its nodes in their new order
+// in `place`; `floc` is -1 on entry and exit and spans the block's numbers alone.
+void rcm_block(const Csr& A, const std::vector<int>& inds, int s0, int s, int* place,
                std::vector<int>& floc, RcmBuf& buf) {
   std::vector<int>& mark = buf.mark;
   std::vector<int>& order = buf.order;
@@ -1117,10 +1120,14 @@ void rcm_block(const Csr& A, const std::vector<int>& inds, int s0, int s, std::v
   std::vector<char>& placed = buf.placed;
   LocalGraph& g = buf.g;
   if (s <= 1) {
-    if (s == 1) out[s0] = inds[s0];
+    if (s == 1) place[0] = 0;
     return;
   }
-  for (int li = 0; li < s; li++) floc[inds[s0 + li]] = li;
+  const auto range = std::minmax_element(inds.begin() + s0, inds.begin() + s0 + s);
+  const int first = *range.first;
+  const unsigned span = (unsigned)(*range.second - first) + 1;  // floc[span]: outside
+  if (floc.size() <= span) floc.assign((size_t)span + 1, -1);
+  for (int li = 0; li < s; li++) floc[inds[s0 + li] - first] = li;
   g.ptr.assign((size_t)s + 1, 0);
   g.deg.assign((size_t)s, 0);
   {
@@ -1136,7 +1143,7 @@ void rcm_block(const Csr& A, const std::vector<int>& inds, int s0, int s, std::v
     for (int li = 0; li < s; li++) {
       const int gi = inds[s0 + li];
       for (int p = A.ptr[gi]; p < A.ptr[gi + 1]; p++) {
-        const int lj = fl[acol[p]];
+        const int lj = fl[std::min((unsigned)(acol[p] - first), span)];
         adj[top] = lj;
         top += (lj >= 0) & (lj != li);
       }
@@ -1144,7 +1151,7 @@ void rcm_block(const Csr& A, const std::vector<int>& inds, int s0, int s, std::v
       g.deg[li] = g.ptr[li + 1] - g.ptr[li];
     }
   }
-  for (int li = 0; li < s; li++) floc[inds[s0 + li]] = -1;
+  for (int li = 0; li < s; li++) floc[inds[s0 + li] - first] = -1;
   mark.assign((size_t)s, 0);
   placed.assign((size_t)s, 0);
   order.clear();
@@ -1238,7 +1245,7 @@ void rcm_block(const Csr& A, const std::vector<int>& inds, int s0, int s, std::v
     }
     order.resize((size_t)tail);
   }
-  for (int q = 0; q < s; q++) out[s0 + q] = inds[s0 + order[s - 1 - q]];
+  for (int q = 0; q < s; q++) place[q] = order[s - 1 - q];
 }
 
 }  // namespace
@@ -1251,32 +1258,41 @@ struct RankNode {
 struct RankScratch {
   int n = 0;
   std::vector<RankNode> nd;
-  std::vector<int> floc;  // -1 between uses (block_rcm scratch)
   int tick = 0;
-  explicit RankScratch(int n_) : n(n_), nd((size_t)n_), floc((size_t)n_, -1) {}
+  explicit RankScratch(int n_) : n(n_), nd((size_t)n_) {}
 };
 
 void block_rcm(const Csr& A, const std::vector<int>& starts, const std::vector<int>& inds,
-               std::vector<int>& out, RankWorkspaces* ws) {
+               std::vector<int>& out, const std::vector<int>* same) {
   const int nb = (int)starts.size() - 1;
-  out.assign(inds.begin(), inds.end());
-  int nth = std::max(1, std::min(setup_threads(), nb));
-  // as many threads as lent scratch arrays (a fresh one costs more than a
-  // thread gains)
-  if (ws && !ws->w.empty() && ws->w[0] && ws->w[0]->n == A.nrows) nth = std::min(nth, (int)ws->w.size());
-  std::vector<std::thread> th;
-  for (int t = 0; t < nth; t++)
-    th.emplace_back([&, t]() {
-      // a node-indexed scratch of the whole matrix: the rank workers' one
-      // when it fits (-1 between uses), else a fresh one
-      RankScratch* rs = ws && t < (int)ws->w.size() && ws->w[t] && ws->w[t]->n == A.nrows ? ws->w[t].get() : nullptr;
-      std::vector<int> own;
-      if (!rs) own.assign((size_t)A.nrows, -1);
-      std::vector<int>& floc = rs ? rs->floc : own;
-      RcmBuf buf;
-      for (int b = t; b < nb; b += nth) rcm_block(A, inds, starts[b], starts[b + 1] - starts[b], out, floc, buf);
-    });
-  for (auto& x : th) x.join();
+  out.resize(inds.size());
+  // blocks to order, and the one that each block takes its order from
+  std::vector<int> own, like((size_t)nb);
+  std::unique_ptr<int[]> place(new int[inds.size()]);
+  std::unordered_map<int, int> first;
+  for (int b = 0; b < nb; b++) {
+    like[b] = same && (*same)[b] >= 0 ? first.emplace((*same)[b], b).first->second : b;
+    if (like[b] == b) own.push_back(b);
+  }
+  auto parallel = [&](int count, auto&& f) {
+    const int nth = std::max(1, std::min(setup_threads(), count));
+    std::vector<std::thread> th;
+    for (int t = 0; t < nth; t++) th.emplace_back(f, t, nth);
+    for (auto& x : th) x.join();
+  };
+  parallel((int)own.size(), [&](int t, int nth) {
+    std::vector<int> floc;
+    RcmBuf buf;
+    for (size_t k = (size_t)t; k < own.size(); k += (size_t)nth) {
+      const int s0 = starts[own[k]];
+      rcm_block(A, inds, s0, starts[own[k] + 1] - s0, place.get() + s0, floc, buf);
+    }
+  });
+  parallel(nb, [&](int t, int nth) {
+    for (int b = t; b < nb; b += nth)
+      for (int q = 0; q < starts[b + 1] - starts[b]; q++)
+        out[starts[b] + q] = inds[starts[b] + place[starts[like[b]] + q]];
+  });
 }
 
 // ---------------------------------------------------------------------------

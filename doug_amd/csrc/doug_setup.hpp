@@ -113,11 +113,11 @@ void set_setup_thread_cap(int cap);
 
 // Reverse Cuthill-McKee order of each block of `inds` over the graph of A
 // restricted to the block: out holds the same blocks, each a permutation of
-// its input.  Independent of the thread count.
-// `ws`, when given, lends its workers' node-indexed scratch.
-struct RankWorkspaces;
+// its input.  Independent of the thread count.  Blocks with the same number
+// (not negative) in `same`, when given, are ordered alike by the first of them:
+// they have to have the same local graph, entry by entry.
 void block_rcm(const Csr& A, const std::vector<int>& starts, const std::vector<int>& inds,
-               std::vector<int>& out, RankWorkspaces* ws = nullptr);
+               std::vector<int>& out, const std::vector<int>* same = nullptr);
 
 // Project graph partitioner (stands in for METIS): recursive bisection of a
 // symmetric adjacency (0-based CSR, no self loops) into nparts parts of

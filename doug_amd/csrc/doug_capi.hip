@@ -2360,6 +2360,9 @@ int doug_setup(doug_ctx* ctx, int32_t precision) {
   ctx->precision = precision;
   HIPCHK(hipSetDevice(ctx->device));
   free_device(ctx, true);
+  // a set-up that ended early may have left work on its streams, in the
+  // temporaries that this one takes over
+  for (hipStream_t q : {(hipStream_t)ctx->stream, ctx->stream2, ctx->stream3}) HIPCHK(hipStreamSynchronize(q));
   double t0 = now();
   // [0, 1] subdomain factorisation, [2, 3] coarse factorisation, [4] the
   // input of the subdomain factorisation, [5] its end

@@ -814,15 +814,19 @@ bool build_front_patterns(const Csr& A, const std::vector<int>& starts, const st
   bool ok = true;
   int limit = groups;  // workgroups that suit every pattern so far
   const int nth = std::max(1, std::min(setup_threads(), nb));
-  auto parallel = [&](auto&& f) {
+  // f on every thread; next() deals out the numbers below `count`, one at a time
+  // (another thread of the set-up may keep a core busy for part of it)
+  auto parallel = [&](int count, auto&& f) {
+    std::atomic<int> taken{0};
+    auto next = [&]() { return std::min(taken++, count); };
     std::vector<std::thread> th;
-    for (int t = 0; t < nth; t++) th.emplace_back(f, t);
+    for (int t = 0; t < nth; t++) th.emplace_back([&]() { f(next); });
     for (auto& x : th) x.join();
   };
-  parallel([&](int t) {
+  parallel(nb, [&](auto&& next) {
     std::vector<int> floc;
     Graph g;
-    for (int b = t; b < nb; b += nth) {
+    for (int b = next(); b < nb; b = next()) {
       const int s0 = starts[b], s = starts[b + 1] - s0;
       bool mirrored;
       const uint64_t h = local_graph(A, inds.data() + s0, s, floc, g, mirrored);
@@ -860,10 +864,10 @@ bool build_front_patterns(const Csr& A, const std::vector<int>& starts, const st
   });
   // the others follow the one that takes the fewest workgroups
   for (; ok; limit /= 2) {
-    std::atomic<int> next{0};
+    const int count = (int)known.size();
     std::atomic<bool> fits{true};
-    parallel([&](int) {
-      for (int k = next++; k < (int)known.size() && fits; k = next++)
+    parallel(count, [&](auto&& next) {
+      for (int k = next(); k < count && fits; k = next())
         if (known[k]->p.groups != limit && !make_pattern(known[k]->t, max_work, nw, limit, ug, known[k]->p)) fits = false;
     });
     if (fits) break;
@@ -876,8 +880,8 @@ bool build_front_patterns(const Csr& A, const std::vector<int>& starts, const st
     patterns.push_back(std::move(k->p));
     patterns.back().mirrored = k->mirrored;
   }
-  parallel([&](int t) {
-    for (int b = t; b < nb; b += nth) {
+  parallel(nb, [&](auto&& next) {
+    for (int b = next(); b < nb; b = next()) {
       const std::vector<int32_t>& o = patterns[pat[b]].order;
       for (size_t p = 0; p < o.size(); p++) out[starts[b] + p] = inds[starts[b] + o[p]];
     }

@@ -1276,20 +1276,23 @@ void block_rcm(const Csr& A, const std::vector<int>& starts, const std::vector<i
   }
   auto parallel = [&](int count, auto&& f) {
     const int nth = std::max(1, std::min(setup_threads(), count));
+    std::atomic<int> taken{0};
+    auto next = [&]() { return std::min(taken++, count); };
     std::vector<std::thread> th;
-    for (int t = 0; t < nth; t++) th.emplace_back(f, t, nth);
+    for (int t = 0; t < nth; t++) th.emplace_back([&]() { f(next); });
     for (auto& x : th) x.join();
   };
-  parallel((int)own.size(), [&](int t, int nth) {
+  const int orders = (int)own.size();
+  parallel(orders, [&](auto&& next) {
     std::vector<int> floc;
     RcmBuf buf;
-    for (size_t k = (size_t)t; k < own.size(); k += (size_t)nth) {
+    for (int k = next(); k < orders; k = next()) {
       const int s0 = starts[own[k]];
       rcm_block(A, inds, s0, starts[own[k] + 1] - s0, place.get() + s0, floc, buf);
     }
   });
-  parallel(nb, [&](int t, int nth) {
-    for (int b = t; b < nb; b += nth)
+  parallel(nb, [&](auto&& next) {
+    for (int b = next(); b < nb; b = next())
       for (int q = 0; q < starts[b + 1] - starts[b]; q++)
         out[starts[b] + q] = inds[starts[b] + place[starts[like[b]] + q]];
   });

@@ -2150,7 +2150,7 @@ static int device_fine(doug_ctx* ctx, hipEvent_t ev0, hipEvent_t ev1) {
     // eight wavefronts where a CU takes several subdomains (512, FP64: 806 us,
     // 852 us with sixteen), sixteen where there is a CU for each (9 subdomains:
     // 113 us, 122 us with eight)
-    ctx->front_nw = ctx->nsub > 256 ? 8 : 16;
+    ctx->front_nw = ctx->nsub > kCus ? 8 : 16;
     // (the envelope solve's size limit holds for either: the batched solve uses it)
     bool sizes = true;
     for (size_t b = 0; b + 1 < ctx->sstarts.size(); b++)
@@ -2162,7 +2162,7 @@ static int device_fine(doug_ctx* ctx, hipEvent_t ev0, hipEvent_t ev1) {
     // with one and 184 us with two (FP64; in FP32 64 of 4300 103 us with one
     // and 75 us with four, 100 103 us with one and 88 us with two)
     ctx->front_groups = 1;
-    while (2 * ctx->front_groups * ctx->nsub <= 256 && ctx->front_groups < kFrontGroupsMax)
+    while (2 * ctx->front_groups * ctx->nsub <= kCus && ctx->front_groups < kFrontGroupsMax)
       ctx->front_groups *= 2;
     const int units = f32 ? kFrontUnitGroups32 : kFrontUnitGroups64;
     ctx->fronts = sizes && build_front_patterns(A, ctx->sstarts, ctx->sinds, max_work, ctx->front_nw, ctx->front_groups,
@@ -2729,9 +2729,11 @@ int doug_prec_apply_device(doug_ctx* ctx, const double* dr, double* dz) {
 }  // extern "C"
 
 // ---------------------------------------------------------------------------
-// Allocation-free preconditioner apply: the work vectors of an apply live in
-// one file-scope device array per GPU, of kNoAllocDoubles doubles (32 MiB),
-// which the loaded code object holds until the process ends.  Host code
+// Allocation-free preconditioner apply: the subdomain and coarse work vectors
+// of an apply live in one file-scope device array per GPU, of kNoAllocDoubles
+// doubles (32 MiB), which the loaded code object holds until the process ends;
+// what several workgroups of one subdomain hand over goes through the context's
+// d_updates, from the set-up.  Host code
 // never passes the array's name to a kernel: its device address comes from
 // hipGetSymbolAddress, once per device, with that device current.
 constexpr int64_t kNoAllocDoubles = 4194304;
@@ -3518,17 +3520,17 @@ int doug_autotune(doug_ctx* ctx, int32_t reps, doug_tuning* out) {
   bool uneven = false;
   for (size_t b = 1; b < ctx->h_sub.size(); b++) uneven = uneven || ctx->h_sub[b - 1].nt < ctx->h_sub[b].nt;
   if (ctx->batch_ready && ctx->fronts && uneven) {
-    // the order above is the fronts': the batch's envelopes are timed by themselves
-    const int rt = std::max(2, reps / 8);
-    double ms[2];
-    for (int o = 0; o < 2; o++) {
-      ctx->batch_order = o;
-      if ((rc = apply_orders(ctx)) ||
-          (rc = time_launches(ctx, rt, [&]() { enqueue_prec_multi(ctx, kMaxRhs, ctx->d_Rm, ctx->d_Zm); }, &ms[o])))
-        return rc;
+    // the order so far is the fronts': the other one, for the batch's envelopes
+    double ms;
+    ctx->batch_order = 1 - order;
+    if ((rc = apply_orders(ctx)) ||
+        (rc = time_launches(ctx, std::max(2, reps / 8),
+                            [&]() { enqueue_prec_multi(ctx, kMaxRhs, ctx->d_Rm, ctx->d_Zm); }, &ms)))
+      return rc;
+    if (ms >= tu.trsm_ms[kb - 1]) {
+      ctx->batch_order = order;
+      if ((rc = apply_orders(ctx))) return rc;
     }
-    ctx->batch_order = ms[1] < ms[0] ? 1 : 0;
-    if ((rc = apply_orders(ctx))) return rc;
   }
   tu.trsm_col_groups = cg;
   HIPCHK(hipStreamSynchronize(ctx->stream));

@@ -576,6 +576,9 @@ __device__ __forceinline__ void load_panel(UnitLoad& b, const float* pan, const 
 // memory (as doubles, unrounded).  Stage 0 is all of it in one workgroup.
 // 64 subdomains of 5250 unknowns: 181 us (248 us in one workgroup each); of
 // 4300 in two dimensions 75 us (103); 4 of 4300: 57 us (95).
+// The matrix-core form below has been measured in FP64 only, where it gave 3 to
+// 9 %.  Here another order of the sums also moves the iteration counts of some
+// systems by one (8 of 384 inputs between fronts and envelopes).
 enum { kWhole = 0, kSubtreesForward = 1, kApex = 2, kSubtreesBackward = 3 };
 template <int NW, int STAGE>
 __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(4))) void k_front_solve(

@@ -979,8 +979,11 @@ __global__ __launch_bounds__(256) void k_dot_chunks(const double* __restrict__ a
 // thread and in k_reduce_finish's order.  Up to that many (262,144 unknowns)
 // the kernel that needs a sum forms it itself, each workgroup again, instead
 // of waiting for a launch of one workgroup (4.2 us each, two an iteration):
-// solves of 16,384 unknowns 3.64 to 3.58 ms, of 250,000 14.21 to 14.09 ms.
-// Above, the partials are more than a workgroup should read again.
+// solves of 16,384 unknowns 3.64 to 3.58 ms, of 250,000 14.21 to 14.09 ms (a
+// grid of 250,000: 307 against 310 us per iteration).  With a limit four times
+// as high 518,400 unknowns took 836 against 830 us and a million 2455 against
+// 2440, each workgroup reading all partials again, and the smaller grids 4 to 5
+// us more, each thread holding places for sixteen.
 __device__ __forceinline__ double fold_partials(const double* __restrict__ partial, int count, double* sh) {
   const int t = threadIdx.x, lane = t & 63, w = t >> 6;
   double v[kFoldPartials / 256];

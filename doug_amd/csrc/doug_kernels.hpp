@@ -9,6 +9,7 @@ constexpr int kTile = 64;              // dense tile edge (one wavefront wide)
 constexpr int kTileElems = kTile * kTile;
 constexpr int kSpmvThreads = 256;      // CSR-stream block
 constexpr int kSpmvChunk = 2048;       // products staged in LDS per block
+constexpr int kCus = 256;              // compute units of an MI355X
 constexpr int kLdsBytes = 160 * 1024;   // of a CU, all of which a workgroup may take
 constexpr int kMaxTrsvTiles = 256;     // subdomain size limit of the one-block solve (16384)
 constexpr int kRedBlocks = 1024;       // fixed partial count of the grid reductions

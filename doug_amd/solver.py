@@ -286,7 +286,7 @@ class Solver:
 
     # -- several right-hand sides --
     def prepare_batch(self):
-        """Explicit inverse subdomain factors for batched applies (doug_prepare_batch)."""
+        """Workspaces of the batched solves, and their envelope factors beside frontal ones (doug_prepare_batch)."""
         self._check(self._L.doug_prepare_batch(self.h))
 
     def pcg_batch(self, B, tol=1e-8, maxit=-1, X0=None):

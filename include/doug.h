@@ -63,8 +63,9 @@ typedef struct {
 } doug_params;
 
 /* Sizes and timings of the last doug_setup (seconds).  factor_bytes counts
- * the stored subdomain factors (frontal panels, or the 64x64 tiles inside
- * each factor's envelope) and factor_tiles the same in units of 4096 entries;
+ * the stored subdomain factors of the single-vector solves (frontal panels, or
+ * the 64x64 tiles inside each factor's envelope; what doug_prepare_batch adds
+ * is not in it) and factor_tiles the same in units of 4096 entries;
  * factor_flops is the work of their factorisation. */
 typedef struct {
   int32_t n, nagr_fine, nagr_coarse, nsub, ncoarse, overlap, smoothers;
@@ -236,7 +237,8 @@ int doug_prec_apply_device(doug_ctx *ctx, const double *dr, double *dz);
  * call: the apply's work vectors (the subdomain vectors, the coarse vectors
  * and their partial sums) live in one static device array per GPU of
  * 4194304 doubles (32 MiB), held until the process ends; a set-up needing
- * more is refused with DOUG_E_ARG.  The results equal
+ * more is refused with DOUG_E_ARG.  (What several workgroups of one subdomain
+ * hand over goes through a buffer that doug_setup has left in the context.)  The results equal
  * doug_prec_apply_device's bit for bit.  Every call on one GPU shares that
  * array, so calls that overlap on one GPU (several threads, or contexts on
  * the same device) race.  No counterpart in the reference: it serves callers
@@ -296,8 +298,8 @@ int doug_get_tuning(const doug_ctx *ctx, doug_tuning *out);
  * DOUG_OPT_SPMV_SHAPE (0..5) and DOUG_OPT_TRSV_ORDER (0/1) set what
  * doug_autotune would choose, see doug_tuning.  DOUG_OPT_LOCAL_ORDER
  * (default 1) places each subdomain's unknowns in its factor in nested
- * dissection order, for frontal factors, or, where a subdomain is too large
- * for them, in reverse Cuthill-McKee order, which narrows the stored tile
+ * dissection order, for frontal factors, or, where any subdomain is too large
+ * for them, all in reverse Cuthill-McKee order, which narrows the stored tile
  * envelope; 0 keeps the index-set order (envelopes).  It needs a new
  * doug_setup and changes rounding only.
  * DOUG_OPT_DEVICE_COARSE (default 1): build the smoothed restriction and the
@@ -310,7 +312,8 @@ int doug_get_tuning(const doug_ctx *ctx, doug_tuning *out);
  * the host scatter map, which 0 selects; a matrix holding a duplicate
  * (i, j) pair always uses the host map); at the next doug_setup.
  * DOUG_OPT_KEEP_SETUP_TEMPS (default 1): keep the coarse build's device
- * temporaries between set-ups (doug_info.temp_bytes), so that a repeated
+ * temporaries and the subdomain factorisation's update matrices between
+ * set-ups (doug_info.temp_bytes), so that a repeated
  * set-up of the same size neither allocates nor frees them; 0 frees them
  * now and at the end of every set-up.
  * DOUG_OPT_BATCH_COLUMN_GROUPS (1, 2 or 3, default 1): layout of the

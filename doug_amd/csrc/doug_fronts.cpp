@@ -353,7 +353,8 @@ struct Tree {
   std::vector<int> listed;  // position -> node
   std::vector<Front> fronts;
   std::vector<int> parent;
-  std::vector<std::vector<uint16_t>> rows;
+  std::vector<uint16_t> rows;  // front f's: rptr[f] ..
+  std::vector<int> rptr;
 };
 
 // False where a front or the graph exceeds the format.
@@ -394,15 +395,16 @@ bool make_tree(const Graph& g, Tree& T) {
   std::vector<int> pos((size_t)n);
   for (int p = 0; p < n; p++) pos[D.listed[p]] = p;
   const int words = (n + 63) / 64;
-  std::vector<std::vector<uint16_t>>& rows = T.rows;
-  rows.resize((size_t)nf);
+  std::vector<uint16_t>& rows = T.rows;
+  std::vector<int>& rptr = T.rptr;
+  rptr.assign(1, 0);
   std::vector<uint64_t> bits((size_t)words);
   for (int f = 0; f < nf; f++) {
     const int c0 = F[f].c0, c1 = c0 + F[f].k;
     std::fill(bits.begin() + c0 / 64, bits.end(), 0);
     for (int c : F[f].child)
       if (c >= 0) {
-        for (uint16_t r : rows[c]) bits[r >> 6] |= 1ull << (r & 63);
+        for (int i = rptr[c]; i < rptr[c + 1]; i++) bits[rows[i] >> 6] |= 1ull << (rows[i] & 63);
       }
     for (int p = c0; p < c1; p++) {
       const int v = D.listed[p];
@@ -414,10 +416,12 @@ bool make_tree(const Graph& g, Tree& T) {
     for (int w = c1 / 64; w < words; w++) {
       uint64_t x = bits[w];
       if (w == c1 / 64) x &= ~0ull << (c1 & 63);
-      for (; x; x &= x - 1) rows[f].push_back((uint16_t)(64 * w + __builtin_ctzll(x)));
+      for (; x; x &= x - 1) rows.push_back((uint16_t)(64 * w + __builtin_ctzll(x)));
     }
-    F[f].m = (uint16_t)rows[f].size();
-    if ((int)F[f].k + F[f].m > 64 * 250) return false;
+    const int m = (int)rows.size() - rptr[f];
+    rptr.push_back((int)rows.size());
+    if ((int)F[f].k + m > 64 * 250) return false;
+    F[f].m = (uint16_t)m;
   }
   T.listed.swap(D.listed);
   return true;
@@ -434,7 +438,6 @@ bool make_pattern(const Tree& T, int64_t max_work, int nw, int groups, int ug, F
   std::vector<Front>& F = P.fronts;
   const int nf = (int)F.size();
   const std::vector<int>& parent = T.parent;
-  const std::vector<std::vector<uint16_t>>& rows = T.rows;
   std::vector<int64_t> cost((size_t)nf);
   for (int f = 0; f < nf; f++) {
     cost[f] = front_cost(F[f], ug);
@@ -538,7 +541,7 @@ bool make_pattern(const Tree& T, int64_t max_work, int nw, int groups, int ug, F
     if (nbottom == nf) P.top0 = n;
   }
   std::vector<Front> G((size_t)nf);
-  std::vector<std::vector<uint16_t>> R((size_t)nf);
+  P.rpos.reserve(T.rows.size() + (size_t)n);
   std::vector<int> lv((size_t)nf), wv((size_t)nf), hv((size_t)nf);
   int at = 0;
   int64_t elems = 0, recs = 0;
@@ -554,8 +557,8 @@ bool make_pattern(const Tree& T, int64_t max_work, int nw, int groups, int ug, F
     recs += f.k + f.m;
     if (elems > INT32_MAX || recs > INT32_MAX) return false;
     // ancestors keep their relative order, so the rows stay ascending
-    R[q].resize(f.m);
-    for (int r = 0; r < f.m; r++) R[q][r] = (uint16_t)newpos[rows[o][r]];
+    for (int c = 0; c < f.k; c++) P.rpos.push_back((uint16_t)(f.c0 + c));
+    for (int r = T.rptr[o]; r < T.rptr[o + 1]; r++) P.rpos.push_back((uint16_t)newpos[T.rows[r]]);
     lv[q] = level[o];
     wv[q] = group[o] * nw + wave[o];
     hv[q] = height[o];
@@ -598,22 +601,20 @@ bool make_pattern(const Tree& T, int64_t max_work, int nw, int groups, int ug, F
   if ((int64_t)n + P.usz > std::min<int64_t>(max_work, 65535)) return false;
   for (int q = 0; q < nf; q++) F[q].u = (uint16_t)(n + u[q]);
   // row records
-  P.rpos.resize((size_t)recs);
   P.src.resize((size_t)recs);
   for (int q = 0; q < nf; q++) {
     const Front& f = F[q];
-    uint16_t* rp = P.rpos.data() + f.row0;
+    const uint16_t* rp = P.rpos.data() + f.row0;
     uint32_t* sr = P.src.data() + f.row0;
-    for (int c = 0; c < f.k; c++) rp[c] = (uint16_t)(f.c0 + c);
-    std::copy(R[q].begin(), R[q].end(), rp + f.k);
     const int h = f.k + f.m;
     for (int r = 0; r < h; r++) sr[r] = (uint32_t)n | (uint32_t)n << 16;
     for (int b = 0; b < 2; b++) {
       const int c = f.child[b];
       if (c < 0) continue;
+      const uint16_t* rc = P.rpos.data() + F[c].row0 + F[c].k;
       int r = 0;
       for (int j = 0; j < F[c].m; j++) {  // both ascending
-        while (rp[r] != R[c][j]) r++;
+        while (rp[r] != rc[j]) r++;
         const uint32_t idx = (uint32_t)F[c].u + (uint32_t)j;
         sr[r] = b == 0 ? (sr[r] & 0xffff0000u) | idx : (sr[r] & 0xffffu) | idx << 16;
       }

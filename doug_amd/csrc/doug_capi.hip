@@ -2148,15 +2148,15 @@ static int device_fine(doug_ctx* ctx, hipEvent_t ev0, hipEvent_t ev1) {
     const bool f32 = ctx->precision == DOUG_PREC_FP32_FACTORS;
     const int64_t max_work = kLdsBytes / (f32 ? 4 : 8) - 64 - (f32 ? 0 : 64 * kFrontWavesMax);
     // eight wavefronts where a CU takes several subdomains (512, FP64: 806 us,
-    // 852 us with sixteen), sixteen where there is a CU for each (9 subdomains:
-    // 113 us, 122 us with eight)
+    // 852 us with sixteen), sixteen where there is a CU for each (4 of 4224
+    // unknowns: 113 us, 122 us with eight)
     ctx->front_nw = ctx->nsub > kCus ? 8 : 16;
     // (the envelope solve's size limit holds for either: the batched solve uses it)
     bool sizes = true;
     for (size_t b = 0; b + 1 < ctx->sstarts.size(); b++)
       sizes = sizes && ctx->sstarts[b + 1] - ctx->sstarts[b] <= kMaxTrsvTiles * kTile;
-    // two, four or eight workgroups per subdomain as long as each has a CU: 9
-    // subdomains of 2100 unknowns took 110 us with one, 74 us with four and
+    // two, four or eight workgroups per subdomain as long as each has a CU: 4
+    // subdomains of 4224 unknowns took 110 us with one, 74 us with four and
     // 61 us with eight, 64 of 4300 171, 108 and (two rounds) 129 us, 100 of
     // 4300 121 us with one, 96 us with two and 122 us with four, 225 137 us
     // with one and 184 us with two (FP64; in FP32 64 of 4300 103 us with one

@@ -575,7 +575,7 @@ __device__ __forceinline__ void load_panel(UnitLoad& b, const float* pan, const 
 // the subtrees backward; y and the updates in between go through global
 // memory (as doubles, unrounded).  Stage 0 is all of it in one workgroup.
 // 64 subdomains of 5250 unknowns: 181 us (248 us in one workgroup each); of
-// 4300 in two dimensions 75 us (103); 4 of 4300: 57 us (95).
+// 4300 in two dimensions 75 us (103); 4 of 4224: 57 us (95).
 // The matrix-core form below has been measured in FP64 only, where it gave 3 to
 // 9 %.  Here another order of the sums also moves the iteration counts of some
 // systems by one (8 of 384 inputs between fronts and envelopes).
@@ -869,8 +869,8 @@ __device__ __forceinline__ int panel_bytes(int H, int g1) { return 32 * (g1 * H 
 //
 // The stages are those of the vector form.  64 subdomains of 4300
 // unknowns in two dimensions: 35 + 38 + 34 us (171 us in one workgroup each,
-// the vector form 188, envelopes 709); 9 of 2100: 15 + 30 + 17 us (110, 113,
-// 310).
+// the vector form 188, envelopes 709); 4 of 4224: 15 + 30 + 17 us (110, 113,
+// 302).
 template <int NW, int STAGE>
 __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(4))) void k_front_solve_mma(
     const double* __restrict__ tiles, const FrontSub* __restrict__ subs, int groups, int maxwork,
